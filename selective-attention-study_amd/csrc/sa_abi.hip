@@ -21,7 +21,7 @@ using namespace sa_host;
 
 extern "C" {
 
-int sa_abi_version(void) { return 5; }
+int sa_abi_version(void) { return 6; }
 
 int sa_timing_enable(int on) {
   TimingRegistry& r = timing();
@@ -74,6 +74,11 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
   const int64_t es = dtype == SA_DTYPE_BF16 ? 2 : 4;
   if (dtype == SA_DTYPE_BF16 && head_dim == 64 && auto_group(dtype, head_dim, heads, group, false) <= 2) return 0;
   return align_up(nseq * heads * head_dim * sa_transposed_ld(tk) * es, 256);
+}
+
+int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim) {
+  if (!valid_dims(nseq, heads, t) || (head_dim != 32 && head_dim != 64 && head_dim != 128)) return -1;
+  return fwd_reach_bytes(nseq, heads, t);
 }
 
 int sa_forward(const void* q, const void* k, const void* v, float* out, float* rmax, float* rden, float* carry,
@@ -144,6 +149,12 @@ int sa_forward_strided(const void* q, const sa_view_strides* q_strides, const vo
   c.state_out = state_out;
   c.state_ld = state_ld;
   c.ws = workspace;
+  // skipping tiles needs the extra scratch; damped histories are not monotone over the queries
+  if (workspace && tk >= REACH_MIN_KEYS && damp_mode == 0 &&
+      workspace_bytes >= need + fwd_reach_bytes(nseq, heads, tk) && (uintptr_t)workspace % 4 == 0) {
+    c.kn = reinterpret_cast<float*>(static_cast<char*>(workspace) + need);
+    c.kt = c.kn + nseq * heads * cdiv(tk, TILE);
+  }
   c.nseq = (int)nseq;
   c.H = (int)heads;
   c.Tq = (int)tq;

@@ -172,6 +172,17 @@ inline BwdLayout bwd_layout(int64_t nseq, int64_t heads, int64_t t, int64_t D, i
   return L;
 }
 
+// Optional extra workspace, past the sizes above, in which the kernels find the key tiles that still
+// carry weight (sa_reach_bytes): without it every causal tile is computed. Forward: kn, one bound on
+// the key norms per head and key tile; kt, the least selection total of each key tile. A launch looks for tiles to skip only from REACH_MIN_KEYS keys
+// on: below, a query block has few tiles that a history can have outgrown.
+constexpr int REACH_MIN_KEYS = 1024;
+constexpr int REACH_MASK_WORDS = 128;   // a workgroup's tile mask: its newest 64 * 128 key tiles
+
+inline int64_t fwd_reach_bytes(int64_t nseq, int64_t heads, int64_t tk) {
+  return align_up(nseq * (heads + 1) * cdiv(tk, TILE) * 4, 256);
+}
+
 inline bool valid_dims(int64_t nseq, int64_t heads, int64_t t) {
   const int64_t lim = (int64_t)1 << 30;
   return nseq >= 1 && heads >= 1 && t >= 1 && nseq < 65536 && heads < 65536 && t < lim && nseq * heads < 65536;
@@ -212,6 +223,7 @@ struct FwdCall {
   float* state_out;
   int64_t state_ld;
   void* ws;
+  float *kn, *kt;   // key-tile norm bounds and selection totals (fwd_reach_bytes), NULL: compute every tile
   int nseq, H, Tq, Tk;
   int q_off;
   float scale;

@@ -43,6 +43,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -681,17 +682,275 @@ __device__ __forceinline__ float block_selection_sum(const f32x16& acc, bool int
 }
 
 // ---------------------------------------------------------------------------------------------
+// Skipping key tiles that carry no weight. F only grows with the query, so once a key's history has
+// outgrown its logit by enough, its softmax weight is an exact fp32 zero for every later query, and so
+// are its terms in every sum it enters. For a tile of keys and a block of queries,
+//
+//     log2 weight <= s log2e (max |q|) (max |k|) - log2e (min F) - (min row maximum so far),
+//
+// and exp2 returns exactly zero below -149 (-126 where denormals flush). A tile whose bound lies
+// below -REACH_ZERO (a margin for the rounding of the bound's own terms: the norms are taken 1% high,
+// F a thousandth low) is left out of the sweep: the skipped terms are zeros, so the results keep their
+// bits. Nothing is skipped where a zero weight would not give a zero term: a tile with a key or value
+// that is not finite, or so large that a product of two rows could overflow, gets the bound infinity,
+// and every comparison is written so that a NaN keeps the tile.
+// Measured (forward kernel, bf16, D=64, N(0,1) inputs, whose histories grow by 0.4 a query): B=1 H=16
+// T=16384 918 -> 97 us, the last 16384 queries of 131072 13.2 -> 0.17 ms, B=2 H=12 T=2048 85 -> 35 us; where
+// one pair in a hundred is selected and nothing can be left out: B=2 H=12 T=5003 249 -> 250 us, B=1 H=12
+// T=16384 740 -> 751 us, and the key norms add 2 and 6 us to the column sums' launch.
+constexpr float REACH_ZERO = 160.f;
+constexpr float REACH_NORM2 = 1e37f;      // sums of squares at or past this count as not finite
+constexpr float REACH_Q = 1.01f * LOG2E;
+constexpr float REACH_F = 0.999f * LOG2E;
+constexpr int NORM_KEYS = 256;            // keys per workgroup of the norms
+
+// The sum of squares of 8 elements of a row.
+template <typename E>
+__device__ __forceinline__ float sumsq8(const E* p) {
+  float s = 0.f;
+  if constexpr (sizeof(E) == 2) {
+    const uint4 u = *reinterpret_cast<const uint4*>(p);
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float lo = __uint_as_float(w[i] << 16), hi = __uint_as_float(w[i] & 0xFFFF0000u);
+      s = fmaf(lo, lo, s);
+      s = fmaf(hi, hi, s);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float4 f = reinterpret_cast<const float4*>(p)[i];
+      s = fmaf(f.x, f.x, fmaf(f.y, f.y, fmaf(f.z, f.z, fmaf(f.w, f.w, s))));
+    }
+  }
+  return s;
+}
+
+// kn[r][kt] = max |k_j| over the keys of tile kt of head r = b * H + head, infinity when a key or a
+// value of the tile is not finite (or too large, REACH_NORM2). Workgroup `blk` takes NORM_KEYS keys of
+// head r: a wavefront two tiles, D/8 lanes per row, a tile's loads all issued before their use. Bound
+// by HBM (each key and value read once).
+template <typename E, int D>
+__device__ __forceinline__ void key_norms_block(const E* k, const E* v, const Strides& ks, const Strides& vs, int H,
+                                                int Tk, float* kn, int r, int blk) {
+  constexpr int LPR = D / 8, RPW = 64 / LPR, PASSES = TILE / RPW;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int NKT = (Tk + TILE - 1) / TILE;
+  const E* kh = k + ks.at(r / H, r % H) + (lane % LPR) * 8;
+  const E* vh = v + vs.at(r / H, r % H) + (lane % LPR) * 8;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int kt = blk * (NORM_KEYS / TILE) + wave * 2 + u;
+    if (kt >= NKT) break;
+    float sk[PASSES], sv[PASSES];
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const int64_t j = min(kt * TILE + p * RPW + lane / LPR, Tk - 1);   // (the last key again past the end)
+      sk[p] = sumsq8(kh + j * ks.row);
+      sv[p] = sumsq8(vh + j * vs.row);
+    }
+    float mx = 0.f;
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+#pragma unroll
+      for (int o = LPR / 2; o > 0; o >>= 1) {
+        sk[p] += __shfl_xor(sk[p], o);
+        sv[p] += __shfl_xor(sv[p], o);
+      }
+      mx = fmaxf(mx, (sk[p] < REACH_NORM2 && sv[p] < REACH_NORM2) ? sk[p] : INFINITY);
+    }
+#pragma unroll
+    for (int o = LPR; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if (lane == 0) kn[(int64_t)r * NKT + kt] = sqrtf(mx);
+  }
+}
+
+template <typename E, int D>
+__global__ __launch_bounds__(NTHREADS) void key_norms_kernel(const E* __restrict__ k, const E* __restrict__ v, Strides ks,
+                                                             Strides vs, int H, int Tk, float* __restrict__ kn) {
+  key_norms_block<E, D>(k, v, ks, vs, H, Tk, kn, blockIdx.y, blockIdx.x);
+}
+
+// The maximum over the 32 lanes of each half-wavefront (those of them that are active).
+__device__ __forceinline__ float half_max(float x) {
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) x = fmaxf(x, __shfl_xor(x, o));
+  return x;
+}
+
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) |
+         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
+}
+
+// The tiles a workgroup has to visit, newest first, as runs of consecutive tiles: a sweep counts down
+// within a run and takes the next one from LDS at its end (a tile list or a bit mask walked in the tile
+// loop cost it 2% where nothing is skipped, in scalar instructions and spilled scalar registers).
+struct TileRun {
+  int hi, lo;
+};
+constexpr int REACH_RUNS = 64;   // at most; what would need more ends in one run down to tile 0
+
+// The set bits of the words (bit i of word w: tile first + 64 w + i), then every tile below first, as runs
+// ending in {-1, INT_MIN}, below which a sweep finds no tile. One wavefront.
+__device__ __forceinline__ void write_reach_runs(TileRun* runs, const uint64_t* words, int nwords, int first, int lane) {
+  int n = 0;
+  TileRun open{-1, -1};
+  auto add = [&](int hi, int lo) {
+    if (open.hi >= 0 && hi == open.lo - 1) {
+      open.lo = lo;
+      return;
+    }
+    if (open.hi >= 0) {
+      if (lane == 0) runs[n] = open;
+      ++n;
+    }
+    open = {hi, lo};
+  };
+  int w = nwords;
+  while (w > 0) {   // the newest word before w that holds a tile, 64 words at a time
+    const int base = max(w - 64, 0);
+    const uint64_t some = __ballot(base + lane < w && words[min(base + lane, w - 1)] != 0);
+    if (some == 0) {
+      w = base;
+      continue;
+    }
+    w = base + 63 - __builtin_clzll(some);
+    uint64_t word = uniform64(words[w]);
+    while (word != 0) {
+      const int bit = 63 - __builtin_clzll(word);
+      const uint64_t gaps = ~word << (63 - bit);
+      const int len = min(gaps != 0 ? __builtin_clzll(gaps) : 64, bit + 1);
+      add(first + 64 * w + bit, first + 64 * w + bit - len + 1);
+      word &= (bit - len >= 0) ? (2ull << (bit - len)) - 1 : 0;
+      if (n == REACH_RUNS - 2) {
+        open.lo = 0;
+        word = 0;
+        w = 0;
+        first = 0;
+      }
+    }
+  }
+  if (first > 0) add(first - 1, 0);
+  if (lane == 0) {
+    if (open.hi >= 0) runs[n++] = open;
+    runs[n] = {-1, INT_MIN};
+  }
+}
+
+// Whether looking for tiles to skip can pay: every key of one of the 64 oldest tiles has received enough by
+// the sequence's end. total: this lane's such tile's least selection total (reach_total, loaded before
+// the sweep so that it costs no wait). Only the time depends on the answer.
+__device__ __forceinline__ float reach_total(const float* kt_min, int ntiles, int lane) {
+  return kt_min != nullptr && lane < ntiles ? kt_min[lane] : 0.f;
+}
+__device__ __forceinline__ bool reach_worth(float total) { return __any(total * LOG2E > REACH_ZERO - 16.f); }
+
+// Sum of squares of a lane's part of its query row.
+template <class OP, int NS>
+__device__ __forceinline__ float frag_sumsq(const typename OP::frag (&f)[NS]) {
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    if constexpr (OP::KS == 16) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s = fmaf((float)f[i][e], (float)f[i][e], s);
+    } else {
+      s = fmaf(f[i], f[i], s);
+    }
+  }
+  return s;
+}
+
+// The key tiles below `cut` that a forward workgroup has to visit, as runs (write_reach_runs), once its
+// diagonal tiles are behind it: qf the lane's parts of its query of each head, m the query's running
+// maximum (log2 units), row whether there is such a query; kn the first head's key norms, the next
+// heads' NKT apart; kt_min the least selection total of each tile; crow the carry row of the workgroup's first query block (later
+// blocks' histories are no smaller). The tiles below i_lo (exempt keys have no history) are always visited. A lane decides a
+// tile by its 128 carry bytes (eight 16-byte loads; past the row's end they read zero, which keeps the
+// tile), a wavefront every fourth word of 64 tiles; the tiles older than the words hold are visited.
+// All wavefronts of the workgroup; the runs may be read on return.
+template <class OP, int G, int NS>
+__device__ __forceinline__ void find_reach(const typename OP::frag (&qf)[G][NS], const float (&m)[G], bool row,
+                                           float scale, const float* kn, const float* kt_min, int NKT,
+                                           const float* crow, int Tk, int cut,
+                                           int i_lo, float (*bound)[2 * G], uint64_t* words, TileRun* runs, int lane,
+                                           int wave) {
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    float qn = frag_sumsq<OP, NS>(qf[g]);
+    qn += xor32(qn);
+    qn = half_max(qn < REACH_NORM2 ? qn : INFINITY);
+    const float ml = -half_max(row ? (m[g] > -3.0e38f ? -m[g] : INFINITY) : -INFINITY);
+    if (lane == 0) {
+      bound[wave][2 * g] = sqrtf(qn);
+      bound[wave][2 * g + 1] = ml;
+    }
+  }
+  __syncthreads();
+  float a[G], b[G];   // log2 weight <= a kn + b - F log2e - REACH_ZERO for every query of the workgroup
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    float qn = bound[0][2 * g], ml = bound[0][2 * g + 1];
+#pragma unroll
+    for (int w = 1; w < NWAVES; ++w) {
+      qn = fmaxf(qn, bound[w][2 * g]);
+      ml = fminf(ml, bound[w][2 * g + 1]);
+    }
+    a[g] = qn * scale * REACH_Q;
+    b[g] = REACH_ZERO - ml;
+  }
+  const int all = (cut + 63) / 64, nwords = min(all, REACH_MASK_WORDS), first = 64 * (all - nwords);
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)crow, 0, (int)((int64_t)Tk * 4), RSRC_WORD3);
+  for (int w = wave; w < nwords; w += NWAVES) {
+    const int kt = first + 64 * w + lane, ktc = min(kt, cut - 1);
+    bool skip = kt >= i_lo && kt < cut;   // every comparison that meets a NaN keeps the tile
+    float thr = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const float t = fmaf(a[g], kn[(int64_t)g * NKT + ktc], b[g]);
+      skip = skip && t < INFINITY;
+      thr = fmaxf(thr, t);
+    }
+    skip = skip && kt_min[ktc] * REACH_F > thr;   // (its total is at least its history at any query)
+    if (__any(skip)) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const auto x = __builtin_amdgcn_raw_buffer_load_b128(rs, ktc * (TILE * 4) + 16 * c, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) skip = skip && __uint_as_float(x[e]) * REACH_F > thr;
+      }
+    }
+    const uint64_t bits = __ballot(kt < cut && !skip);
+    if (lane == 0) words[w] = bits;
+  }
+  __syncthreads();
+  if (wave == 0) write_reach_runs(runs, words, nwords, first, lane);
+  __syncthreads();
+}
+
+// ---------------------------------------------------------------------------------------------
 // Selection column sums: colsum[b][rb][j] = sum over the queries r of block rb (chunk-relative)
 // of S[r, j]. One wavefront per key block (its K rows in registers); a workgroup walks RB query
-// blocks, each staged once in LDS for its four wavefronts while the next one loads.
+// blocks, each staged once in LDS for its four wavefronts while the next one loads. The grid's z past the
+// sequences takes the key norms (key_norms_block) of all heads along: work of the same launch that the
+// forward needs next to the carry, in place of a launch of its own (2-3 us).
 constexpr int SEL_RB = 8;   // query blocks per workgroup
 
 template <class OP, int D>
 __global__ __launch_bounds__(NTHREADS) void sel_colsum_kernel(
     const typename OP::elem* __restrict__ q, const typename OP::elem* __restrict__ k,
     float* __restrict__ colsum, int H, int Tq, int Tk, Strides qs, Strides ks, int q_off, int exempt, float scale,
-    int RB) {
+    int RB, const typename OP::elem* __restrict__ v, Strides vs, int nseq, float* __restrict__ kn) {
   using elem = typename OP::elem;
+  if ((int)blockIdx.z >= nseq) {
+    const int nkb = (Tk + NORM_KEYS - 1) / NORM_KEYS;
+    const int64_t e = ((int64_t)(blockIdx.z - nseq) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    if (e < (int64_t)nseq * H * nkb) key_norms_block<elem, D>(k, v, ks, vs, H, Tk, kn, (int)(e / nkb), (int)(e % nkb));
+    return;
+  }
   using frag = typename OP::frag;
   constexpr int NS = D / OP::KS;
   constexpr int LDK = D + OP::KPAD;
@@ -741,10 +1000,11 @@ __global__ __launch_bounds__(NTHREADS) void sel_colsum_kernel(
 }
 
 // carry[b][rb][j] = state_in[b][j] + sum_{rb' < rb} colsum[b][rb'][j] (in place);
-// state_out[b][j] = the sum over all blocks. state_in is read for j < q_off only.
+// state_out[b][j] = the sum over all blocks. state_in is read for j < q_off only. kt (may be NULL):
+// the smallest of them in each key tile (of its 32 keys: a last tile with fewer holds no such figure).
 __global__ __launch_bounds__(NTHREADS) void sel_scan_kernel(
     float* __restrict__ carry, const float* state_in, float* state_out, int64_t state_ld,
-    int NBq, int Tk, int q_off) {
+    int NBq, int Tk, int q_off, float* __restrict__ kt) {
   const int j = blockIdx.x * NTHREADS + threadIdx.x;
   const int b = blockIdx.y;
   if (j >= Tk) return;
@@ -768,6 +1028,10 @@ __global__ __launch_bounds__(NTHREADS) void sel_scan_kernel(
     run += c;
   }
   state_out[(int64_t)b * state_ld + j] = run;
+  if (kt) {   // (lanes past the last key have left: a half-wavefront's first lane is never one of them)
+    const float mn = -half_max(-run);
+    if ((threadIdx.x & 31) == 0) kt[(int64_t)b * ((Tk + TILE - 1) / TILE) + j / TILE] = mn;
+  }
 }
 
 // The selection carry in one pass, for bf16 storage at head dim 64 when the call has key blocks
@@ -795,7 +1059,7 @@ constexpr int SEL_CARRY_MIN_BLOCKS = 256;    // workgroups below which the two-k
 __global__ __launch_bounds__(NTHREADS) void sel_carry64_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, float* __restrict__ carry,
     const float* state_in, float* state_out, int64_t state_ld, int Tq, int Tk, Strides qs, Strides ks, int q_off,
-    int exempt, float scale) {
+    int exempt, float scale, float* __restrict__ kt) {
   using OP = OpBF16;
   using frag = OP::frag;
   constexpr int D = 64, NS = 4, KPW = SEL_CARRY_KPW, NBUF = SEL_CARRY_NBUF, AHEAD = NBUF - 1;
@@ -914,16 +1178,21 @@ __global__ __launch_bounds__(NTHREADS) void sel_carry64_kernel(
   if (t + 2 < nb) step(t + 2, std::integral_constant<int, 2>{});
   wait_loads();   // nothing may be left in flight into LDS when the workgroup ends
 #pragma unroll
-  for (int u = 0; u < KPW; ++u)
+  for (int u = 0; u < KPW; ++u) {
     if (owner[u]) state_out[(int64_t)b * state_ld + jj[u]] = run[u];
+    if (kt) {
+      const float mn = -half_max(owner[u] ? -run[u] : -INFINITY);
+      if (lane == 0 && kb[u] < NKT) kt[(int64_t)b * NKT + kb[u]] = mn;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
 // Forward. grid (ceil(NBq/4), nseq * H/G); wavefront w of block x owns query block
 // (gridDim.x-1-x)*4 + w (heavy causal rows launch first) of heads [gi*G, gi*G+G). Key tiles are
 // visited newest first, so each row's maximum is usually settled by its diagonal tile and later
-// tiles rarely trigger a rescale of the output (skipped when no lane's maximum rises). The next
-// tile's K, V^T and carry rows are loaded while the current one is computed (double-buffered LDS).
+// tiles rarely trigger a rescale of the output (skipped when no lane's maximum rises). Tiles whose keys
+// carry no weight any more are left out (find_reach). The next tile's K, V^T and carry rows are loaded while the current one is computed (double-buffered LDS).
 
 // Workgroups per CU the forward's register allocation must allow: three at bf16 head dims <= 64
 // with one head per wavefront (its LDS fits three), which holds it to 168 registers without spills.
@@ -939,7 +1208,8 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
     const typename OP::elem* __restrict__ vt, const float* __restrict__ carry,
     float* __restrict__ out, float* __restrict__ rmax, float* __restrict__ rden,
     typename OP::elem* __restrict__ y, Strides ys, int H, int Tq, int Tk, Strides qs, Strides ks, int q_off,
-    int64_t ldv, int exempt, float scale, int damp_mode, float train_len) {
+    int64_t ldv, int exempt, float scale, int damp_mode, float train_len, const float* __restrict__ kn,
+    const float* __restrict__ kt_min) {
   using elem = typename OP::elem;
   using frag = typename OP::frag;
   constexpr int NS = D / OP::KS;          // MFMA steps over D
@@ -958,6 +1228,9 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
   constexpr int LDF = TILE + 4;
   __shared__ __attribute__((aligned(16))) float sF[NWAVES][TILE * LDF];   // each wavefront's F tile
   __shared__ __attribute__((aligned(16))) float sDamp[NWAVES][TILE];      // its queries' damping factors
+  __shared__ uint64_t sMask[REACH_MASK_WORDS];    // the tiles to visit, as bits and as runs (find_reach)
+  __shared__ TileRun sRuns[REACH_RUNS];
+  __shared__ float sBound[NWAVES][2 * G];         // per wavefront and head: max |q|, min row maximum
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
@@ -1066,6 +1339,15 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
     if (tid < NWAVES * TILE) sC[buf][tid >> 5][tid & (TILE - 1)] = nC_ok ? nC * neg_inv_scale : 0.f;
   };
 
+  // The tiles in the order of the sweep: cur, then nxt (negative: none), newest first; those reaching
+  // past the workgroup's first query and one more (down to cut) always, the rest as far as their keys
+  // carry weight (find_reach)
+  const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
+  const int i_hi = max(i_lo, min(min(q_off + qsb * NWAVES * TILE, Tk) / TILE, wg_end));
+  const int cut = max(0, i_hi - 1);
+  int cur = wg_end - 1, nxt = wg_end - 2, t = 0;
+  const float oldest = reach_total(kt_min != nullptr ? kt_min + (int64_t)b * NKT : nullptr, cut, lane);
+
   // the next key tile is loaded into registers while this one is computed (stored to the other LDS
   // buffer after it)
   load_tile(wg_end - 1);
@@ -1075,12 +1357,12 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
   // one key tile; INTERIOR: every key of the tile strictly precedes every query of the workgroup,
   // lies before the end and is not exempt, for every wavefront (straight-line code without masks)
   // DAMP: history damping on (a compile-time fact, so the undamped loops carry no branch for it)
-  auto tile_step = [&](int t, auto interior_tag, auto damp_tag) __attribute__((always_inline)) {
+  auto tile_step = [&](auto interior_tag, auto damp_tag) __attribute__((always_inline)) {
     constexpr bool INTERIOR = decltype(interior_tag)::value;
     constexpr bool DAMP = decltype(damp_tag)::value;
-    const int kt = wg_end - 1 - t;
+    const int kt = cur;
     const int buf = NBUF == 2 ? (t & 1) : 0;
-    if (t + 1 < wg_end) load_tile(kt - 1);
+    if (nxt >= 0) load_tile(nxt);
     if (kt < my_end) {   // (a wavefront past the last query block has none)
       const int kbase = kt * TILE;
       // edge: some key of the tile does not strictly precede every query of the block, lies past
@@ -1201,18 +1483,33 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
       body();
     }
     if constexpr (NBUF == 1) __syncthreads();   // the one buffer is free again
-    if (t + 1 < wg_end) store_tile(NBUF == 2 ? buf ^ 1 : 0);
+    if (nxt >= 0) store_tile(NBUF == 2 ? buf ^ 1 : 0);
     __syncthreads();
   };
   // key tiles newest first: the diagonals and the sequence end, the interior tiles
   // [i_lo, i_hi), then the tiles holding exempt keys
-  const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
-  const int i_hi = max(i_lo, min(min(q_off + qsb * NWAVES * TILE, Tk) / TILE, wg_end));
   auto sweep = [&](auto damp_tag) {
-    int t = 0;
-    for (; t < wg_end - i_hi; ++t) tile_step(t, std::false_type{}, damp_tag);
-    for (; t < wg_end - i_lo; ++t) tile_step(t, std::true_type{}, damp_tag);
-    for (; t < wg_end; ++t) tile_step(t, std::false_type{}, damp_tag);
+    int run_lo = INT_MIN, run_i = 0;   // the run nxt lies in
+    auto shift = [&]() {
+      cur = nxt;
+      ++t;
+      if (__builtin_expect(--nxt < run_lo, 0)) {
+        const TileRun r = sRuns[run_i++];
+        nxt = __builtin_amdgcn_readfirstlane(r.hi);
+        run_lo = __builtin_amdgcn_readfirstlane(r.lo);
+      }
+    };
+    for (; cur >= i_hi; shift()) tile_step(std::false_type{}, damp_tag);
+    nxt = cut - 1;   // the tiles below cut: all of them, or the runs found
+    if (reach_worth(oldest)) {
+      find_reach<OP, G, NS>(qf, m, q_rel < Tq, scale, kn + (seq_row + hd0) * NKT, kt_min + (int64_t)b * NKT, NKT,
+                            carry + ((int64_t)b * NBq + qsb * NWAVES) * Tk, Tk, cut, i_lo, sBound, sMask, sRuns, lane, wave);
+      const TileRun r = sRuns[run_i++];
+      nxt = __builtin_amdgcn_readfirstlane(r.hi);
+      run_lo = __builtin_amdgcn_readfirstlane(r.lo);
+    }
+    for (; cur >= i_lo; shift()) tile_step(std::true_type{}, damp_tag);
+    for (; cur >= 0; shift()) tile_step(std::false_type{}, damp_tag);
   };
   if (damp_mode != 0) sweep(std::true_type{});
   else sweep(std::false_type{});
@@ -1283,7 +1580,8 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const float* __restrict__ carry, float* __restrict__ out, float* __restrict__ rmax, float* __restrict__ rden,
     uint16_t* __restrict__ y, Strides ys, int H, int Tq, int Tk, Strides qs, Strides ks, Strides vs, int q_off,
-    int exempt, float scale, int damp_mode, float train_len) {
+    int exempt, float scale, int damp_mode, float train_len, const float* __restrict__ kn,
+    const float* __restrict__ kt_min) {
   using OP = OpBF16;
   using elem = uint16_t;
   using frag = OP::frag;
@@ -1310,11 +1608,17 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
   //             the writes across the step's barrier.
   //   sDamp     per wavefront, its queries' damping factors: written once before the prologue's
   //             barrier, read only after it.
+  //   sBound, sMask, sRuns  written once, in find_reach (after the barrier that ends the last diagonal tile), each
+  //             with a barrier between its writes and its reads.
+  // (tile t: the t-th tile visited; without skipping it is key tile wg_end - 1 - t)
   __shared__ FwdTileBuf64<G> sB0, sB1;   // tile t's K and V rows in buffer t mod 2
   __shared__ FwdSelBuf64 sS0, sS1;    // tile t's head-0 K rows and carry rows in buffer t mod 2
   constexpr int LDF = TILE + 4;
   __shared__ __attribute__((aligned(16))) float sF[NWAVES][TILE * LDF];   // each wavefront's F tile
   __shared__ __attribute__((aligned(16))) float sDamp[NWAVES][TILE];      // its queries' damping factors
+  __shared__ uint64_t sMask[REACH_MASK_WORDS];    // the tiles to visit, as bits and as runs (find_reach)
+  __shared__ TileRun sRuns[REACH_RUNS];
+  __shared__ float sBound[NWAVES][2 * G];         // per wavefront and head: max |q|, min row maximum
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
@@ -1461,6 +1765,16 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
     }
   };
 
+  // The tiles in the order of the sweep: cur, then n1 and n2 (-1: none), newest first. Every tile down to
+  // `cut` -- those reaching past the workgroup's first query, and two more, so that the loads one and
+  // two tiles ahead never run past what is known -- is visited; the rest as far as its keys carry
+  // weight, once the row maxima of the diagonal tiles are known (find_reach).
+  const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
+  const int i_hi = max(i_lo, min(min(q_off + qsb * NWAVES * TILE, Tk) / TILE, wg_end));
+  const int cut = max(0, i_hi - 2);
+  int cur = wg_end - 1, n1 = wg_end - 2, n2 = wg_end - 3;
+  const float oldest = reach_total(kt_min != nullptr ? kt_min + (int64_t)b * NKT : nullptr, cut, lane);
+
   // the first tile's operands, head-0 rows and carry of the first two (its F at the sweep's start)
   load_tile(wg_end - 1, sB0);
   load_sel(wg_end - 1, sS0);
@@ -1468,18 +1782,18 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
   wait_loads();
   __syncthreads();
 
-  // tile t (buffer t mod 2, named by ODD); INTERIOR and DAMP as in fwd_kernel (INTERIOR for tile t;
-  // the selection of tile t + 1 checks its own tile)
-  auto tile_step = [&](int t, auto interior_tag, auto damp_tag, auto odd_tag) __attribute__((always_inline)) {
+  // the t-th tile of the sweep, cur (buffer t mod 2, named by ODD); INTERIOR and DAMP as in fwd_kernel
+  // (INTERIOR for this tile; the selection of the next one checks its own tile)
+  auto tile_step = [&](auto interior_tag, auto damp_tag, auto odd_tag) __attribute__((always_inline)) {
     constexpr bool INTERIOR = decltype(interior_tag)::value;
     constexpr bool DAMP = decltype(damp_tag)::value;
     constexpr bool ODD = decltype(odd_tag)::value;
     FwdTileBuf64<G>& B = ODD ? sB1 : sB0;
-    const int kt = wg_end - 1 - t;
-    // free since the last barrier: the other tile buffer, and this parity's head-0 buffer (tile t's
-    // rows were used by the selection of tile t during tile t - 1)
-    if (t + 1 < wg_end) load_tile(kt - 1, ODD ? sB0 : sB1);
-    if (t + 2 < wg_end) load_sel(kt - 2, ODD ? sS1 : sS0);
+    const int kt = cur;
+    // free since the last barrier: the other tile buffer, and this parity's head-0 buffer (this tile's
+    // rows were used by its selection during the tile before)
+    if (n1 >= 0) load_tile(n1, ODD ? sB0 : sB1);
+    if (n2 >= 0) load_sel(n2, ODD ? sS1 : sS0);
     if (kt < my_end) {   // (a wavefront past the last query block has none)
       const int kbase = kt * TILE;
       const bool edge =
@@ -1545,29 +1859,55 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
       }
     }
     // the next tile's F (after this tile's reads of the wavefront's F rows, in program order)
-    if (t + 1 < wg_end && kt - 1 < my_end) select(kt - 1, ODD ? sS0 : sS1, damp_tag);
+    if (n1 >= 0 && n1 < my_end) select(n1, ODD ? sS0 : sS1, damp_tag);
     wait_loads();
     __syncthreads();   // the next tile's operands are in; every wavefront is done with this one
   };
-  const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
-  const int i_hi = max(i_lo, min(min(q_off + qsb * NWAVES * TILE, Tk) / TILE, wg_end));
   auto sweep = [&](auto damp_tag) {
     if (wg_end - 1 < my_end) select(wg_end - 1, sS0, damp_tag);   // the first tile's F
     // The first tile step loads tile 2's head-0 K rows into sS0, whose rows every wavefront has
     // just read for that F: all of them must be past their reads first.
     __syncthreads();
-    auto run = [&](int t0, int t1, auto interior_tag) {
-      int t = t0;
-      if (t < t1 && (t & 1)) tile_step(t++, interior_tag, damp_tag, std::true_type{});
-      for (; t + 1 < t1; t += 2) {
-        tile_step(t, interior_tag, damp_tag, std::false_type{});
-        tile_step(t + 1, interior_tag, damp_tag, std::true_type{});
+    // tiles from cur down to `stop`, in pairs (buffer 0, buffer 1); run_lo, run_i: the run n2 lies in
+    bool odd = false;
+    int run_lo = INT_MIN, run_i = 0;
+    auto shift = [&]() {
+      cur = n1;
+      n1 = n2;
+      if (__builtin_expect(--n2 < run_lo, 0)) {
+        const TileRun r = sRuns[run_i++];
+        n2 = __builtin_amdgcn_readfirstlane(r.hi);
+        run_lo = __builtin_amdgcn_readfirstlane(r.lo);
       }
-      if (t < t1) tile_step(t, interior_tag, damp_tag, std::false_type{});
     };
-    run(0, wg_end - i_hi, std::false_type{});
-    run(wg_end - i_hi, wg_end - i_lo, std::true_type{});
-    run(wg_end - i_lo, wg_end, std::false_type{});
+    auto run = [&](int stop, auto interior_tag) {
+      if (odd && cur >= stop) {
+        tile_step(interior_tag, damp_tag, std::true_type{});
+        shift();
+        odd = false;
+      }
+      while (cur >= stop) {
+        tile_step(interior_tag, damp_tag, std::false_type{});
+        shift();
+        if (cur < stop) {
+          odd = true;
+          break;
+        }
+        tile_step(interior_tag, damp_tag, std::true_type{});
+        shift();
+      }
+    };
+    run(i_hi, std::false_type{});
+    n2 = cut - 1;   // the tiles below cut: all of them, or the runs found
+    if (reach_worth(oldest)) {
+      find_reach<OP, G, NS>(qf, m, q_rel < Tq, scale, kn + (seq_row + hd0) * NKT, kt_min + (int64_t)b * NKT,
+                            NKT, carry + ((int64_t)b * NBq + qsb * NWAVES) * Tk, Tk, cut, i_lo, sBound, sMask, sRuns, lane, wave);
+      const TileRun r = sRuns[run_i++];
+      n2 = __builtin_amdgcn_readfirstlane(r.hi);
+      run_lo = __builtin_amdgcn_readfirstlane(r.lo);
+    }
+    run(i_lo, std::true_type{});
+    run(0, std::false_type{});
   };
   if (damp_mode != 0) sweep(std::true_type{});
   else sweep(std::false_type{});
@@ -3439,6 +3779,7 @@ template <class OP, int D>
 int run_selection(const FwdCall& c, hipStream_t st) {
   using elem = typename OP::elem;
   const int NBq = (int)cdiv(c.Tq, TILE), NKT = (int)cdiv(c.Tk, TILE);
+  const int64_t nkb = cdiv(c.Tk, NORM_KEYS);
   TimedLaunch timed(SA_KERNEL_SELECTION, st);
   if constexpr (sizeof(elem) == 2 && D == 64) {
     const int64_t wgs = cdiv(NKT, NWAVES * SEL_CARRY_KPW);
@@ -3446,18 +3787,23 @@ int run_selection(const FwdCall& c, hipStream_t st) {
     if (wgs * c.nseq >= SEL_CARRY_MIN_BLOCKS && (int64_t)NBq * c.Tk * 4 < ((int64_t)1 << 31)) {
       hipLaunchKernelGGL(sel_carry64_kernel, dim3((unsigned)wgs, (unsigned)c.nseq), dim3(NTHREADS), 0,
                          st, static_cast<const uint16_t*>(c.q), static_cast<const uint16_t*>(c.k), c.carry,
-                         c.state_in, c.state_out, c.state_ld, c.Tq, c.Tk, c.qs, c.ks, c.q_off, c.exempt, c.scale);
+                         c.state_in, c.state_out, c.state_ld, c.Tq, c.Tk, c.qs, c.ks, c.q_off, c.exempt, c.scale, c.kt);
+      if (c.kn)
+        hipLaunchKernelGGL((key_norms_kernel<elem, D>), dim3((unsigned)nkb, (unsigned)(c.nseq * c.H)), dim3(NTHREADS), 0,
+                           st, static_cast<const elem*>(c.k), static_cast<const elem*>(c.v), c.ks, c.vs, c.H, c.Tk,
+                           c.kn);
       return launch_status();
     }
   }
   const int RB = SEL_RB;
   dim3 g1((unsigned)cdiv(NKT, NWAVES), (unsigned)cdiv(NBq, RB), (unsigned)c.nseq);
+  if (c.kn) g1.z += (unsigned)cdiv((int64_t)c.nseq * c.H * nkb, (int64_t)g1.x * g1.y);   // the key norms' workgroups
   hipLaunchKernelGGL((sel_colsum_kernel<OP, D>), g1, dim3(NTHREADS), 0, st, static_cast<const elem*>(c.q),
                      static_cast<const elem*>(c.k), c.carry, c.H, c.Tq, c.Tk, c.qs, c.ks, c.q_off, c.exempt, c.scale,
-                     RB);
+                     RB, static_cast<const elem*>(c.v), c.vs, c.nseq, c.kn);
   dim3 g2((unsigned)cdiv(c.Tk, NTHREADS), (unsigned)c.nseq);
   hipLaunchKernelGGL(sel_scan_kernel, g2, dim3(NTHREADS), 0, st, c.carry, c.state_in, c.state_out, c.state_ld, NBq,
-                     c.Tk, c.q_off);
+                     c.Tk, c.q_off, c.kt);
   return launch_status();
 }
 
@@ -3475,7 +3821,7 @@ void launch_fwd(const FwdCall& c, const typename OP::elem* vt, int64_t ldv) {   
   hipLaunchKernelGGL((fwd64_kernel<CVV, G>), grid, dim3(NTHREADS), 0, c.st, static_cast<const elem*>(c.q),       \
                      static_cast<const elem*>(c.k), static_cast<const elem*>(c.v), c.carry, c.out, c.rmax,        \
                      c.rden, static_cast<elem*>(c.y), c.ys, c.H, c.Tq, c.Tk, c.qs, c.ks, c.vs, c.q_off, c.exempt, \
-                     c.scale, c.damp_mode, c.train_len)
+                     c.scale, c.damp_mode, c.train_len, c.kn, c.kt)
     if (cv) SA_LAUNCH_FWD64(true);
     else SA_LAUNCH_FWD64(false);
 #undef SA_LAUNCH_FWD64
@@ -3483,7 +3829,8 @@ void launch_fwd(const FwdCall& c, const typename OP::elem* vt, int64_t ldv) {   
 #define SA_LAUNCH_FWD(CVV)                                                                                        \
   hipLaunchKernelGGL((fwd_kernel<OP, D, G, CVV>), grid, dim3(NTHREADS), 0, c.st, static_cast<const elem*>(c.q),  \
                      static_cast<const elem*>(c.k), vt, c.carry, c.out, c.rmax, c.rden, static_cast<elem*>(c.y),  \
-                     c.ys, c.H, c.Tq, c.Tk, c.qs, c.ks, c.q_off, ldv, c.exempt, c.scale, c.damp_mode, c.train_len)
+                     c.ys, c.H, c.Tq, c.Tk, c.qs, c.ks, c.q_off, ldv, c.exempt, c.scale, c.damp_mode, c.train_len, c.kn, \
+                     c.kt)
     if (cv) SA_LAUNCH_FWD(true);
     else SA_LAUNCH_FWD(false);
 #undef SA_LAUNCH_FWD

@@ -201,6 +201,12 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def _forward_scratch(lib, batch: int, heads: int, tk: int, kdim: int, code: int, group: int) -> int:
+    """Bytes of sa_forward's workspace, the part for skipping tiles without weight included."""
+    return max(int(lib.sa_forward_workspace_bytes(batch, heads, tk, kdim, code, group))
+               + int(lib.sa_reach_bytes(batch, heads, tk, kdim)), 1)
+
+
 def _launch_forward(qs: Tensor, ks: Tensor, vs: Tensor, kstride: int, scale: float, exempt: int, group: int,
                     damp_mode: int, train_len: int, state_in: Tensor | None = None, q_offset: int = 0,
                     state: Tensor | None = None):
@@ -220,8 +226,7 @@ def _launch_forward(qs: Tensor, ks: Tensor, vs: Tensor, kstride: int, scale: flo
     carry = torch.empty(batch, nb, tk, device=dev, dtype=torch.float32)
     if state is None:
         state = torch.empty(batch, tk, device=dev, dtype=torch.float32)
-    ws = torch.empty(max(int(lib.sa_forward_workspace_bytes(batch, heads, tk, kdim, code, group)), 1), device=dev,
-                     dtype=torch.uint8)
+    ws = torch.empty(_forward_scratch(lib, batch, heads, tk, kdim, code, group), device=dev, dtype=torch.uint8)
     with torch.cuda.device(dev):
         _lib.check(lib.sa_forward(
             qs.data_ptr(), ks.data_ptr(), vs.data_ptr(), out.data_ptr(), rmax.data_ptr(), rden.data_ptr(),
@@ -304,8 +309,7 @@ def _qkv_forward_op(qkv: Tensor, heads: int, exempt: int) -> tuple[Tensor, Tenso
     rden = torch.empty(batch, heads, seq, device=dev, dtype=torch.float32)
     carry = torch.empty(batch, (seq + CARRY_M - 1) // CARRY_M, seq, device=dev, dtype=torch.float32)
     state = torch.empty(batch, seq, device=dev, dtype=torch.float32)
-    ws = torch.empty(max(int(lib.sa_forward_workspace_bytes(batch, heads, seq, head_dim, code, 0)), 1), device=dev,
-                     dtype=torch.uint8)
+    ws = torch.empty(_forward_scratch(lib, batch, heads, seq, head_dim, code, 0), device=dev, dtype=torch.uint8)
     qkv_s, y_s = _packed_strides(batch, seq, heads, head_dim)
     base = qkv.data_ptr()
     with torch.cuda.device(dev):

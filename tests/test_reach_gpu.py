@@ -1,0 +1,84 @@
+"""Leaving out the tiles without weight keeps every bit: the C ABI called with the scratch that finds them
+(sa_reach_bytes) and without it, on inputs whose histories outgrow their logits, on inputs whose histories
+do not, and on inputs that are not finite or too large for the bound. The kernels' results against the
+oracle are the other tests' matter."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from selective_attention import _lib, kernels
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(t):
+    return t.contiguous().view(torch.int16 if t.element_size() == 2 else torch.int32)
+
+
+def _inputs(cuda, b, h, t, d, dtype, kind, seed=11):
+    g = torch.Generator(device=cuda).manual_seed(seed)
+    q, k, v, do = (torch.randn(b, h, t, d, device=cuda, generator=g) for _ in range(4))
+    if kind == "sparse":      # few positive selector logits: no tile can be left out
+        q[:, 0] += math.sqrt(3.0 * math.sqrt(d) / d)
+        k[:, 0] -= math.sqrt(3.0 * math.sqrt(d) / d)
+    elif kind == "holes":     # a few keys that nobody selects among selected ones: short and long runs
+        k[:, 0, torch.arange(5, t, 97, device=cuda)] = 0.0
+    elif kind == "special":   # values a zero weight does not silence, keys and queries beyond the bound
+        v[:, -1, 3] = float("inf")
+        v[:, 0, 200] = float("nan")
+        k[:, -1, 70] = 3e18
+        q[:, 0, t - 3] = 1e19
+        do[:, -1, t - 5, 0] = float("inf")
+    return tuple(x.to(dtype) for x in (q, k, v, do))
+
+
+def _forward(q, k, v, exempt, reach, chunk=0, group=0):
+    """sa_forward over the last `chunk` queries (0: all) with or without the scratch of sa_reach_bytes."""
+    lib = _lib.load()
+    b, h, tk, d = k.shape
+    tq = chunk or tk
+    dev, code = q.device, kernels._code_of(q)
+    qs = q[:, :, tk - tq:].contiguous()
+    out, rmax, rden = (torch.empty(b, h, tq, *s, device=dev) for s in ((d,), (), ()))
+    carry = torch.empty(b, (tq + 31) // 32, tk, device=dev)
+    g = torch.Generator(device=dev).manual_seed(3)
+    pos = torch.arange(tk, device=dev)
+    state = (0.4 * (tk - tq - 1 - pos).clamp_min(0)).expand(b, tk) + torch.rand(b, tk, device=dev, generator=g)
+    state[:, :exempt] = 0.0
+    base = lib.sa_forward_workspace_bytes(b, h, tk, d, code, group)
+    size = base + (lib.sa_reach_bytes(b, h, tk, d) if reach else 0)
+    ws = torch.empty(max(size, 1), dtype=torch.uint8, device=dev)
+    _lib.check(lib.sa_forward(qs.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), rmax.data_ptr(),
+                              rden.data_ptr(), carry.data_ptr(), state.data_ptr() if chunk else None, state.data_ptr(), tk,
+                              ws.data_ptr(), size, b, h, tq, tk, tk - tq, 0, d, 1 / math.sqrt(d), code, exempt, group, 0, 0,
+                              torch.cuda.current_stream().cuda_stream))
+    return out, rmax, rden, carry, state
+
+
+# (B, H, T, D, dtype): both widths of the head-dim-64 forward and odd head counts, the other head dims and
+# group widths, fp32; lengths around tiles, workgroups and mask words
+SHAPES = [(1, 2, 1024, 64, "bf16"), (2, 3, 2081, 64, "bf16"), (1, 16, 8200, 64, "bf16"), (3, 1, 4127, 64, "bf16"),
+          (1, 4, 1500, 32, "bf16"), (1, 2, 2049, 128, "bf16"), (1, 2, 1377, 64, "f32"), (1, 1, 1111, 32, "f32"),
+          (1, 2, 1056, 128, "f32")]
+
+
+@pytest.mark.parametrize("kind", ["normal", "holes", "sparse", "special"])
+@pytest.mark.parametrize("b,h,t,d,dtype", SHAPES)
+def test_forward_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
+    print(f"case forward {b} {h} {t} {d} {dtype} {kind}", flush=True)
+    q, k, v, _ = _inputs(cuda, b, h, t, d, torch.bfloat16 if dtype == "bf16" else torch.float32, kind)
+    for exempt, chunk in ((1, 0), (16, 0), (40, 0), (3, 77), (1, 300)):
+        for got, want in zip(_forward(q, k, v, exempt, True, chunk), _forward(q, k, v, exempt, False, chunk)):
+            assert torch.equal(_bits(got), _bits(want)), (exempt, chunk)
+
+
+def test_forward_past_the_mask_keeps_its_bits(cuda):
+    """More key tiles than a workgroup's mask holds (128 words of 64): the oldest are all visited."""
+    t = 64 * 32 * 128 + 3000
+    q, k, v, _ = _inputs(cuda, 1, 1, t, 64, torch.bfloat16, "normal")
+    for got, want in zip(_forward(q, k, v, 1, True, 500), _forward(q, k, v, 1, False, 500)):
+        assert torch.equal(_bits(got), _bits(want))
