@@ -80,10 +80,11 @@ int64_t sa_transposed_ld(int64_t t);
  * reads the value rows themselves (workspace may then be NULL). */
 int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int64_t head_dim, int dtype, int group);
 
-/* Optional bytes of scratch beyond sa_forward_workspace_bytes (-1 for invalid sizes): given a workspace
- * larger by this much, sa_forward skips the key tiles whose softmax weights are exact fp32 zeros because
- * their history has outgrown every logit. The results have the same bits with and without it. t: the
- * number of keys. */
+/* Optional bytes of scratch beyond sa_forward_workspace_bytes and sa_backward_workspace_bytes (-1 for
+ * invalid sizes): given a workspace larger by this much, sa_forward and sa_backward leave out the tiles
+ * whose softmax weights are exact fp32 zeros because their keys' history has outgrown every logit. The
+ * results have the same bits with and without it, but for the gradients of at most 32 exempt keys, which
+ * the backward then sums in another order. t: the number of keys. */
 int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim);
 
 /*

@@ -15,6 +15,8 @@
 #   sa_bf16_kvg.hip  the bf16 key-side instances at head dims 32 and 128: accumulators in VGPRs,
 #                the default scheduler (the two options together crash this compiler on them)
 #   sa_bf16_dec.hip  the bf16 decode-step kernels, the default scheduler (faster for them)
+#   sa_bf16_prep.hip  the bf16 backward preparation, the compiler's own accumulator placement (the
+#                options of sa_bf16.hip crash this compiler on one of its instances)
 #   sa_f32.hip   fp32-storage kernels, the compiler's own accumulator placement
 #   sa_abi.hip   the C ABI (host code only)
 # Every HIP compile: -packed-fp32-ops off (no v_pk_*_f32 from the compiler).
@@ -54,6 +56,8 @@ unit sa_bf16_kvg.hip sa_bf16_kvg.o -mllvm -amdgpu-mfma-vgpr-form &
 p6=$!
 unit sa_bf16_dec.hip sa_bf16_dec.o -mllvm -amdgpu-mfma-vgpr-form &
 p5=$!
+unit sa_bf16_prep.hip sa_bf16_prep.o &
+p8=$!
 unit sa_f32.hip sa_f32.o &
 p2=$!
 unit sa_abi.hip sa_abi.o &
@@ -66,8 +70,9 @@ wait $p4 || rc=1
 wait $p5 || rc=1
 wait $p6 || rc=1
 wait $p7 || rc=1
+wait $p8 || rc=1
 [ $rc -eq 0 ] || { echo "build.sh: a compile failed" >&2; exit 1; }
-hipcc --offload-arch=gfx950 -shared -fPIC "$tmp/sa_bf16.o" "$tmp/sa_bf16_kv.o" "$tmp/sa_bf16_kv1.o" "$tmp/sa_bf16_kvg.o" "$tmp/sa_bf16_dec.o" "$tmp/sa_f32.o" \
+hipcc --offload-arch=gfx950 -shared -fPIC "$tmp/sa_bf16.o" "$tmp/sa_bf16_kv.o" "$tmp/sa_bf16_kv1.o" "$tmp/sa_bf16_kvg.o" "$tmp/sa_bf16_dec.o" "$tmp/sa_bf16_prep.o" "$tmp/sa_f32.o" \
   "$tmp/sa_abi.o" \
   -o "$out.tmp"
 mv "$out.tmp" "$out"

@@ -78,7 +78,7 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
 
 int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim) {
   if (!valid_dims(nseq, heads, t) || (head_dim != 32 && head_dim != 64 && head_dim != 128)) return -1;
-  return fwd_reach_bytes(nseq, heads, t);
+  return std::max(fwd_reach_bytes(nseq, heads, t), bwd_reach_layout(nseq, heads, t, head_dim).total);
 }
 
 int sa_forward(const void* q, const void* k, const void* v, float* out, float* rmax, float* rden, float* carry,
@@ -229,6 +229,10 @@ int sa_backward_strided(const void* q, const sa_view_strides* q_strides, const v
   c.dk = dk;
   c.dv = dv;
   c.ws = workspace;
+  const int64_t base = sa_backward_workspace_bytes(nseq, heads, t, head_dim, dtype, group);
+  if (t >= REACH_MIN_KEYS && workspace_bytes >= base + bwd_reach_layout(nseq, heads, t, head_dim).total &&
+      (uintptr_t)workspace % 16 == 0)
+    c.reach = static_cast<char*>(workspace) + base;
   c.dqs = st(dq_strides);
   c.dks = st(dk_strides);
   c.dvs = st(dv_strides);

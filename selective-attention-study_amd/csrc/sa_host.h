@@ -179,6 +179,31 @@ inline BwdLayout bwd_layout(int64_t nseq, int64_t heads, int64_t t, int64_t D, i
 constexpr int REACH_MIN_KEYS = 1024;
 constexpr int REACH_MASK_WORDS = 128;   // a workgroup's tile mask: its newest 64 * 128 key tiles
 
+// Backward: per head and QSTAT_ROWS rows the largest query norm and the least lse; per head group and 128
+// keys the last query block their weights reach; and the exempt keys' gradients, summed per QSTAT_ROWS
+// rows, where there are at most EXEMPT_APART of them (bwd_rowprep_kernel).
+constexpr int QSTAT_ROWS = 128;
+constexpr int EXEMPT_APART = 32;
+struct BwdReach {
+  float2* qstat;   // (nseq * heads, nseg); NULL: every causal tile
+  int* hi;         // (head groups, nseq, nkg)
+  float* xpart;    // (nseq * heads, nseg, xk, 2, D): dK (unscaled), dV of the exempt keys
+  int nseg, nkg;
+  int xk;          // exempt keys whose gradients come from xpart (0: none, the key side has them all)
+};
+struct BwdReachLayout {
+  int64_t qstat, hi, xpart, total;
+};
+inline BwdReachLayout bwd_reach_layout(int64_t nseq, int64_t heads, int64_t t, int64_t D) {
+  const int64_t R = nseq * heads, nseg = cdiv(t, QSTAT_ROWS);
+  BwdReachLayout L;
+  L.qstat = 0;
+  L.hi = align_up(R * nseg * 8, 256);
+  L.xpart = L.hi + align_up(R * cdiv(t, NWAVES * TILE) * 4, 256);
+  L.total = L.xpart + align_up(R * nseg * EXEMPT_APART * 2 * D * 4, 256);
+  return L;
+}
+
 inline int64_t fwd_reach_bytes(int64_t nseq, int64_t heads, int64_t tk) {
   return align_up(nseq * (heads + 1) * cdiv(tk, TILE) * 4, 256);
 }
@@ -242,6 +267,7 @@ struct BwdCall {
   Strides dos;
   const float *rmax, *rden, *carry;
   void *dq, *dk, *dv, *ws;
+  char* reach;   // bwd_reach_layout of scratch, NULL: every causal tile
   Strides dqs, dks, dvs;
   int nseq, H, T;
   float scale;
@@ -284,8 +310,16 @@ struct KvLaunch {
   int64_t ldt;
   int exempt;
   float scale;
+  BwdReach reach;
   hipStream_t st;
 };
+// The backward preparation's outputs (bwd_rowprep_kernel), for a launch from another translation unit.
+struct PrepLaunch {
+  float *lse, *ndbar;
+  int64_t ldt;
+  BwdReach reach;
+};
+SA_HIDDEN void launch_rowprep_bf16(const BwdCall& c, const PrepLaunch& p);            // sa_bf16_prep.hip
 SA_HIDDEN int launch_bwd_kv_bf16(int D, int G, bool cv, const KvLaunch& a);           // sa_bf16_kv.hip
 SA_HIDDEN int launch_bwd_kv_bf16_generic(int D, int G, bool cv, const KvLaunch& a);   // sa_bf16_kvg.hip
 SA_HIDDEN int launch_bwd_kv64_solo(bool cv, const KvLaunch& a);                       // sa_bf16_kv1.hip

@@ -16,15 +16,17 @@
 //                the accumulator registers. Head 0's logits are built (queries x keys) instead,
 //                so the selection's prefix over queries runs down each lane's registers; F then
 //                reaches the softmax layout through the wavefront's LDS rows.
+//   bwd_rowprep  row statistics, bounds for the tiles without weight, the exempt keys' gradients
 //   bwd_kv       key-parallel. A wavefront owns 32 keys of G heads and sweeps the query tiles
-//                last to first. Tiles are (queries x keys), so the selection prefix F and the
+//                last to first, from the last that holds weight for its workgroup's keys. Tiles are (queries x keys), so the selection prefix F and the
 //                suffix U = sum_h sum_{i>r} dz_h[i,j] run down registers. dK, dV (and the
 //                group's share of head 0's dK) stay in registers; K, V rows sit in LDS. U is
 //                checkpointed per query tile for bwd_dq.
 //   bwd_dq       query-parallel. A wavefront owns 32 queries and walks the key tiles up to its
 //                diagonal, recomputing P, dz and the selection gradient g from the key side's
 //                U checkpoints; dQ = dz K takes dz through a per-wavefront LDS tile.
-//   bwd_finish   gradient epilogue: scale, add head 0's shares, convert to the output dtype.
+//   bwd_finish   gradient epilogue: scale, add head 0's shares and the exempt keys' partial sums, convert
+//                to the output dtype.
 // The group holding head 0 folds g = -gate*U into head 0's own dz; every other group stores its
 // share of head 0's gradients in a slot of its own, and bwd_finish sums the slots in a fixed order
 // (no atomics: the backward is bitwise repeatable).
@@ -1943,49 +1945,323 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// Backward preparation: lse = rmax + log2(rden), ndbar = -rowsum(dO * O) (negated: the dO.v
-// products accumulate onto it), and, except at bf16 head dim 64 (whose kernels read the rows
-// transposed from LDS), the transposed copies Q^T, dO^T, K^T (R, D, ldt). The
-// statistics are laid out (R, ldt), each head's rows padded to ldt with lse = +inf (P = 0) and
-// ndbar = 0, so a 32-row tile of them is always in bounds; they take D/8 lanes per row (8 elements
-// each, so the loads of a row are contiguous across its lanes); transposes go by tiles.
+// Backward preparation, a wavefront per 32 query rows, a workgroup per QSTAT_ROWS rows of one head. Always:
+// lse = rmax + log2(rden) and ndbar = -rowsum(dO * O) (negated: the dO.v products accumulate onto it), laid
+// out (R, ldt), each head's rows padded to ldt with lse = +inf (P = 0) and ndbar = 0, so a 32-row tile of
+// them is always in bounds; D/8 lanes per row, 8 elements each, so a row's loads are contiguous.
+//
+// With reach.qstat, for the key side's search for the tiles without weight (kv_last_block): the largest
+// |q| and the least lse of the workgroup's rows, infinities where a row is not finite or a product with it
+// could overflow.
+//
+// With reach.xk, the gradients of the first xk keys, the exempt ones. They have no history (F = 0), so
+// every later query keeps weight on them: the key side would sweep every query tile for those few
+// columns, long after its other keys' weights are gone. Here they are one more set of products on the rows
+// at hand, which go to the wavefront's LDS tiles for it: P and dz of the 32 first keys (columns from xk on
+// masked), dV += P^T dO and dK += dz^T Q with P and dz as split operands (hi + lo, as these sums run over
+// every query), the rows taken transposed from LDS. The wavefronts' sums add up in LDS, the workgroups' in
+// bwd_finish_kernel, both in a fixed order.
+// Bound by HBM (dO, O and Q once). Measured at B=1 H=16 T=16384 bf16: 25 us without exempt keys apart (5.4
+// TB/s), 33 us with one of them, 39 with 16.
 
 template <class OP, int D>
-__global__ __launch_bounds__(NTHREADS) void bwd_rowstats_kernel(
-    const typename OP::elem* __restrict__ dout, Strides dos, int H, int T, const float* __restrict__ out,
-    const float* __restrict__ rmax, const float* __restrict__ rden,
-    float* __restrict__ lse, float* __restrict__ ndbar, int64_t ldt, int64_t rows) {
+__global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 && D <= 64 ? 4 : 1)) void bwd_rowprep_kernel(
+    const typename OP::elem* __restrict__ q, const typename OP::elem* __restrict__ k,
+    const typename OP::elem* __restrict__ v, const typename OP::elem* __restrict__ dout, Strides qs, Strides ks,
+    Strides vs, Strides dos, int H, int T, const float* __restrict__ out, const float* __restrict__ rmax,
+    const float* __restrict__ rden, float* __restrict__ lse, float* __restrict__ ndbar, int64_t ldt, float scale,
+    BwdReach reach) {
   using elem = typename OP::elem;
-  constexpr int LPR = D / 8;   // lanes per row
-  const int64_t g = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
-  const int64_t pr = g / LPR;   // padded row: head pr / ldt, row t
-  const int part = (int)(g % LPR);
-  const int64_t hr = pr / ldt;   // b * H + head
-  const int t = (int)(pr - hr * ldt);
-  const int64_t r = hr * T + t;
-  float acc = 0.f;
-  if (pr < rows && t < T) {
-    const elem* dr = dout + dos.at(hr / H, hr % H) + (int64_t)t * dos.row + part * 8;
-    const float* orow = out + r * D + part * 8;
-    const float4 o0 = *reinterpret_cast<const float4*>(orow);
-    const float4 o1 = *reinterpret_cast<const float4*>(orow + 4);
-    const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
-    elem dv[8];
-    if constexpr (sizeof(elem) == 2) {
-      *reinterpret_cast<uint4*>(dv) = *reinterpret_cast<const uint4*>(dr);
-    } else {
-      *reinterpret_cast<float4*>(dv) = *reinterpret_cast<const float4*>(dr);
-      *reinterpret_cast<float4*>(dv + 4) = *reinterpret_cast<const float4*>(dr + 4);
+  using frag = typename OP::frag;
+  constexpr int NS = D / OP::KS, DB = D / 32, AS = OP::acc_steps;
+  constexpr int LPR = D / 8, RPW = 64 / LPR, PASSES = TILE / RPW;
+  constexpr bool TR = sizeof(elem) == 2 && D == 64;   // rows in swzq, taken transposed by get_trq
+  constexpr int LD = TR ? D : D + OP::KPAD;
+  static_assert(QSTAT_ROWS == NWAVES * TILE, "a wavefront per row tile");
+  constexpr int SUMLD = 2 * D + 4;   // floats of one key's dK and dV (padded: keys on shifted banks)
+  union Shared {
+    elem rows[NWAVES][2][TILE * LD];   // a wavefront's dO rows and Q rows
+    float sum[NWAVES][8 * SUMLD];      // then its dK and dV sums of eight keys
+  };
+  __shared__ __attribute__((aligned(16))) Shared sh;
+  __shared__ __attribute__((aligned(16))) float sRow[NWAVES][2][TILE];   // a wavefront's rows' lse and -dbar
+  __shared__ float sStat[NWAVES][2];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  const int n = lane & 31, h = lane >> 5;
+  const int r = blockIdx.y, seg = blockIdx.x;
+  const int b = r / H, hh = r % H;
+  const int xk = reach.xk;
+  const int qbase = (seg * NWAVES + wave) * TILE;
+  const int part = lane % LPR;
+  const bool stats = reach.qstat != nullptr;
+
+  union Row {
+    elem e[8];
+    uint4 u[sizeof(elem) == 2 ? 1 : 2];
+  };
+  Row dr[PASSES], qr[PASSES];
+  float4 o4[PASSES][2];
+  float mv[PASSES], nv[PASSES];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {   // every load of the tile in flight (the last row again past the end)
+    const int row = qbase + p * RPW + lane / LPR;
+    const int64_t rr = min(row, T - 1);
+    const uint4* ds = reinterpret_cast<const uint4*>(dout + dos.at(b, hh) + rr * dos.row + 8 * part);
+    const uint4* qv = reinterpret_cast<const uint4*>(q + qs.at(b, hh) + rr * qs.row + 8 * part);
+    const float4* os = reinterpret_cast<const float4*>(out + ((int64_t)r * T + rr) * D + 8 * part);
+#pragma unroll
+    for (int c = 0; c < (int)(sizeof(elem) / 2); ++c) {
+      dr[p].u[c] = ds[c];
+      if (stats) qr[p].u[c] = qv[c];
+    }
+    o4[p][0] = os[0];
+    o4[p][1] = os[1];
+    mv[p] = rmax[(int64_t)r * T + rr];
+    nv[p] = rden[(int64_t)r * T + rr];
+  }
+  float qmax = 0.f, lmin = INFINITY;
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int rl = p * RPW + lane / LPR, row = qbase + rl;
+    const bool ok = row < T;
+    const float lv = ok ? mv[p] + __log2f(nv[p]) : INFINITY;
+    if (!ok) {   // (zeros)
+#pragma unroll
+      for (int c = 0; c < (int)(sizeof(elem) / 2); ++c) dr[p].u[c] = qr[p].u[c] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    const float ov[8] = {o4[p][0].x, o4[p][0].y, o4[p][0].z, o4[p][0].w, o4[p][1].x, o4[p][1].y, o4[p][1].z, o4[p][1].w};
+    float acc = 0.f, dd = 0.f, qq = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float d = OP::to_float(dr[p].e[e]);
+      acc += d * ov[e];
+      if (stats) {
+        const float x = OP::to_float(qr[p].e[e]);
+        dd = fmaf(d, d, dd);
+        qq = fmaf(x, x, qq);
+      }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc += OP::to_float(dv[e]) * ov[e];
+    for (int o = LPR / 2; o > 0; o >>= 1) {
+      acc += __shfl_xor(acc, o);
+      if (stats) {
+        dd += __shfl_xor(dd, o);
+        qq += __shfl_xor(qq, o);
+      }
+    }
+    const float nd = ok ? -acc : 0.f;
+    if (part == 0 && row < ldt) {
+      lse[(int64_t)r * ldt + row] = lv;
+      ndbar[(int64_t)r * ldt + row] = nd;
+    }
+    if (stats && ok) {
+      qmax = fmaxf(qmax, qq < REACH_NORM2 && dd < REACH_NORM2 && fabsf(nd) < REACH_NORM2 ? qq : INFINITY);
+      lmin = fminf(lmin, fabsf(lv) < 3.0e38f ? lv : -INFINITY);
+    }
+    if (xk > 0) {
+      if (part == 0) {
+        sRow[wave][0][rl] = lv;
+        sRow[wave][1][rl] = nd;
+      }
+      elem* dst = &sh.rows[wave][0][TR ? swzq(rl, part) : rl * LD + 8 * part];
+#pragma unroll
+      for (int c = 0; c < (int)(sizeof(elem) / 2); ++c) {
+        reinterpret_cast<uint4*>(dst)[c] = dr[p].u[c];
+        reinterpret_cast<uint4*>(dst + TILE * LD)[c] = qr[p].u[c];
+      }
+    }
+  }
+  if (!stats) return;
+
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    qmax = fmaxf(qmax, __shfl_xor(qmax, o));
+    lmin = fminf(lmin, __shfl_xor(lmin, o));
+  }
+  if (lane == 0) {
+    sStat[wave][0] = qmax;
+    sStat[wave][1] = lmin;
+  }
+  f32x16 dkx[DB], dvx[DB];
+  if (xk > 0) {
+    frag kx[NS], vx[NS];   // the first keys and values (B operands: lane = key)
+    const elem* kh = k + ks.at(b, hh);
+    const elem* vh = v + vs.at(b, hh);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      kx[s] = ld_std_bounded<OP>(kh, ks.row, n, T, h, s);
+      vx[s] = ld_std_bounded<OP>(vh, vs.row, n, T, h, s);
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      dkx[db] = zero16();
+      dvx[db] = zero16();
+    }
+    lds_wave_sync();
+    auto rfrag = [&](int x, int s) -> frag {   // A operand: lane = query row
+      const elem* y = sh.rows[wave][x];
+      if constexpr (TR) return *reinterpret_cast<const frag*>(y + swzq(n, 2 * s + h));
+      else return OP::ld_std(y, LD, n, h, s);
+    };
+    // acc[db] (D x keys) += Y^T X: Y the wavefront's rows, X a (queries x keys) tile
+    auto acc_t = [&](f32x16 (&acc)[DB], int which, const f32x16& x) {
+      const elem* y = sh.rows[wave][which];
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int s = 0; s < AS; ++s) {
+          frag yt;
+          if constexpr (TR) {
+            yt = get_trq<true>(y, lane, db, s);
+          } else if constexpr (sizeof(elem) == 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const elem raw = y[(16 * s + 8 * (e >> 2) + 4 * h + (e & 3)) * LD + db * 32 + n];
+              yt[e] = *reinterpret_cast<const bf16_t*>(&raw);
+            }
+          } else {
+            yt = y[crow(s, h) * LD + db * 32 + n];
+          }
+          acc[db] = OP::mma(yt, OP::from_acc(x, s), acc[db]);
+          if constexpr (OP::SPLIT) acc[db] = OP::mma(yt, OP::from_acc_lo(x, s), acc[db]);
+        }
+    };
+    f32x16 p = zero16(), dz = rows16(sRow[wave][1], h);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      p = OP::mma(rfrag(1, s), kx[s], p);
+      dz = OP::mma(rfrag(0, s), vx[s], dz);
+    }
+    const f32x16 ls = rows16(sRow[wave][0], h);
+    const float sl2 = scale * LOG2E;
+    const int thr = n < xk ? n - qbase - 4 * h : 32;   // key n <= query qbase + crow(i, h)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      p[i] = crow(i, 0) >= thr ? fast_exp2(fmaf(p[i], sl2, -ls[i])) : 0.f;
+      dz[i] = p[i] * dz[i];
+    }
+    acc_t(dvx, 0, p);
+    acc_t(dkx, 1, dz);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < NWAVES; ++w) {
+      qmax = fmaxf(qmax, sStat[w][0]);
+      lmin = fminf(lmin, sStat[w][1]);
+    }
+    reach.qstat[(int64_t)r * reach.nseg + seg] = make_float2(sqrtf(qmax), lmin);
+  }
+  if (xk == 0) return;
+  float4* dst = reinterpret_cast<float4*>(reach.xpart + ((int64_t)r * reach.nseg + seg) * xk * 2 * D);
+  for (int j0 = 0; j0 < xk; j0 += 8) {   // (every wavefront is past its reads of the rows)
+    if (n >= j0 && n < min(j0 + 8, xk)) {
+      float* mine = &sh.sum[wave][(n - j0) * SUMLD];
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          const int d = db * 32 + 8 * a + 4 * h;
+          *reinterpret_cast<float4*>(mine + d) =
+              make_float4(dkx[db][4 * a], dkx[db][4 * a + 1], dkx[db][4 * a + 2], dkx[db][4 * a + 3]);
+          *reinterpret_cast<float4*>(mine + D + d) =
+              make_float4(dvx[db][4 * a], dvx[db][4 * a + 1], dvx[db][4 * a + 2], dvx[db][4 * a + 3]);
+        }
+    }
+    __syncthreads();
+    const int quads = min(8, xk - j0) * (2 * D / 4);
+    for (int i = tid; i < quads; i += NTHREADS) {
+      const int at = (i / (2 * D / 4)) * SUMLD + 4 * (i % (2 * D / 4));
+      float4 x = *reinterpret_cast<const float4*>(&sh.sum[0][at]);
+#pragma unroll
+      for (int w = 1; w < NWAVES; ++w) {
+        const float4 y = *reinterpret_cast<const float4*>(&sh.sum[w][at]);
+        x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+      }
+      dst[j0 * (2 * D / 4) + i] = x;
+    }
+    __syncthreads();
+  }
+}
+
+// (Measured, N(0,1) inputs, B=1 H=16 T=16384 bf16: the key side 1560 -> 195 us, the query side 1510 -> 215 us.)
+// The last query block on which some key of a wavefront's 32 (from key0) keeps a weight that is not an
+// exact zero, of the blocks up to NB - 1 (the key tile's own block at least): a lane group of 8 probes one
+// block (4 keys per lane), eight blocks at a time; the history never falls, so the blocks past the last
+// one are all without weight. thr: see find_reach, with the head's least lse for the row maxima. Keys
+// below xk (their gradients are taken elsewhere) and past the end do not count. The first probe, the last
+// block, is all it costs where nothing can be left out.
+__device__ __forceinline__ int kv_last_block(const float* carry_b, int T, int NB, int key0, int xk, float thr,
+                                             int lane) {
+  const int part = lane >> 3, j0 = key0 + 4 * (lane & 7);
+  auto gone = [&](int qb) {   // (qb < NB; lanes of a probe past the interval read a block inside it)
+    const float* p = carry_b + (int64_t)qb * T;
+    bool ok = thr < INFINITY;   // every comparison that meets a NaN keeps the block
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = j0 + e;
+      const float f = p[min(j, T - 1)];
+      ok = ok && (j >= T || j < xk || f * REACH_F > thr);
+    }
+    return ok;
+  };
+  if (__ballot(gone(NB - 1)) != ~0ull) return NB - 1;
+  int lo = key0 / TILE, hi = NB - 1;   // lo: kept; hi: without weight
+  while (hi - lo > 1) {
+    const int stride = max(1, (hi - lo) / 9);
+    const uint64_t m = __ballot(gone(min(lo + (part + 1) * stride, hi)));
+    int first = 8;
+#pragma unroll
+    for (int i = 7; i >= 0; --i) first = ((m >> (8 * i)) & 0xFF) == 0xFF ? i : first;
+    const int nhi = first < 8 ? min(lo + (first + 1) * stride, hi) : hi;
+    lo = min(lo + first * stride, nhi - 1);
+    hi = nhi;
+  }
+  return lo;
+}
+
+// The head's bounds from its row segments: the largest |q| and the least lse.
+__device__ __forceinline__ float2 head_qstat(const BwdReach& reach, int64_t r, int lane) {
+  float qm = 0.f, lm = INFINITY;
+  for (int i = lane; i < reach.nseg; i += 64) {
+    const float2 x = reach.qstat[r * reach.nseg + i];
+    qm = fmaxf(qm, x.x);
+    lm = fminf(lm, x.y);
   }
 #pragma unroll
-  for (int o = LPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-  if (pr < rows && part == 0) {
-    ndbar[pr] = t < T ? -acc : 0.f;
-    lse[pr] = t < T ? rmax[r] + __log2f(rden[r]) : INFINITY;
+  for (int o = 1; o < 64; o <<= 1) {
+    qm = fmaxf(qm, __shfl_xor(qm, o));
+    lm = fminf(lm, __shfl_xor(lm, o));
   }
+  return make_float2(qm, lm);
+}
+
+// kv_last_block's threshold of one head for a wavefront's keys: kf, vf the lane's parts of its key and value.
+template <class OP, int NS>
+__device__ __forceinline__ float kv_threshold(const typename OP::frag (&kf)[NS], const typename OP::frag (&vf)[NS],
+                                              const float2& qstat, float scale) {
+  float kk = frag_sumsq<OP, NS>(kf), vv = frag_sumsq<OP, NS>(vf);
+  kk += xor32(kk);
+  vv += xor32(vv);
+  const float kn = sqrtf(half_max(kk < REACH_NORM2 && vv < REACH_NORM2 ? kk : INFINITY));
+  const float t = fmaf(qstat.x * scale * REACH_Q, kn, REACH_ZERO - qstat.y);
+  return t < INFINITY ? t : INFINITY;   // (a NaN, from 0 * inf, keeps everything)
+}
+
+// The query blocks (NB - 1 at most) that a key-side workgroup's sweep starts from, once every wavefront's
+// last block is in last[]; the query side finds it in hi, and reads the selection-suffix checkpoints of
+// whole groups of eight query blocks: the rows of the sweep's group past its start hold zeros.
+__device__ __forceinline__ int kv_sweep_start(const int* last, int NB, int qb_lo, int wave, int lane, int key0, int T,
+                                              float* uplane, int* hi) {
+  int top = qb_lo + NWAVES - 1;
+#pragma unroll
+  for (int w = 0; w < NWAVES; ++w) top = max(top, last[w]);
+  top = min(__builtin_amdgcn_readfirstlane(top), NB - 1);
+  if (wave == 0 && lane == 0) *hi = top;
+  const int j = key0 + lane;
+  for (int qb = top + 1; qb <= min(top | 7, NB - 1); ++qb)
+    if (lane < TILE && j < T) uplane[utri_row(qb) + j] = 0.f;
+  return top;
 }
 
 // in (R = nseq * H views of T rows, Strides is) -> outT (R, D, ldt), zero past T; a workgroup moves
@@ -2111,9 +2387,9 @@ __device__ __forceinline__ void store_grad4(const GradView& v, int64_t b, int hh
 //   selection: j <  r  (and exempt <= j < T) <=>  crow(i, 0) >  thr_s = j - qbase - 4h  (32 if not)
 struct TileMasks {
   int thr_p, thr_s;
-  __device__ __forceinline__ TileMasks(int j, int qbase, int T, int exempt, int h) {
+  __device__ __forceinline__ TileMasks(int j, int qbase, int T, int exempt, int h, int xk = 0) {
     const int d = j - qbase - 4 * h;
-    thr_p = j < T ? d : 32;
+    thr_p = (j < T && j >= xk) ? d : 32;   // (keys below xk: no P, no dz)
     thr_s = (j < T && j >= exempt) ? d : 32;
   }
 };
@@ -2249,7 +2525,7 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
     const typename OP::elem* __restrict__ dout, const typename OP::elem* __restrict__ dot, Strides qs,
     Strides ks, Strides vs, Strides dos, const float* __restrict__ lse, const float* __restrict__ dbar,
     const float* __restrict__ carry, float* __restrict__ ucheck, float* __restrict__ dk0h, float* __restrict__ dk0x,
-    GradView dkv, GradView dvv, int nseq, int H, int T, int64_t ldt, int exempt, float scale) {
+    GradView dkv, GradView dvv, int nseq, int H, int T, int64_t ldt, int exempt, float scale, BwdReach reach) {
   using elem = typename OP::elem;
   using frag = typename OP::frag;
   constexpr int NS = D / OP::KS;
@@ -2275,6 +2551,7 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
   constexpr bool KVLDS = sizeof(elem) == 2 && D == 64 && OTHER_LDS + NWAVES * NKV * TILE * D * 2 <= 80 * 1024;
   __shared__ __attribute__((aligned(16))) elem sKV[KVLDS ? NWAVES : 1][KVLDS ? NKV : 1][KVLDS ? TILE * D : 8];
 
+  __shared__ int sLast[NWAVES];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
   const int groups = H / G;
@@ -2376,9 +2653,29 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
   float ucarry = 0.f;
   const float sl2 = scale * LOG2E;
   const float neg_inv_scale = -1.f / scale;
-  // query tiles the workgroup visits, last to first: NB-1 down to the first that reaches its keys
+  // query tiles the workgroup visits, last to first: qb_hi down to the first that reaches its keys
   const int qb_lo = bxy.x * NWAVES;
-  const int ntiles = NB - qb_lo;
+  int qb_hi = NB - 1;   // the first tile of the sweep: later ones hold no weight for the workgroup's keys
+  if (reach.qstat) {
+    if constexpr (KVLDS) lds_wave_sync();   // (the wavefront's own rows)
+    float thr = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      frag kg[NS], vg[NS];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        kg[s] = k_frag(g, s);
+        vg[s] = v_frag(g, s);
+      }
+      thr = fmaxf(thr, kv_threshold<OP, NS>(kg, vg, head_qstat(reach, seq_row + hd0 + g, lane), scale));
+    }
+    const int last = key0 < T ? kv_last_block(carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane) : 0;
+    if (lane == 0) sLast[wave] = last;
+    __syncthreads();
+    qb_hi = kv_sweep_start(sLast, NB, qb_lo, wave, lane, key0, T, uplane,
+                           reach.hi + ((int64_t)gi * nseq + b) * reach.nkg + bxy.x);
+  }
+  const int ntiles = qb_hi - qb_lo + 1;
 
   // Staging of one query tile: Q, Q^T, dO, dO^T of the group (+ head 0's Q, Q^T), lse, dbar.
   RowTile<elem, D> nQ[NH], ndO[G];
@@ -2466,7 +2763,7 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
     // is exempt, so the body is straight-line code without the masks and split products
     auto tile_step = [&](int t, auto interior_tag) {
       constexpr bool INTERIOR = decltype(interior_tag)::value;
-      const int qb = NB - 1 - t;
+      const int qb = qb_hi - t;
       const int qbase = qb * TILE;
       load_tile(qb);
       const float hist = carry_col[(int64_t)qb * T];
@@ -2480,7 +2777,7 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
         // stay in their own lanes, which are never written)
         const bool edge = !INTERIOR && ((qbase <= key0 + TILE - 1) || key0 < exempt);
         const bool split = !INTERIOR && split_keys;
-        const TileMasks mk(j, qbase, T, exempt, h);
+        const TileMasks mk(j, qbase, T, exempt, h, reach.xk);
         // (a lambda: inlined late, its loop-invariant parts are not hoisted out of the tile loop,
         // which would hold them in registers across it)
         auto body = [&]() {
@@ -2543,7 +2840,7 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
   if (has_h0) sweep(std::true_type{});
   else sweep(std::false_type{});
 
-  if (j >= T) return;
+  if (j >= T || j < reach.xk) return;   // (the first xk keys' gradients: bwd_finish_kernel)
   // dV of every head and dK of heads other than 0 go to the caller's views; head 0's dK to its
   // fp32 sums, where the other groups' shares join it
 #pragma unroll
@@ -2600,7 +2897,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
     const uint16_t* __restrict__ dout, Strides qs, Strides ks, Strides vs, Strides dos,
     const float* __restrict__ lse, const float* __restrict__ dbar, const float* __restrict__ carry,
     float* __restrict__ ucheck, float* __restrict__ dk0h, float* __restrict__ dk0x, GradView dkv, GradView dvv,
-    int nseq, int H, int T, int64_t ldt, int exempt, float scale) {
+    int nseq, int H, int T, int64_t ldt, int exempt, float scale, BwdReach reach) {
   using OP = OpBF16;
   using elem = uint16_t;
   using frag = OP::frag;
@@ -2610,7 +2907,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   // every access names its buffer at compile time: the compiler then knows the direct loads into
   // one buffer do not write what the tile reads from the other, and waits for them only at the end
   // of the tile (a single array indexed by tile parity made it wait before the tile's first read).
-  // LDS lifetimes (tile t = query tile NB - 1 - t):
+  // LDS lifetimes (tile t = query tile qb_hi - t):
   //   sB0, sB1  tile t's Q, dO and head 0's Q rows, its rows' lse and -dbar, each wavefront's carry
   //             row, buffer t mod 2. Filled: by direct loads of all four wavefronts (rows a quarter
   //             each; statistics by wavefronts 0 and 1; each its own carry row), for tile 0 before
@@ -2626,6 +2923,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   //             barrier, only read after it.
   __shared__ KvTileBuf64 sB0, sB1;
   __shared__ __attribute__((aligned(16))) elem sV[NWAVES][TW];
+  __shared__ int sLast[NWAVES];   // kv_last_block of each wavefront: written and read before the first tile
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
@@ -2666,6 +2964,20 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
     }
   }
 
+  // Exempt keys whose gradients are taken apart (j < xk) need no masks in this workgroup's interior tiles:
+  // head 0's key is zeroed in their lanes, so their logits select nothing, and their history is taken as
+  // beyond any logit, so their P and dz are zeros. (The masks on every tile made the first workgroup of a
+  // head, whose sweep is the longest, half again as slow as the others: with 16 exempt keys, B=2 H=12 T=5003,
+  // nothing left out, the kernel runs 317 us instead of 342.)
+  const bool apart = j < reach.xk;
+  if (apart) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      k0f[s] = OP::zero();
+      if (has_h0) kf[s] = OP::zero();
+    }
+  }
+
   f32x16 dkt[DB], dvt[DB], dk0t[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) {
@@ -2676,9 +2988,27 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   float ucarry = 0.f;
   const float sl2 = scale * LOG2E;
   const float neg_inv_scale = -1.f / scale;
-  // query tiles the workgroup visits, last to first: NB-1 down to the first that reaches its keys
+  // fragment s of row n of a swzq tile (A operand: lane = query row; or B: lane = key)
+  auto rfrag = [&](const elem* tile, int s) -> frag {
+    return *reinterpret_cast<const frag*>(tile + swzq(n, 2 * s + h));
+  };
+  // query tiles the workgroup visits, last to first: qb_hi (later ones hold no weight for its keys) down
+  // to the first that reaches its keys
   const int qb_lo = bxy.x * NWAVES;
-  const int ntiles = NB - qb_lo;
+  int qb_hi = NB - 1;
+  if (reach.qstat) {
+    lds_wave_sync();   // the wavefront's V rows
+    frag vg[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) vg[s] = rfrag(sV[wave], s);
+    const float thr = kv_threshold<OP, NS>(kf, vg, head_qstat(reach, seq_row + hh, lane), scale);
+    const int last = key0 < T ? kv_last_block(carry_b, T, NB, key0, reach.xk, thr, lane) : 0;
+    if (lane == 0) sLast[wave] = last;
+    __syncthreads();
+    qb_hi = kv_sweep_start(sLast, NB, qb_lo, wave, lane, key0, T, uplane,
+                           reach.hi + ((int64_t)hh * nseq + b) * reach.nkg + bxy.x);
+  }
+  const int ntiles = qb_hi - qb_lo + 1;
 
   // operand sources (buffer resources over one head's rows) and this lane's parts of the direct
   // loads
@@ -2696,7 +3026,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   // every tile), the row statistics (wavefronts 0, 1), and each wavefront's carry row of its keys
   // (keys past the end read zero). Tiles load in order, last to first, so the carry row steps back
   // one row per call.
-  const float* carry_row = carry_b + (int64_t)(NB - 1) * T;
+  const float* carry_row = carry_b + (int64_t)qb_hi * T;
   auto load_tile = [&](int qb, KvTileBuf64& B) {
     const int qbase = qb * TILE;
     if (wave == 0)
@@ -2710,8 +3040,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
     g2l_rowsq(B.r[1], rs_do, rl_do, do_ld, qbase, wave);
     if (!has_h0) g2l_rowsq(B.r[2], rs_q0, rl_q, q_ld, qbase, wave);
   };
-  // the first tile (NB - 1)
-  load_tile(NB - 1, sB0);
+  // the first tile
+  load_tile(qb_hi, sB0);
   wait_loads();
   __syncthreads();
 
@@ -2734,10 +3064,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
         for (int s = 0; s < AS; ++s) acc[db] = OP::mma(get_trq<true>(y, lane, db, s), xf[s], acc[db]);
     }
   };
-  // fragment s of row n of a swzq tile (A operand: lane = query row; or B: lane = key)
-  auto rfrag = [&](const elem* tile, int s) -> frag {
-    return *reinterpret_cast<const frag*>(tile + swzq(n, 2 * s + h));
-  };
 
   // Keys below `exempt` are never selected, so they gather attention from every later query and
   // their dV / dK sums run over all of them: their products take the split operands.
@@ -2747,24 +3073,26 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   auto sweep = [&](auto h0_tag) {
     constexpr bool H0 = decltype(h0_tag)::value;
     // the checkpoint row of tile t's query block (the rows lie end to end, tiles run last to first)
-    float* urow = uplane + utri_row(NB - 1);
+    float* urow = uplane + utri_row(qb_hi);
     // tile t (buffer t mod 2, named by ODD)
-    auto tile_step = [&](int t, auto interior_tag, auto odd_tag) {
-      constexpr bool INTERIOR = decltype(interior_tag)::value;
+    // kind 0: some pairs masked; 1: none; 2: none, with the split products of the tile that holds exempt keys
+    auto tile_step = [&](int t, auto kind_tag, auto odd_tag) {
+      constexpr int KIND = decltype(kind_tag)::value;
+      constexpr bool INTERIOR = KIND != 0;
       constexpr bool ODD = decltype(odd_tag)::value;
       KvTileBuf64& B = ODD ? sB1 : sB0;
-      const int qb = NB - 1 - t;
+      const int qb = qb_hi - t;
       const int qbase = qb * TILE;
       const bool more = t + 1 < ntiles;
       if (more) load_tile(qb - 1, ODD ? sB0 : sB1);   // into the other buffer, free since the last barrier
       if (INTERIOR || qbase + TILE - 1 >= key0) {   // else every query of the tile precedes every key
         if (h == 0 && j < T) urow[j] = ucarry;   // j < (qb + 1) * TILE here
         const bool edge = !INTERIOR && ((qbase <= key0 + TILE - 1) || key0 < exempt);
-        const bool split = !INTERIOR && split_keys;
-        const TileMasks mk(j, qbase, T, exempt, h);
+        const bool split = KIND != 1 && split_keys;
+        const TileMasks mk(j, qbase, T, exempt, h, reach.xk);
         auto body = [&]() {
           // (keys past the end read a zero carry through the load's range check)
-          const float hist = B.hist[wave][lane];
+          const float hist = KIND == 2 && apart ? 1e30f : B.hist[wave][lane];
           const elem* q0s = H0 ? B.r[0] : B.r[2];
           // the four fragments of head 0's Q rows are all requested before the chain of logit
           // products starts, so the chain waits for one LDS latency rather than one per product
@@ -2812,26 +3140,28 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
       wait_loads();
       __syncthreads();   // the next tile's operands are in; every wavefront is done with this one
     };
-    // The last NWAVES tiles hold the wavefronts' diagonals; a workgroup with an exempt key runs
-    // every tile with the masks.
-    const int n_int = (qb_lo * TILE < exempt) ? 0 : max(ntiles - NWAVES, 0);
+    // The last NWAVES tiles hold the wavefronts' diagonals; a workgroup with an exempt key that is not
+    // taken apart runs every tile with the masks.
+    const bool first = qb_lo * TILE < exempt;
+    const int n_int = (first && reach.xk == 0) ? 0 : max(ntiles - NWAVES, 0);
     // tiles [t0, t1) in pairs, even tiles from buffer 0 and odd ones from buffer 1
-    auto run = [&](int t0, int t1, auto interior_tag) {
+    auto run = [&](int t0, int t1, auto kind_tag) {
       int t = t0;
-      if (t < t1 && (t & 1)) tile_step(t++, interior_tag, std::true_type{});
+      if (t < t1 && (t & 1)) tile_step(t++, kind_tag, std::true_type{});
       for (; t + 1 < t1; t += 2) {
-        tile_step(t, interior_tag, std::false_type{});
-        tile_step(t + 1, interior_tag, std::true_type{});
+        tile_step(t, kind_tag, std::false_type{});
+        tile_step(t + 1, kind_tag, std::true_type{});
       }
-      if (t < t1) tile_step(t, interior_tag, std::false_type{});
+      if (t < t1) tile_step(t, kind_tag, std::false_type{});
     };
-    run(0, n_int, std::true_type{});
-    run(n_int, ntiles, std::false_type{});
+    if (first) run(0, n_int, std::integral_constant<int, 2>{});
+    else run(0, n_int, std::integral_constant<int, 1>{});
+    run(n_int, ntiles, std::integral_constant<int, 0>{});
   };
   if (SOLO || has_h0) sweep(std::true_type{});
   else if constexpr (!SOLO) sweep(std::false_type{});
 
-  if (j >= T) return;
+  if (j >= T || j < reach.xk) return;   // (the first xk keys' gradients: bwd_finish_kernel)
   // dV and the dK of heads other than 0 go to the caller's views; head 0's dK to its fp32 sums,
   // where the other heads' shares join it (to its view too when it is the sequence's only head)
 #pragma unroll
@@ -2858,6 +3188,56 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
+// The key tiles that a query-side workgroup has to visit, ascending, from the key side's sweep starts
+// (hi, one per four key tiles): those whose sweep reached the workgroup's first query block qb0 -- past
+// it their weights and selection suffixes are zeros -- and the tiles of exempt keys, [0, i_lo). As runs of
+// groups of four tiles counted from the workgroup's last group (write_reach_runs counts down).
+struct QueryWalk {
+  const TileRun* runs;
+  int groups, run_to, i;
+  bool far;   // the first group is visited for its exempt keys alone
+  __device__ __forceinline__ void none() {   // every tile
+    run_to = INT_MAX;
+    far = false;
+    i = 0;
+  }
+  template <int NW>
+  __device__ __forceinline__ void find(const int* hi, int qb0, int wg_end, int i_lo, uint64_t* words, TileRun* r,
+                                       int lane, int wave) {
+    groups = (wg_end + 3) / 4;
+    far = __builtin_amdgcn_readfirstlane(hi[0]) < qb0;
+    const int all = (groups + 63) / 64, nwords = min(all, REACH_MASK_WORDS), first = 64 * (all - nwords);
+    for (int w = wave; w < nwords; w += NW) {
+      const int m = first + 64 * w + lane, g = groups - 1 - m;
+      const uint64_t bits = __ballot(g >= 0 && hi[max(g, 0)] >= qb0);
+      if (lane == 0) words[w] = bits;
+    }
+    __syncthreads();
+    if (wave == 0) write_reach_runs(r, words, nwords, first, lane);
+    __syncthreads();
+    runs = r;
+    i = 0;
+    if (far) {
+      run_to = i_lo - 1;
+    } else {
+      int from;
+      next_run(from);   // (starts at tile 0)
+    }
+  }
+  __device__ __forceinline__ void next_run(int& from) {
+    const TileRun r = runs[i++];
+    const int hi = __builtin_amdgcn_readfirstlane(r.hi), lo = __builtin_amdgcn_readfirstlane(r.lo);
+    from = 4 * (groups - 1 - hi);   // (past the workgroup's last tile at the end)
+    run_to = hi < 0 ? INT_MAX : 4 * (groups - 1 - lo) + 3;
+  }
+  __device__ __forceinline__ int after(int kt) {
+    int n = kt + 1;
+    if (__builtin_expect(n > run_to, 0)) next_run(n);
+    return n;
+  }
+};
+
+// ---------------------------------------------------------------------------------------------
 // Backward, query side. grid (ceil(T/128), nseq * H/G); wavefront w owns queries
 // [x*128 + 32w, +32) of heads [gi*G, gi*G+G) (late query blocks launch first) and walks the key
 // tiles up to its diagonal, with Q, dO and the dQ sums in registers. It recomputes P and dz as the
@@ -2872,7 +3252,7 @@ __global__ __launch_bounds__(NTHREADS, (dq_min_blocks<OP, D>())) void bwd_dq_ker
     const typename OP::elem* __restrict__ dout, Strides qs, Strides ks, Strides vs, Strides dos,
     const float* __restrict__ lse, const float* __restrict__ dbar, const float* __restrict__ carry,
     const float* __restrict__ ucheck, float* __restrict__ dq0h, float* __restrict__ dq0x, GradView dqv, int nseq,
-    int H, int T, int64_t ldt, int exempt, float scale) {
+    int H, int T, int64_t ldt, int exempt, float scale, BwdReach reach) {
   using elem = typename OP::elem;
   using frag = typename OP::frag;
   constexpr int NS = D / OP::KS;
@@ -2887,6 +3267,8 @@ __global__ __launch_bounds__(NTHREADS, (dq_min_blocks<OP, D>())) void bwd_dq_ker
   __shared__ __attribute__((aligned(16))) elem sKt[NH][D * LDKT];
   __shared__ __attribute__((aligned(16))) elem sV[G][TILE * LDK];
   __shared__ __attribute__((aligned(16))) elem sZ[NWAVES][TILE * LDZ];
+  __shared__ uint64_t sMask[REACH_MASK_WORDS];   // the tiles to visit (QueryWalk)
+  __shared__ TileRun sRuns[REACH_RUNS];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
@@ -3064,6 +3446,16 @@ __global__ __launch_bounds__(NTHREADS, (dq_min_blocks<OP, D>())) void bwd_dq_ker
     uv = (jj < T) ? urow[jj] : 0.f;
   };
 
+  // tiles holding exempt keys [0, i_lo), then the interior ones (below every wavefront's diagonal,
+  // which also keeps them clear of the sequence end), then the diagonals from i_hi on
+  const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
+  const int i_hi = max(i_lo, min(qsb * NWAVES, wg_end));
+  QueryWalk walk;
+  walk.none();
+  if (reach.qstat)
+    walk.template find<NWAVES>(reach.hi + ((int64_t)gi * nseq + b) * reach.nkg, qsb * NWAVES, wg_end, i_lo, sMask, sRuns,
+                               lane, wave);
+
   // The tile loop in two instances, for the group holding head 0 and for the others (as on the
   // key side).
   auto sweep = [&](auto h0_tag) {
@@ -3077,6 +3469,7 @@ __global__ __launch_bounds__(NTHREADS, (dq_min_blocks<OP, D>())) void bwd_dq_ker
       float hist, uin;
       load_tile(ktile);
       key_vals(ktile, hist, uin);
+      if (!INTERIOR && walk.far && ktile < i_lo) uin = 0.f;   // (past the sweep's start: no row written)
       if (ktile > 0) __syncthreads();   // every wavefront is done with the previous tile
       store_tile();
       __syncthreads();
@@ -3141,13 +3534,10 @@ __global__ __launch_bounds__(NTHREADS, (dq_min_blocks<OP, D>())) void bwd_dq_ker
         }
       }
     };
-    // tiles holding exempt keys, then the interior ones (below every wavefront's diagonal, which
-    // also keeps them clear of the sequence end), then the diagonals
-    const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
-    const int i_hi = max(i_lo, min(qsb * NWAVES, wg_end));
-    for (int ktile = 0; ktile < i_lo; ++ktile) tile_step(ktile, std::false_type{});
-    for (int ktile = i_lo; ktile < i_hi; ++ktile) tile_step(ktile, std::true_type{});
-    for (int ktile = i_hi; ktile < wg_end; ++ktile) tile_step(ktile, std::false_type{});
+    int ktile = 0;
+    for (; ktile < i_lo; ktile = walk.after(ktile)) tile_step(ktile, std::false_type{});
+    for (; ktile < i_hi; ktile = walk.after(ktile)) tile_step(ktile, std::true_type{});
+    for (; ktile < wg_end; ktile = walk.after(ktile)) tile_step(ktile, std::false_type{});
   };
   if (has_h0) sweep(std::true_type{});
   else sweep(std::false_type{});
@@ -3212,17 +3602,17 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
     const uint16_t* __restrict__ dout, Strides qs, Strides ks, Strides vs, Strides dos,
     const float* __restrict__ lse, const float* __restrict__ dbar, const float* __restrict__ carry,
     const float* __restrict__ ucheck, float* __restrict__ dq0h, float* __restrict__ dq0x, GradView dqv, int nseq,
-    int H, int T, int64_t ldt, int exempt, float scale, int order_slots) {
+    int H, int T, int64_t ldt, int exempt, float scale, int order_slots, BwdReach reach) {
   using OP = OpBF16;
   using elem = uint16_t;
   using frag = OP::frag;
   constexpr int D = 64, NS = 4, DB = 2, AS = 2;
-  // LDS lifetimes (key tile t):
+  // LDS lifetimes (t: the t-th key tile visited; key tile t where none is left out):
   //   sB0, sB1  tile t's K, head 0's K and V rows, each wavefront's carry and U-checkpoint values,
   //             buffer t mod 2. Filled: by direct loads (K rows by wavefronts 0-3, V rows by 4-7, a
   //             quarter each; every wavefront its own carry and checkpoint values), tile 0 before the
   //             first barrier, tile t in tile step t - 1. Drained: tile step t only (a wavefront
-  //             whose diagonal lies before tile t reads nothing but still loads and synchronises).
+  //             whose diagonal lies before the tile reads nothing but still loads and synchronises).
   //             Separated: as in bwd_kv64_kernel, each tile step ends with wait_loads() and
   //             __syncthreads(), between the last reads of a buffer and its next fill, and between a
   //             fill and its reads. The last tile step loads nothing.
@@ -3235,6 +3625,8 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
   __shared__ DqTileBuf64 sB0, sB1;
   __shared__ __attribute__((aligned(16))) elem sZ[DQ64_WAVES][TILE * TILE];   // per wavefront: dz, g transposed
   __shared__ __attribute__((aligned(16))) float sRow[DQ64_WAVES][2][TILE];   // per wavefront: its rows' lse, -dbar
+  __shared__ uint64_t sMask[REACH_MASK_WORDS];   // the tiles to visit (QueryWalk): written before the first tile
+  __shared__ TileRun sRuns[REACH_RUNS];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
@@ -3350,27 +3742,39 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
     lds_wave_order();
   };
 
-  // the first key tile
+  // the first key tile (position 0 is always exempt, so tile 0 is always visited)
   load_tile(0, sB0);
+  // tiles holding exempt keys [0, i_lo), then the interior ones (below every wavefront's diagonal,
+  // which also keeps them clear of the sequence end), then the diagonals from i_hi on
+  const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
+  const int i_hi = max(i_lo, min(qsb * DQ64_WAVES, wg_end));
+  QueryWalk walk;
+  walk.none();
+  if (reach.qstat)
+    walk.template find<DQ64_WAVES>(reach.hi + ((int64_t)hh * nseq + b) * reach.nkg, qsb * DQ64_WAVES, wg_end, i_lo, sMask,
+                                   sRuns, lane, wave);
+  int ktile = 0, next = walk.after(0);   // this tile and the one after it
   wait_loads();
   __syncthreads();
 
   // the tile loop in two instances, for head 0's workgroups and the others (see bwd_kv_kernel)
   auto sweep = [&](auto h0_tag) {
     constexpr bool H0 = decltype(h0_tag)::value;
-    // key tile ktile (buffer ktile mod 2, named by ODD); INTERIOR: no pair of the tile is masked or
-    // exempt for any wavefront
-    auto tile_step = [&](int ktile, auto interior_tag, auto odd_tag) {
+    // key tile ktile, the t-th visited (buffer t mod 2, named by ODD); INTERIOR: no pair of the tile is
+    // masked or exempt for any wavefront
+    auto tile_step = [&](auto interior_tag, auto odd_tag) {
       constexpr bool INTERIOR = decltype(interior_tag)::value;
       constexpr bool ODD = decltype(odd_tag)::value;
       DqTileBuf64& B = ODD ? sB1 : sB0;
       const int kbase = ktile * TILE;
-      if (ktile + 1 < wg_end) load_tile(ktile + 1, ODD ? sB0 : sB1);   // free since the last barrier
+      if (next < wg_end) load_tile(next, ODD ? sB0 : sB1);   // free since the last barrier
       if (ktile < my_end) {
         const int j = kbase + n;
         const bool edge = !INTERIOR && ((kbase + TILE - 1 >= qbase) || (kbase + TILE > T) || kbase < exempt);
         const TileMasks mk(j, qbase, T, exempt, h);
-        const float hist = B.hist[wave][lane], uin = B.uin[wave][lane];
+        const float hist = B.hist[wave][lane];
+        float uin = B.uin[wave][lane];
+        if (!INTERIOR && walk.far && ktile < i_lo) uin = 0.f;   // (past the sweep's start: no row written)
         const elem* k0s = H0 ? B.k[0] : B.k[1];
         f32x16 l0 = zero16();
 #pragma unroll
@@ -3406,22 +3810,31 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
       wait_loads();
       __syncthreads();   // the next tile's operands are in; every wavefront is done with this one
     };
-    auto run = [&](int t0, int t1, auto interior_tag) {
-      int t = t0;
-      if (t < t1 && (t & 1)) tile_step(t++, interior_tag, std::true_type{});
-      for (; t + 1 < t1; t += 2) {
-        tile_step(t, interior_tag, std::false_type{});
-        tile_step(t + 1, interior_tag, std::true_type{});
+    bool odd = false;
+    auto run = [&](int stop, auto interior_tag) {   // tiles from ktile up to `stop`, in pairs
+      auto shift = [&]() {
+        ktile = next;
+        next = walk.after(next);
+      };
+      if (odd && ktile < stop) {
+        tile_step(interior_tag, std::true_type{});
+        shift();
+        odd = false;
       }
-      if (t < t1) tile_step(t, interior_tag, std::false_type{});
+      while (ktile < stop) {
+        tile_step(interior_tag, std::false_type{});
+        shift();
+        if (ktile >= stop) {
+          odd = true;
+          break;
+        }
+        tile_step(interior_tag, std::true_type{});
+        shift();
+      }
     };
-    // tiles holding exempt keys, then the interior ones (below every wavefront's diagonal, which
-    // also keeps them clear of the sequence end), then the diagonals
-    const int i_lo = min((exempt + TILE - 1) / TILE, wg_end);
-    const int i_hi = max(i_lo, min(qsb * DQ64_WAVES, wg_end));
-    run(0, i_lo, std::false_type{});
-    run(i_lo, i_hi, std::true_type{});
-    run(i_hi, wg_end, std::false_type{});
+    run(i_lo, std::false_type{});
+    run(i_hi, std::true_type{});
+    run(wg_end, std::false_type{});
   };
   if (SOLO || has_h0) sweep(std::true_type{});
   else if constexpr (!SOLO) sweep(std::false_type{});
@@ -3453,14 +3866,43 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
   }
 }
 
-// Head 0's gradients: its own fp32 sums plus the other groups' shares, summed slot after slot in
-// group order (so every run adds the same values in the same order), (b, t, D) contiguous, four
-// elements per thread, to the caller's views. nslots slots of total4 float4s each.
+// The gradient epilogue. Workgroups [0, main_blocks): head 0's gradients, its own fp32 sums plus the other
+// groups' shares, summed slot after slot in group order (so every run adds the same values in the same
+// order), (b, t, D) contiguous, four elements per thread, to the caller's views; nslots slots of total4
+// float4s each. The workgroups past them: the first xk (exempt) keys' dK and dV of all R heads, the sums of
+// bwd_rowprep_kernel's row segments: 32 float4s of a head per workgroup, eight threads along the segments,
+// their sums added in order.
 __global__ __launch_bounds__(NTHREADS) void bwd_finish_kernel(
     const float4* __restrict__ dq0h, const float4* __restrict__ dk0h, const float4* __restrict__ dq0x,
-    const float4* __restrict__ dk0x, int nslots, GradView dqv, GradView dkv, int D, int64_t TD, int64_t total4,
-    float scale) {
-  for (int64_t e = (int64_t)blockIdx.x * NTHREADS + threadIdx.x; e < total4; e += (int64_t)gridDim.x * NTHREADS) {
+    const float4* __restrict__ dk0x, int nslots, GradView dqv, GradView dkv, GradView dvv, int D, int64_t TD,
+    int64_t total4, float scale, int main_blocks, int R, int H, BwdReach reach) {
+  if ((int)blockIdx.x >= main_blocks) {
+    __shared__ float4 sSum[8][32];
+    const int per = reach.xk * 2 * D / 4;   // float4s of one head: (key, dK | dV, D)
+    const int64_t e = (int64_t)(blockIdx.x - main_blocks) * 32 + (threadIdx.x & 31);
+    const bool ok = e < (int64_t)R * per;
+    const int r = ok ? (int)(e / per) : 0, i = ok ? (int)(e % per) : 0, sl = threadIdx.x >> 5;
+    const float4* p = reinterpret_cast<const float4*>(reach.xpart) + (int64_t)r * reach.nseg * per + i;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 8
+    for (int s = sl; s < reach.nseg; s += 8) {
+      const float4 x = p[(int64_t)s * per];
+      a = make_float4(a.x + x.x, a.y + x.y, a.z + x.z, a.w + x.w);
+    }
+    sSum[sl][threadIdx.x & 31] = a;
+    __syncthreads();
+    if (sl != 0 || !ok) return;
+#pragma unroll
+    for (int w = 1; w < 8; ++w) {
+      const float4 x = sSum[w][threadIdx.x];
+      a = make_float4(a.x + x.x, a.y + x.y, a.z + x.z, a.w + x.w);
+    }
+    const int j = i / (2 * D / 4), c = i % (2 * D / 4), d = 4 * (c % (D / 4));
+    if (c < D / 4) store_grad4(dkv, r / H, r % H, j, d, make_float4(a.x * scale, a.y * scale, a.z * scale, a.w * scale));
+    else store_grad4(dvv, r / H, r % H, j, d, a);
+    return;
+  }
+  for (int64_t e = (int64_t)blockIdx.x * NTHREADS + threadIdx.x; e < total4; e += (int64_t)main_blocks * NTHREADS) {
     const int64_t b = (4 * e) / TD, off = 4 * e - b * TD;
     const int t = (int)(off / D), d = (int)(off - (int64_t)t * D);
     float4 q = dq0h[e], k = dk0h[e];
@@ -3470,7 +3912,7 @@ __global__ __launch_bounds__(NTHREADS) void bwd_finish_kernel(
       k = make_float4(k.x + kx.x, k.y + kx.y, k.z + kx.z, k.w + kx.w);
     }
     store_grad4(dqv, b, 0, t, d, make_float4(q.x * scale, q.y * scale, q.z * scale, q.w * scale));
-    store_grad4(dkv, b, 0, t, d, k);
+    if (t >= reach.xk) store_grad4(dkv, b, 0, t, d, k);
   }
 }
 
@@ -3863,6 +4305,15 @@ int forward_impl(const FwdCall& c) {
   return launch_status();
 }
 
+template <class OP, int D>
+void launch_rowprep(const BwdCall& c, const PrepLaunch& p) {
+  using elem = typename OP::elem;
+  hipLaunchKernelGGL((bwd_rowprep_kernel<OP, D>), dim3((unsigned)cdiv(p.ldt, QSTAT_ROWS), (unsigned)(c.nseq * c.H)),
+                     dim3(NTHREADS), 0, c.st, static_cast<const elem*>(c.q), static_cast<const elem*>(c.k),
+                     static_cast<const elem*>(c.v), static_cast<const elem*>(c.dout), c.qs, c.ks, c.vs, c.dos, c.H, c.T,
+                     c.out, c.rmax, c.rden, p.lse, p.ndbar, p.ldt, c.scale, p.reach);
+}
+
 // Launch of the key-side kernel from its arguments (the grid as launch_bwd's).
 template <class OP, int D, int G, bool CV>
 void launch_kv_from(const KvLaunch& a) {
@@ -3872,7 +4323,7 @@ void launch_kv_from(const KvLaunch& a) {
                      static_cast<const elem*>(a.k), static_cast<const elem*>(a.v), static_cast<const elem*>(a.qt),
                      static_cast<const elem*>(a.dout), static_cast<const elem*>(a.dot), a.qs, a.ks, a.vs, a.dos, a.lse,
                      a.dbar, a.carry, a.ucheck, a.dk0h, a.dk0x, a.dkv, a.dvv, a.nseq, a.H, a.T, a.ldt, a.exempt,
-                     a.scale);
+                     a.scale, a.reach);
 }
 
 template <bool CV, bool SOLO>
@@ -3881,14 +4332,14 @@ void launch_kv64_from(const KvLaunch& a) {
   hipLaunchKernelGGL((bwd_kv64_kernel<CV, SOLO>), grid, dim3(NTHREADS), 0, a.st, static_cast<const uint16_t*>(a.q),
                      static_cast<const uint16_t*>(a.k), static_cast<const uint16_t*>(a.v),
                      static_cast<const uint16_t*>(a.dout), a.qs, a.ks, a.vs, a.dos, a.lse, a.dbar, a.carry, a.ucheck,
-                     a.dk0h, a.dk0x, a.dkv, a.dvv, a.nseq, a.H, a.T, a.ldt, a.exempt, a.scale);
+                     a.dk0h, a.dk0x, a.dkv, a.dvv, a.nseq, a.H, a.T, a.ldt, a.exempt, a.scale, a.reach);
 }
 
 // The two backward kernels; returns the launch status.
 template <class OP, int D, int G>
 int launch_bwd(const BwdCall& c, const typename OP::elem* qt, const typename OP::elem* kt,
                 const typename OP::elem* dot, const float* lse, const float* dbar, float* ucheck, float* dq0h,
-                float* dk0h, float* dq0x, float* dk0x, int64_t ldt) {
+                float* dk0h, float* dq0x, float* dk0x, int64_t ldt, const BwdReach& reach) {
   using elem = typename OP::elem;
   const elem* q = static_cast<const elem*>(c.q);
   const elem* k = static_cast<const elem*>(c.k);
@@ -3904,7 +4355,7 @@ int launch_bwd(const BwdCall& c, const typename OP::elem* qt, const typename OP:
   const GradView dqv{c.dq, c.dqs, f32}, dkv{c.dk, c.dks, f32}, dvv{c.dv, c.dvs, f32};
   const KvLaunch kv{q,    k,       v,      qt,   dout, dot,    c.qs, c.ks, c.vs, c.dos,    lse,      dbar,
                     c.carry, ucheck, dk0h, dk0x, dkv,  dvv,    c.nseq, c.H,  c.T,  ldt,      c.exempt, c.scale,
-                    c.st};
+                    reach, c.st};
   // bf16: the key-side kernel's instances live in a translation unit of their own (sa_bf16_kv.hip)
   auto launch_kv = [&](bool cvv) -> int {
     if constexpr (sizeof(elem) == 2) {
@@ -3918,7 +4369,7 @@ int launch_bwd(const BwdCall& c, const typename OP::elem* qt, const typename OP:
 #define SA_LAUNCH_DQ(CVV)                                                                                         \
   hipLaunchKernelGGL((bwd_dq_kernel<OP, D, G, CVV>), grid, dim3(NTHREADS), 0, c.st, q, k, v, kt, dout, c.qs, c.ks, \
                      c.vs, c.dos, lse, dbar, c.carry, ucheck, dq0h, dq0x, dqv, c.nseq, c.H, c.T, ldt, c.exempt,   \
-                     c.scale)
+                     c.scale, reach)
   {
     TimedLaunch timed(SA_KERNEL_BACKWARD, c.st);
     const int rc = launch_kv(cv);
@@ -3931,7 +4382,7 @@ int launch_bwd(const BwdCall& c, const typename OP::elem* qt, const typename OP:
 #define SA_LAUNCH_DQ64(CVV, SOLO, SNAKE)                                                                           \
   hipLaunchKernelGGL((bwd_dq64_kernel<CVV, SOLO, SNAKE>), grid64, dim3(DQ64_WAVES * 64), 0, c.st, q, k, v, dout, c.qs, \
                      c.ks, c.vs, c.dos, lse, dbar, c.carry, ucheck, dq0h, dq0x, dqv, c.nseq, c.H, c.T, ldt, c.exempt, \
-                     c.scale, dq_slots)
+                     c.scale, dq_slots, reach)
       const int dq_slots = bwd_snake_slots((int64_t)grid64.x * grid64.y, 1, device_cus());
       if (c.H == 1) {   // one-head sequences: head 0's loop only
         if (cv) SA_LAUNCH_DQ64(true, true, false);
@@ -3984,11 +4435,22 @@ int backward_impl(const BwdCall& c) {
     launch_transpose<elem, D>(dout, dot, T, ldt, c.dos, H, R, st);
     launch_transpose<elem, D>(k, kt, T, ldt, c.ks, H, R, st);
   }
-  hipLaunchKernelGGL((bwd_rowstats_kernel<OP, D>), dim3((unsigned)cdiv(R * ldt * (D / 8), NTHREADS)),
-                     dim3(NTHREADS), 0, st, dout, c.dos, H, T, c.out, c.rmax, c.rden, lse, dbar, ldt, R * ldt);
+  BwdReach reach{};
+  reach.nseg = (int)cdiv(T, QSTAT_ROWS);
+  reach.nkg = (int)cdiv(T, NWAVES * TILE);
+  if (c.reach) {
+    const BwdReachLayout RL = bwd_reach_layout(nseq, H, T, D);
+    reach.qstat = reinterpret_cast<float2*>(c.reach + RL.qstat);
+    reach.hi = reinterpret_cast<int*>(c.reach + RL.hi);
+    reach.xpart = reinterpret_cast<float*>(c.reach + RL.xpart);
+    reach.xk = c.exempt <= EXEMPT_APART ? c.exempt : 0;
+  }
+  const PrepLaunch prep{lse, dbar, ldt, reach};
+  if constexpr (sizeof(elem) == 2) launch_rowprep_bf16(c, prep);
+  else launch_rowprep<OP, D>(c, prep);
   int rc = launch_status();   // the transposes and row statistics
   if (rc) return rc;
-#define SA_LAUNCH_BWD(GG) launch_bwd<OP, D, GG>(c, qt, kt, dot, lse, dbar, ucheck, dq0h, dk0h, dq0x, dk0x, ldt)
+#define SA_LAUNCH_BWD(GG) launch_bwd<OP, D, GG>(c, qt, kt, dot, lse, dbar, ucheck, dq0h, dk0h, dq0x, dk0x, ldt, reach)
   if constexpr (sizeof(elem) == 2 && D <= 32) {
     rc = (G == 2) ? SA_LAUNCH_BWD(2) : SA_LAUNCH_BWD(1);
   } else {
@@ -3996,16 +4458,19 @@ int backward_impl(const BwdCall& c) {
   }
 #undef SA_LAUNCH_BWD
   if (rc) return rc;
-  if (H == 1) return SA_OK;   // a one-head sequence's kernels wrote its gradients to the views
+  // (a one-head sequence's kernels wrote its gradients to the views, but for the exempt keys')
+  if (H == 1 && reach.xk == 0) return SA_OK;
   // head 0's dQ, dK: its own sums plus the other groups' shares
-  const int64_t total4 = (int64_t)nseq * T * D / 4;
+  const int64_t total4 = H == 1 ? 0 : (int64_t)nseq * T * D / 4;
   const int f32 = c.grad_dtype == SA_DTYPE_F32;
-  hipLaunchKernelGGL(bwd_finish_kernel, dim3((unsigned)std::min<int64_t>(cdiv(total4, NTHREADS), 8192)),
+  const unsigned main_blocks = (unsigned)std::min<int64_t>(cdiv(total4, NTHREADS), 8192);
+  const unsigned exempt_blocks = (unsigned)cdiv(R * reach.xk * 2 * D / 4, 32);
+  hipLaunchKernelGGL(bwd_finish_kernel, dim3(main_blocks + exempt_blocks),
                      dim3(NTHREADS), 0, st, reinterpret_cast<const float4*>(dq0h),
                      reinterpret_cast<const float4*>(dk0h), reinterpret_cast<const float4*>(dq0x),
                      reinterpret_cast<const float4*>(dk0x), H / G - 1, GradView{c.dq, c.dqs, f32},
-                     GradView{c.dk, c.dks, f32}, D,
-                     (int64_t)T * D, total4, c.scale);
+                     GradView{c.dk, c.dks, f32}, GradView{c.dv, c.dvs, f32}, D,
+                     (int64_t)T * D, total4, c.scale, (int)main_blocks, (int)R, H, reach);
   return launch_status();
 }
 

@@ -82,3 +82,50 @@ def test_forward_past_the_mask_keeps_its_bits(cuda):
     q, k, v, _ = _inputs(cuda, 1, 1, t, 64, torch.bfloat16, "normal")
     for got, want in zip(_forward(q, k, v, 1, True, 500), _forward(q, k, v, 1, False, 500)):
         assert torch.equal(_bits(got), _bits(want))
+
+
+def _backward(q, k, v, do, aux, exempt, reach, grad_bf16):
+    lib = _lib.load()
+    b, h, t, d = q.shape
+    code = kernels._code_of(q)
+    out, rmax, rden, carry = aux
+    grads = [torch.empty(q.shape, device=q.device, dtype=torch.bfloat16 if grad_bf16 else torch.float32) for _ in range(3)]
+    size = lib.sa_backward_workspace_bytes(b, h, t, d, code, 0) + (lib.sa_reach_bytes(b, h, t, d) if reach else 0)
+    # (the rows of the checkpoint planes that no sweep writes are read as NaN if anything takes them)
+    ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=q.device)
+    _lib.check(lib.sa_backward(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), rmax.data_ptr(),
+                               rden.data_ptr(), carry.data_ptr(), *(x.data_ptr() for x in grads), ws.data_ptr(), size, b, h,
+                               t, d, 1 / math.sqrt(d), code, _lib.DTYPE_BF16 if grad_bf16 else _lib.DTYPE_F32, exempt, 0,
+                               torch.cuda.current_stream().cuda_stream))
+    return grads
+
+
+@pytest.mark.parametrize("kind", ["normal", "holes", "sparse", "special"])
+@pytest.mark.parametrize("b,h,t,d,dtype", SHAPES)
+def test_backward_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
+    """With more than 32 exempt keys the same instances of the kernels run: every bit. Up to 32 of them the
+    exempt keys' dK, dV are summed by row segments, and the first 128 keys' tiles run an instance of their own,
+    whose suffix sums the compiler may round elsewhere (one fp32 ulp seen, in head 0's dQ too): every bit of
+    the later keys' dK, dV, the rest to rounding."""
+    print(f"case backward {b} {h} {t} {d} {dtype} {kind}", flush=True)
+    bf16 = dtype == "bf16"
+    q, k, v, do = _inputs(cuda, b, h, t, d, torch.bfloat16 if bf16 else torch.float32, kind)
+    for exempt in (1, 16, 32, 40):
+        aux = _forward(q, k, v, exempt, True)[:4]
+        half = bf16 and exempt == 1
+        got = _backward(q, k, v, do, aux, exempt, True, half)
+        want = _backward(q, k, v, do, aux, exempt, False, half)
+        first = 128 if exempt <= 32 else 0
+        for x, y in zip(got[1:], want[1:]):
+            assert torch.equal(_bits(x[:, :, first:]), _bits(y[:, :, first:])), exempt
+        if first == 0:
+            assert torch.equal(_bits(got[0]), _bits(want[0])), exempt
+            continue
+        for x, y in zip(got, want):
+            x, y = x.double(), y.double()
+            assert torch.equal(x.isnan(), y.isnan())
+            fine = y.isfinite()
+            # dQ: 1e-7 of fp32 rounding; dK, dV of the exempt keys: split bf16 operands (2^-16 each) or fp32
+            # products summed in another order; a bf16 gradient's own rounding beside that
+            tol = 2.0 ** -8 if half else 2.0 ** -14 if bf16 else 2.0 ** -18
+            assert (x - y)[fine].norm() <= tol * y[fine].norm() + 1e-30, exempt
