@@ -244,12 +244,29 @@ def _launch_forward(qs: Tensor, ks: Tensor, vs: Tensor, kstride: int, scale: flo
 
 # -- the C-ABI calls as custom ops ------------------------------------------------------------------
 
-@torch.library.custom_op("selective_attention::forward", mutates_args=(), device_types="cuda")
-def _forward_op(q: Tensor, k: Tensor, v: Tensor, scale: float, exempt: int, group: int, damp_mode: int,
+def _plain(*tensors: Tensor) -> bool:
+    """Whether a custom op call on these tensors could only end in its own CUDA implementation: plain tensors,
+    nothing that traces, transforms or records ops, and no gradient to ask of the op itself (which has no
+    formula: a second derivative raises). The implementation is then called as it is: the op's Python
+    layers take 13 us of host time per call, a tenth of a short training step."""
+    return (all(type(t) in (Tensor, torch.nn.Parameter) for t in tensors)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._ops._len_torch_dispatch_stack_pre_dispatch() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._get_tracing_state()
+            and not torch.autograd._profiler_enabled())
+
+
+def _forward_impl(q: Tensor, k: Tensor, v: Tensor, scale: float, exempt: int, group: int, damp_mode: int,
                 train_len: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """sa_forward on contiguous (B, H, T, Dk) storage tensors (bf16 or fp32): out (B, H, T, Dk) fp32,
     rmax, rden (B, H, T), carry (B, ceil(T/32), T), selected_total (B, T)."""
     return _launch_forward(q, k, v, k.shape[-2] * k.shape[-1], scale, exempt, group, damp_mode, train_len)
+
+
+_forward_op = torch.library.custom_op("selective_attention::forward", mutates_args=(), device_types="cuda")(_forward_impl)
 
 
 @_forward_op.register_fake
@@ -262,8 +279,7 @@ def _forward_fake(q, k, v, scale, exempt, group, damp_mode, train_len):
             q.new_empty((batch, seq), **f32))
 
 
-@torch.library.custom_op("selective_attention::backward", mutates_args=(), device_types="cuda")
-def _backward_op(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, rmax: Tensor, rden: Tensor,
+def _backward_impl(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, rmax: Tensor, rden: Tensor,
                  carry: Tensor, scale: float, exempt: int, group: int,
                  grad_bf16: bool) -> tuple[Tensor, Tensor, Tensor]:
     """sa_backward: dq, dk, dv (B, H, T, Dk) in bf16 (grad_bf16) or fp32, from the storage tensors,
@@ -284,6 +300,9 @@ def _backward_op(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, rma
     return dq, dk, dv
 
 
+_backward_op = torch.library.custom_op("selective_attention::backward", mutates_args=(), device_types="cuda")(_backward_impl)
+
+
 @_backward_op.register_fake
 def _backward_fake(q, k, v, out, dout, rmax, rden, carry, scale, exempt, group, grad_bf16):
     gdt = torch.bfloat16 if grad_bf16 else torch.float32
@@ -297,8 +316,7 @@ def _packed_strides(batch: int, seq: int, heads: int, head_dim: int):
     return _lib.ViewStrides(seq * c3, head_dim, c3), _lib.ViewStrides(seq * cdim, head_dim, cdim)
 
 
-@torch.library.custom_op("selective_attention::qkv_forward", mutates_args=(), device_types="cuda")
-def _qkv_forward_op(qkv: Tensor, heads: int, exempt: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+def _qkv_forward_impl(qkv: Tensor, heads: int, exempt: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """sa_forward_strided on a packed (B, T, 3 * H * D) projection read in place: the output y
     (B, T, H * D) in qkv's dtype, and the fp32 output (B, H, T, D), rmax, rden, carry saved for the
     backward."""
@@ -326,6 +344,9 @@ def _qkv_forward_op(qkv: Tensor, heads: int, exempt: int) -> tuple[Tensor, Tenso
     return y, out, rmax, rden, carry
 
 
+_qkv_forward_op = torch.library.custom_op("selective_attention::qkv_forward", mutates_args=(), device_types="cuda")(_qkv_forward_impl)
+
+
 @_qkv_forward_op.register_fake
 def _qkv_forward_fake(qkv, heads, exempt):
     batch, seq, c3 = qkv.shape
@@ -336,8 +357,7 @@ def _qkv_forward_fake(qkv, heads, exempt):
             qkv.new_empty((batch, (seq + CARRY_M - 1) // CARRY_M, seq), **f32))
 
 
-@torch.library.custom_op("selective_attention::qkv_backward", mutates_args=(), device_types="cuda")
-def _qkv_backward_op(qkv: Tensor, dy: Tensor, out: Tensor, rmax: Tensor, rden: Tensor, carry: Tensor, heads: int,
+def _qkv_backward_impl(qkv: Tensor, dy: Tensor, out: Tensor, rmax: Tensor, rden: Tensor, carry: Tensor, heads: int,
                      exempt: int) -> Tensor:
     """sa_backward_strided for the packed form: the gradient of qkv as one (B, T, 3 * H * D) tensor,
     from dy (B, T, H * D) in qkv's dtype."""
@@ -358,6 +378,9 @@ def _qkv_backward_op(qkv: Tensor, dy: Tensor, out: Tensor, rmax: Tensor, rden: T
             gbase + 2 * cdim * es, qkv_s, ws.data_ptr(), ws.numel(), batch, heads, seq, head_dim,
             1.0 / math.sqrt(head_dim), code, code, exempt, 0, _stream(dev)))
     return dqkv
+
+
+_qkv_backward_op = torch.library.custom_op("selective_attention::qkv_backward", mutates_args=(), device_types="cuda")(_qkv_backward_impl)
 
 
 @_qkv_backward_op.register_fake
@@ -399,8 +422,9 @@ def selective_attention_forward(
     head_dim = q.shape[-1]
     kdim = _kernel_dim(head_dim)
     qs, ks, vs = (_storage(t, code, kdim) for t in (q, k, v))
-    out, rmax, rden, carry, total = _forward_op(qs, ks, vs, 1.0 / math.sqrt(head_dim), exempt, int(group or 0),
-                                                damp_mode, int(train_len))
+    forward = _forward_impl if _plain(qs, ks, vs) else _forward_op
+    out, rmax, rden, carry, total = forward(qs, ks, vs, 1.0 / math.sqrt(head_dim), exempt, int(group or 0), damp_mode,
+                                            int(train_len))
     result = out[..., :head_dim].contiguous() if kdim != head_dim else out
     if return_aux:
         n = q.shape[0] * q.shape[1]
@@ -538,8 +562,8 @@ class _SelectiveAttentionFn(torch.autograd.Function):
         head_dim = q.shape[-1]
         kdim = _kernel_dim(head_dim)
         qs, ks, vs = (_storage(t, code, kdim) for t in (q, k, v))
-        out, rmax, rden, carry, _ = _forward_op(qs, ks, vs, 1.0 / math.sqrt(head_dim), exempt, int(group or 0),
-                                                0, 0)
+        forward = _forward_impl if _plain(qs, ks, vs) else _forward_op
+        out, rmax, rden, carry, _ = forward(qs, ks, vs, 1.0 / math.sqrt(head_dim), exempt, int(group or 0), 0, 0)
         ctx.save_for_backward(qs, ks, vs, out, rmax, rden, carry)
         ctx.exempt, ctx.bwd_group, ctx.head_dim = exempt, bwd_group, head_dim
         ctx.in_dtypes = (q.dtype, k.dtype, v.dtype)
@@ -554,8 +578,8 @@ class _SelectiveAttentionFn(torch.autograd.Function):
         # gradients leave the kernel in the input dtype when every input is stored as-is (bf16 inputs
         # on bf16 operands); otherwise in fp32, cast below (the reference's dq.to(q.dtype))
         as_bf16 = qs.dtype == torch.bfloat16 and all(d == torch.bfloat16 for d in ctx.in_dtypes)
-        grads = _backward_op(qs, ks, vs, out, dos, rmax, rden, carry, 1.0 / math.sqrt(head_dim), ctx.exempt,
-                             group, as_bf16)
+        backward = _backward_impl if _plain(qs, ks, vs, out, dos, rmax, rden, carry) else _backward_op
+        grads = backward(qs, ks, vs, out, dos, rmax, rden, carry, 1.0 / math.sqrt(head_dim), ctx.exempt, group, as_bf16)
         grads = tuple(g[..., :head_dim].to(want) for g, want in zip(grads, ctx.in_dtypes))
         return grads + (None,) * 11
 
@@ -572,7 +596,8 @@ class _SelectiveAttentionQKVFn(torch.autograd.Function):
     def forward(ctx, qkv, heads, dot_precision, exempt):
         _packed_layout(qkv, heads, dot_precision)
         exempt = _check_exempt(exempt)
-        y, out, rmax, rden, carry = _qkv_forward_op(qkv, heads, exempt)
+        forward = _qkv_forward_impl if _plain(qkv) else _qkv_forward_op
+        y, out, rmax, rden, carry = forward(qkv, heads, exempt)
         ctx.save_for_backward(qkv, out, rmax, rden, carry)
         ctx.heads, ctx.exempt = heads, exempt
         return y
@@ -580,7 +605,9 @@ class _SelectiveAttentionQKVFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         qkv, out, rmax, rden, carry = ctx.saved_tensors
-        dqkv = _qkv_backward_op(qkv, dy.to(qkv.dtype).contiguous(), out, rmax, rden, carry, ctx.heads, ctx.exempt)
+        dy = dy.to(qkv.dtype).contiguous()
+        backward = _qkv_backward_impl if _plain(qkv, dy, out, rmax, rden, carry) else _qkv_backward_op
+        dqkv = backward(qkv, dy, out, rmax, rden, carry, ctx.heads, ctx.exempt)
         return dqkv, None, None, None
 
 

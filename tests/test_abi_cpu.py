@@ -235,3 +235,32 @@ def test_packed_form_stays_within_32_bit_row_offsets():
     assert kernels._packed_rows_fit(300_000, c3, 2)
     assert not kernels._packed_rows_fit(350_000, c3, 2)   # (T + 64) * 3072 * 2 bytes >= 2^31
     assert not kernels._packed_rows_fit(175_000, c3, 4)
+
+
+def test_ops_are_passed_by_only_for_plain_eager_tensors():
+    """The implementations are called without their ops only where the op layer could add nothing: not for
+    fake or subclassed tensors, under a dispatch mode, a functorch transform or the profiler, nor when a
+    gradient of the op itself would be asked for."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.zeros(2)
+    p = torch.nn.Parameter(torch.zeros(2))
+    assert kernels._plain(x, x)
+    assert not kernels._plain(x, p)
+    with torch.no_grad():
+        assert kernels._plain(x, p)
+    with FakeTensorMode():
+        assert not kernels._plain(torch.zeros(2))
+    with Mode():
+        assert not kernels._plain(x)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        assert not kernels._plain(x)
+    seen = []
+    torch.func.vmap(lambda t: seen.append(kernels._plain(x)) or t)(torch.zeros(3, 2))
+    assert seen == [False]
+    assert not kernels._plain(torch.zeros(2).as_subclass(type("Sub", (torch.Tensor,), {})))
