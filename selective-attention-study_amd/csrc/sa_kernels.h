@@ -690,17 +690,17 @@ __device__ __forceinline__ float block_selection_sum(const f32x16& acc, bool int
 //
 //     log2 weight <= s log2e (max |q|) (max |k|) - log2e (min F) - (min row maximum so far),
 //
-// and exp2 returns exactly zero below -149 (-126 where denormals flush). A tile whose bound lies
-// below -REACH_ZERO (a margin for the rounding of the bound's own terms: the norms are taken 1% high,
-// F a thousandth low) is left out of the sweep: the skipped terms are zeros, so the results keep their
-// bits. Nothing is skipped where a zero weight would not give a zero term: a tile with a key or value
+// and v_exp_f32 returns exactly zero below -126 (it flushes denormal results). A tile whose bound lies
+// below -REACH_ZERO (a margin for the rounding of the bound's own terms; besides, the norms are taken 1%
+// high and F a thousandth low) is left out of the sweep: the skipped terms are zeros, so the results keep
+// their bits. Nothing is skipped where a zero weight would not give a zero term: a tile with a key or value
 // that is not finite, or so large that a product of two rows could overflow, gets the bound infinity,
 // and every comparison is written so that a NaN keeps the tile.
 // Measured (forward kernel, bf16, D=64, N(0,1) inputs, whose histories grow by 0.4 a query): B=1 H=16
 // T=16384 918 -> 97 us, the last 16384 queries of 131072 13.2 -> 0.17 ms, B=2 H=12 T=2048 85 -> 35 us; where
 // one pair in a hundred is selected and nothing can be left out: B=2 H=12 T=5003 249 -> 250 us, B=1 H=12
 // T=16384 740 -> 751 us, and the key norms add 2 and 6 us to the column sums' launch.
-constexpr float REACH_ZERO = 160.f;
+constexpr float REACH_ZERO = 132.f;
 constexpr float REACH_NORM2 = 1e37f;      // sums of squares at or past this count as not finite
 constexpr float REACH_Q = 1.01f * LOG2E;
 constexpr float REACH_F = 0.999f * LOG2E;
@@ -2189,8 +2189,7 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 && D <= 6
 // exact zero, of the blocks up to NB - 1 (the key tile's own block at least): a lane group of 8 probes one
 // block (4 keys per lane), eight blocks at a time; the history never falls, so the blocks past the last
 // one are all without weight. thr: see find_reach, with the head's least lse for the row maxima. Keys
-// below xk (their gradients are taken elsewhere) and past the end do not count. The first probe, the last
-// block, is all it costs where nothing can be left out.
+// below xk (their gradients are taken elsewhere) and past the end do not count.
 __device__ __forceinline__ int kv_last_block(const float* carry_b, int T, int NB, int key0, int xk, float thr,
                                              int lane) {
   const int part = lane >> 3, j0 = key0 + 4 * (lane & 7);
@@ -2205,17 +2204,31 @@ __device__ __forceinline__ int kv_last_block(const float* carry_b, int T, int NB
     }
     return ok;
   };
-  if (__ballot(gone(NB - 1)) != ~0ull) return NB - 1;
-  int lo = key0 / TILE, hi = NB - 1;   // lo: kept; hi: without weight
-  while (hi - lo > 1) {
-    const int stride = max(1, (hi - lo) / 9);
-    const uint64_t m = __ballot(gone(min(lo + (part + 1) * stride, hi)));
-    int first = 8;
+  int lo = key0 / TILE, hi = NB;   // lo: kept; hi: without weight (or past the end)
+  auto narrow = [&](auto probe) {   // probe(i), i = 0..7, ascending
+    const uint64_t m = __ballot(gone(min(probe(part), NB - 1)));
+    int nlo = lo, nhi = hi;
 #pragma unroll
-    for (int i = 7; i >= 0; --i) first = ((m >> (8 * i)) & 0xFF) == 0xFF ? i : first;
-    const int nhi = first < 8 ? min(lo + (first + 1) * stride, hi) : hi;
-    lo = min(lo + first * stride, nhi - 1);
+    for (int i = 7; i >= 0; --i) {
+      const int p = min(probe(i), NB - 1);
+      if (((m >> (8 * i)) & 0xFF) == 0xFF) nhi = min(nhi, p);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int p = min(probe(i), NB - 1);
+      if (((m >> (8 * i)) & 0xFF) != 0xFF && p < nhi) nlo = max(nlo, p);
+    }
+    lo = nlo;
     hi = nhi;
+  };
+  // first the last block -- where nothing can be left out that is all -- and, for the usual reach of a few
+  // tiles, the blocks 2, 4, ... 128 on
+  const int at = lo;
+  narrow([&](int i) { return i == 7 ? NB - 1 : at + (2 << i); });
+  if (hi == NB) return NB - 1;
+  while (hi - lo > 1) {
+    const int from = lo, stride = max(1, (hi - lo) / 9);
+    narrow([&](int i) { return min(from + (i + 1) * stride, hi - 1); });
   }
   return lo;
 }
