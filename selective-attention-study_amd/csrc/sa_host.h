@@ -69,14 +69,14 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int launch_status() { return hipGetLastError() == hipSuccess ? SA_OK : SA_ERR_LAUNCH; }
 
 // Heads per wavefront of the forward (a group shares head 0's selection work: its logits, F):
-// 4 at head dim <= 32, 2 at 64 (two heads' output sums in registers leave two workgroups per CU,
-// which measures faster than three with one head), 1 beyond; fp32 storage 1.
+// 2 at bf16 head dim <= 64 (one where the grid is small: fwd64_group), 1 beyond; fp32 storage 1. Four
+// heads per wavefront, at head dim 32 on request, measure slower everywhere.
 inline int auto_group(int dtype, int64_t D, int64_t heads, int requested, bool backward) {
   int g = requested;
   if (g <= 0) {
     if (dtype == SA_DTYPE_F32) g = 1;
     else if (backward) g = (D <= 32) ? 2 : 1;
-    else g = (D <= 32) ? 4 : (D <= 64 ? 2 : 1);
+    else g = D <= 64 ? 2 : 1;
   }
   int cap = (dtype == SA_DTYPE_F32) ? 1 : (backward ? 2 : 4);
   if (D >= 128 || (backward && D >= 64)) cap = 1;
@@ -85,7 +85,7 @@ inline int auto_group(int dtype, int64_t D, int64_t heads, int requested, bool b
   return g < 1 ? 1 : g;
 }
 
-// Heads per wavefront of the bf16 head-dim-64 forward when the caller leaves the choice open and
+// Heads per wavefront of the bf16 forward at head dims 32 and 64 when the caller leaves the choice open and
 // auto_group allows two. Two heads per wavefront share head 0's selection and run two workgroups per
 // CU; one head per wavefront runs three per CU with half the work per workgroup, and gives the same
 // bits (fwd64_kernel). Two win once their grid needs more than one round of workgroups (more than two
@@ -95,7 +95,10 @@ inline int auto_group(int dtype, int64_t D, int64_t heads, int requested, bool b
 // ms, one / two heads per wavefront, B x H x T): 1x16x16384 1.27 / 0.99, 1x12x16384 0.90 / 0.71,
 // 2x12x8192 0.46 / 0.36, 4x16x4096 0.33 / 0.27 (more than one round); 1x8x16384 0.61 / 0.65,
 // 1x16x8192 0.31 / 0.33, 1x12x8192 0.28 / 0.32, 2x12x4096 0.15 / 0.17, 1x2x16384 0.50 / 0.62 (one
-// round or less).
+// round or less). The head-dim-32 forward takes the same rule (call, us, one / two / four heads per
+// wavefront, nothing skipped): 8x12x2048 186 / 159 / 188, 1x16x16384 1081 / 891 / 1478 (more than one
+// round); 4x8x1000 50 / 59 / 81, 4x8x2048 103 / 102 / 144, 4x8x4096 219 / 230 / 268, 1x8x8192
+// 285 / 332 / 494 (one or less).
 inline int fwd64_group(int64_t nseq, int64_t heads, int64_t tq, int cus) {
   if (heads % 2 != 0) return 1;
   const int64_t workgroups = nseq * (heads / 2) * cdiv(cdiv(tq, TILE), NWAVES);

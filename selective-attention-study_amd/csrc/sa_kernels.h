@@ -1241,6 +1241,10 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
   const int b = bxy.y / groups, gi = bxy.y % groups;
   const int hd0 = gi * G;
   const bool has_h0 = (gi == 0);
+  // a one-head group holding head 0 sends that head's whole adjusted logit through LDS, one product per
+  // tile instead of two; not at head dim 32 beside other heads, where the host chooses the width per
+  // launch and every width is to give the same bits (see fwd64_kernel)
+  const bool whole = G == 1 && has_h0 && (D > 32 || H == 1);
   const int NBq = (Tq + TILE - 1) / TILE;
   const int NKT = (Tk + TILE - 1) / TILE;
   const int qsb = gridDim.x - 1 - bxy.x;
@@ -1410,10 +1414,9 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
             const float dmv[4] = {dm.x, dm.y, dm.z, dm.w};
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-              // a one-head group holding head 0 sends that head's whole adjusted logit,
-              // q.k - damp F/s, so its (keys x queries) product is not taken again
+              // (whole: q.k - damp F/s, so its (keys x queries) product is not taken again)
               float f = p;
-              if (G == 1 && has_h0) f = DAMP ? fmaf(dmv[t], p, l0t[4 * a + t]) : p + l0t[4 * a + t];
+              if (whole) f = DAMP ? fmaf(dmv[t], p, l0t[4 * a + t]) : p + l0t[4 * a + t];
               fw[crow(4 * a + t, h) * LDF + n] = f;
               p += sel[4 * a + t];
             }
@@ -1431,7 +1434,7 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
           fs[4 * a + 3] = f4.w;
         }
         if constexpr (DAMP) {
-          if (G > 1 || !has_h0) {
+          if (!whole) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) fs[i] *= damp;
           }
@@ -1440,7 +1443,7 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
 #pragma unroll
         for (int g = 0; g < G; ++g) {
           f32x16 lg = fs;   // the product accumulates onto -F: lg = q.k - F/s
-          if (G > 1 || !has_h0) {   // (else head 0's came through LDS whole)
+          if (!whole) {   // (else head 0's came through LDS whole)
 #pragma unroll
             for (int s = 0; s < NS; ++s) lg = OP::mma(OP::ld_std(sK[buf][g], LDK, n, h, s), qf[g][s], lg);
           }
@@ -4299,8 +4302,8 @@ int forward_impl(const FwdCall& c) {
   elem* vt = static_cast<elem*>(c.ws);
   const int dtype = sizeof(elem) == 2 ? SA_DTYPE_BF16 : SA_DTYPE_F32;
   int G = auto_group(dtype, D, c.H, c.group, false);
-  if constexpr (sizeof(elem) == 2 && D == 64) {
-    if (c.group <= 0 && G == 2) G = fwd64_group(c.nseq, c.H, c.Tq, device_cus());
+  if constexpr (sizeof(elem) == 2 && D <= 64) {
+    if (c.group <= 0 && G >= 2) G = fwd64_group(c.nseq, c.H, c.Tq, device_cus());
   }
   // V^T for fwd_kernel (fwd64_kernel, bf16 at head dim 64 with G <= 2, reads the V rows transposed
   // from LDS)

@@ -3,7 +3,7 @@ bf16-valued inputs (reference tests/test_selective_kernels.py:141-172, 203-242).
 
 The launch policy picks the instance from (head_dim, heads, group, bwd_group); with H = 4:
 
-    forward   head_dim 16 / 32 (run at 32): group 1 -> 1 head per wavefront, 2 -> 2, 4 / None -> 4
+    forward   head_dim 16 / 32 (run at 32): group 1 -> 1 head per wavefront, 2 -> 2, 4 -> 4, None as at 64
               head_dim 64:                  group 1 -> 1, 2 -> 2, 4 -> 4, None -> 2, or 1 when
                                             the two-head grid fills the CUs only once (the same bits:
                                             test_fwd64_one_or_two_heads_per_wavefront_same_bits; an
@@ -217,3 +217,16 @@ def test_fwd64_prefill_widths_same_bits(cuda):
     for out, state in runs[1:]:
         assert torch.equal(out, runs[0][0])
         assert torch.equal(state, runs[0][1])
+
+
+@pytest.mark.parametrize("heads,seq", [(2, 33), (4, 700), (6, 257), (12, 1100)])
+def test_d32_widths_same_bits(cuda, heads, seq):
+    """At head dim 32 the forward's width follows the grid (group=None): one, two and, where they divide the
+    heads, four heads per wavefront give the same bits, head 0 included, damped or not."""
+    q, k, v, _ = _inputs(2, heads, seq, 32, seed=heads + seq)
+    qd, kd, vd = (x.to(cuda, torch.bfloat16) for x in (q, k, v))
+    for kw in ({}, {"damp": "sqrt", "train_len": seq // 2}):
+        runs = [kernels.selective_attention_forward(qd, kd, vd, group=g, return_aux=True, **kw) for g in (1, 2, 4, None)]
+        for out, aux in runs[1:]:
+            assert torch.equal(out, runs[0][0])
+            assert all(torch.equal(aux[n], runs[0][1][n]) for n in aux)
