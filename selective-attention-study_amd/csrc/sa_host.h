@@ -22,6 +22,7 @@ namespace sa_host {
 constexpr int TILE = 32;      // tile edge and carry checkpoint spacing (queries)
 constexpr int NTHREADS = 256;
 constexpr int NWAVES = 4;
+constexpr int REACH_MIN_KEYS = 1024;   // keys from which a launch looks for tiles to leave out (below)
 
 // Event timing of the main kernels, for measurement tools (sa_timing_enable / sa_timing_read).
 // Off by default; when on, each timed launch is bracketed by a pair of HIP events recorded on the
@@ -105,6 +106,19 @@ inline int fwd64_group(int64_t nseq, int64_t heads, int64_t tq, int cus) {
   return workgroups > 2 * (int64_t)cus ? 2 : 1;
 }
 
+// Whether the fp32 kernels of head dim <= 64 split each tile row between the wavefronts of a workgroup
+// (fwd_split_kernel and its backward counterparts): where the unsplit grid leaves half the CUs without a
+// workgroup, or three quarters from REACH_MIN_KEYS keys on, where the unsplit kernels leave tiles out; past
+// SPLIT_MAX_T keys what they leave out can outweigh any split. Measured (fwd + bwd, us, split / unsplit,
+// B x H x T, N(0,1) inputs): 1x4x512 159 / 361 (16 workgroups), 2x12x129 126 / 241 (48), 4x8x512 300 / 368
+// (128), 1x1x2048 292 / 298 (16), at head dim 32 1x8x1024 140 / 276 (64); beyond the rule 8x8x512 561 / 384
+// (256), 2x8x1024 507 / 405 (128), 1x8x2048 917 / 409 (128): the split reads every operand four times.
+constexpr int64_t SPLIT_MAX_T = 2048;
+inline bool split_f32_grid(int64_t nseq, int64_t heads, int64_t tq, int64_t tk, int cus) {
+  const int64_t workgroups = nseq * heads * cdiv(cdiv(tq, TILE), NWAVES);
+  return tk <= SPLIT_MAX_T && workgroups <= (tk < REACH_MIN_KEYS ? cus / 2 : cus / 4);
+}
+
 // The dispatch order of the query-side backward kernel at head dim 64 (work_order_block): the number
 // of its workgroups an XCD runs at once when a launch holds 2.7 to 3 of them per slot, where the
 // order that follows each XCD's first round with its shortest workgroups balances the slots better
@@ -179,7 +193,6 @@ inline BwdLayout bwd_layout(int64_t nseq, int64_t heads, int64_t t, int64_t D, i
 // carry weight (sa_reach_bytes): without it every causal tile is computed. Forward: kn, one bound on
 // the key norms per head and key tile; kt, the least selection total of each key tile. A launch looks for tiles to skip only from REACH_MIN_KEYS keys
 // on: below, a query block has few tiles that a history can have outgrown.
-constexpr int REACH_MIN_KEYS = 1024;
 constexpr int REACH_MASK_WORDS = 128;   // a workgroup's tile mask: its newest 64 * 128 key tiles
 
 // Backward: per head and QSTAT_ROWS rows the largest query norm and the least lse; per head group and 128

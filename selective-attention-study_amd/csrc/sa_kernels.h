@@ -3882,6 +3882,445 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// fp32 storage, small grids: the four wavefronts of a workgroup share one 32-row tile (of queries, or of
+// keys on the key side) and split the other axis between them, every fourth tile each.
+//
+// An fp32 tile is a chain of matrix products at the fp32 rate (64 cycles per 32x32x2 instruction, 96 of
+// them per tile in the forward, 192 on the key side: 2.6 and 5.1 us at the least), and a launch lasts as long
+// as its longest wavefront's sweep; with a wavefront per tile row a grid of this size leaves most of the
+// chip's SIMDs idle meanwhile. Split four ways the longest sweep is a quarter and the grid four times as
+// large, at four times the operand reads, which come from L2: nothing is shared through LDS, so nothing is
+// staged there and the tile loops need no barrier but the key side's one per four tiles (below). The
+// contraction runs over the head dim in the order that gives each lane contiguous elements (lane half h
+// takes elements [h D/2, (h+1) D/2)), so a lane's rows load as 16-byte pieces; the products that contract
+// over rows read the untransposed matrices a row per half-wavefront, whole 128-byte segments, so no
+// transposed copies are made. Measured at B=1 H=4 T=512 D=64: forward 72 -> 26 us, key side 122 -> 40, query side
+// 116 -> 35.
+//
+// Taken by split_f32_grid.
+
+// A lane's half of its row (lane n: row row0 + n) of a row-major fp32 matrix, rows past the resource zero.
+template <int D>
+struct HalfRow {
+  float f[D / 2];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int ld, int row, int h) {
+#pragma unroll
+    for (int c = 0; c < D / 8; ++c) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(rs, (row * ld + h * (D / 2) + 4 * c) * 4, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[4 * c + e] = __uint_as_float(x[e]);
+    }
+  }
+};
+// c += A B^T over the head dim, a and b the lanes' rows of A and B.
+template <int D>
+__device__ __forceinline__ f32x16 mma_rows(const HalfRow<D>& a, const HalfRow<D>& b, f32x16 c) {
+#pragma unroll
+  for (int s = 0; s < D / 2; ++s) c = OpF32::mma(a.f[s], b.f[s], c);
+  return c;
+}
+// acc[db] (D x columns) += Y^T X: Y the 32 rows from row0 of a row-major matrix, X a C-layout tile (rows of Y
+// x columns).
+template <int D>
+__device__ __forceinline__ void mma_cols(f32x16 (&acc)[D / 32], __amdgpu_buffer_rsrc_t rs, int ld, int row0, int n, int h,
+                                         const f32x16& x) {
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db) {
+    float y[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      y[s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, ((row0 + crow(s, h)) * ld + db * 32 + n) * 4, 0, 0));
+#pragma unroll
+    for (int s = 0; s < 16; ++s) acc[db] = OpF32::mma(y[s], x[s], acc[db]);
+  }
+}
+// Sums of four wavefronts' (D x 32 columns) C-layout tiles in wavefront order: thread t gets column t / 8,
+// elements [(t mod 8) D/8, +D/8) of the sum. The barrier at the end frees the buffer.
+template <int D>
+__device__ __forceinline__ void sum_tiles(float (*buf)[32 * (D + 4)], const f32x16 (&acc)[D / 32], float scale, int n, int h,
+                                          int wave, int tid, float (&out)[D / 8]) {
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      *reinterpret_cast<float4*>(&buf[wave][n * (D + 4) + db * 32 + 8 * a + 4 * h]) =
+          make_float4(acc[db][4 * a] * scale, acc[db][4 * a + 1] * scale, acc[db][4 * a + 2] * scale,
+                      acc[db][4 * a + 3] * scale);
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    const int at = (tid >> 3) * (D + 4) + (tid & 7) * (D / 8) + 4 * c;
+    float4 x = *reinterpret_cast<const float4*>(&buf[0][at]);
+#pragma unroll
+    for (int w = 1; w < NWAVES; ++w) {
+      const float4 y = *reinterpret_cast<const float4*>(&buf[w][at]);
+      x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+    }
+    out[4 * c] = x.x;
+    out[4 * c + 1] = x.y;
+    out[4 * c + 2] = x.z;
+    out[4 * c + 3] = x.w;
+  }
+  __syncthreads();
+}
+
+// Forward (fwd_kernel's tile work, no damping). grid (ceil(Tq/32), nseq * H), the longest sweeps first; the
+// wavefronts' partial softmax sums merge at the end.
+template <int D>
+__global__ __launch_bounds__(NTHREADS, 1) void fwd_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ carry,
+    float* __restrict__ out, float* __restrict__ rmax, float* __restrict__ rden, float* __restrict__ y, Strides ys, int H,
+    int Tq, int Tk, Strides qs, Strides ks, Strides vs, int q_off, int exempt, float scale) {
+  constexpr int DB = D / 32, LDF = TILE + 4;
+  __shared__ __attribute__((aligned(16))) float sF[NWAVES][TILE * LDF];
+  __shared__ __attribute__((aligned(16))) float sSum[NWAVES][32 * (D + 4)];
+  __shared__ float sM[NWAVES][TILE], sL[NWAVES][TILE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  const int n = lane & 31, h = lane >> 5;
+  const int b = blockIdx.y / H, hh = blockIdx.y % H;
+  const bool whole = hh == 0;   // head 0's adjusted logits go through LDS whole (see fwd_kernel)
+  const int NBq = (Tq + TILE - 1) / TILE, NKT = (Tk + TILE - 1) / TILE;
+  const int rb = gridDim.x - 1 - blockIdx.x;
+  const int q_rel = rb * TILE + n, q_abs = q_off + q_rel;
+  const int end = min((q_off + rb * TILE + TILE - 1) / TILE + 1, NKT);
+  auto head = [&](const float* p, const Strides& s, int x, int rows) {
+    return rsrc(p + s.at(b, x), (int64_t)rows * s.row * 4);
+  };
+  const __amdgpu_buffer_rsrc_t rs_k = head(k, ks, hh, Tk), rs_k0 = head(k, ks, 0, Tk), rs_v = head(v, vs, hh, Tk);
+  HalfRow<D> qf, q0f;
+  qf.load(head(q, qs, hh, Tq), qs.row, q_rel, h);
+  q0f.load(head(q, qs, 0, Tq), qs.row, q_rel, h);
+  const float* crow_ = carry + ((int64_t)b * NBq + rb) * Tk;
+  const float sl2 = scale * LOG2E, neg_inv_scale = -1.f / scale;
+  float m = -INFINITY, l = 0.f;
+  f32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o[db] = zero16();
+
+  for (int kt = end - 1 - wave; kt >= 0; kt -= NWAVES) {
+    const int kbase = kt * TILE;
+    const bool edge = (kbase + TILE - 1 >= q_off + rb * TILE) || (kbase + TILE > Tk) || kbase < exempt;
+    HalfRow<D> kf, k0f;
+    kf.load(rs_k, ks.row, kbase + n, h);
+    if (!whole) k0f.load(rs_k0, ks.row, kbase + n, h);
+    const int jk = kbase + n;
+    float run = jk < Tk ? crow_[jk] * neg_inv_scale : 0.f;
+    const f32x16 l0t = whole ? mma_rows<D>(q0f, kf, zero16()) : mma_rows<D>(q0f, k0f, zero16());
+    f32x16 sel;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sel[i] = __builtin_amdgcn_fmed3f(-l0t[i], -3.0e38f, 0.f);
+    if (edge) {
+      const int thr = jk >= exempt ? jk - (q_off + rb * TILE) - 4 * h : 32;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sel[i] = crow(i, 0) > thr ? sel[i] : 0.f;
+    }
+    float* fw = sF[wave];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const Halves g = halves(((sel[4 * a] + sel[4 * a + 1]) + sel[4 * a + 2]) + sel[4 * a + 3]);
+      float p = (h == 0) ? run : run + g.lo;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        fw[crow(4 * a + t, h) * LDF + n] = whole ? p + l0t[4 * a + t] : p;
+        p += sel[4 * a + t];
+      }
+      run = (run + g.lo) + g.hi;
+    }
+    lds_wave_sync();
+    f32x16 lg;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const float4 f4 = *reinterpret_cast<const float4*>(&fw[n * LDF + 8 * a + 4 * h]);
+      lg[4 * a] = f4.x;
+      lg[4 * a + 1] = f4.y;
+      lg[4 * a + 2] = f4.z;
+      lg[4 * a + 3] = f4.w;
+    }
+    lds_wave_sync();   // (the next tile's writes follow)
+    if (!whole) lg = mma_rows<D>(kf, qf, lg);
+    if (edge) {
+      const int thr = min(q_abs, Tk - 1) - kbase - 4 * h;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lg[i] = crow(i, 0) <= thr ? lg[i] : -INFINITY;
+    }
+    float zmax = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zmax = fmaxf(zmax, lg[i]);
+    const Halves zh = halves(zmax);
+    const float m_new = fmaxf(m, fmaxf(zh.lo, zh.hi) * sl2);
+    if (__any(m_new > m)) {
+      const float alpha = (m_new == -INFINITY) ? 1.f : fast_exp2(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+    }
+    const float mu = (m == -INFINITY) ? 0.f : m;
+    float psum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float p = fast_exp2(fmaf(lg[i], sl2, -mu));
+      lg[i] = p;
+      psum += p;
+    }
+    l += psum;
+    mma_cols<D>(o, rs_v, vs.row, kbase, n, h, lg);
+  }
+
+  // merge: the row's maximum over the wavefronts, then their sums relative to it
+  const Halves lh = halves(l);
+  if (h == 0) {
+    sM[wave][n] = m;
+    sL[wave][n] = lh.lo + lh.hi;
+  }
+  __syncthreads();
+  float M = sM[0][n];
+#pragma unroll
+  for (int w = 1; w < NWAVES; ++w) M = fmaxf(M, sM[w][n]);
+  const float a = m == -INFINITY ? 0.f : fast_exp2(m - M);   // (a wavefront without a tile: no weight)
+  // (a row whose every key weighs -inf or NaN: as the unsplit kernel, nothing to rescale by)
+  float part[D / 8];
+  sum_tiles<D>(sSum, o, m == M ? 1.f : a, n, h, wave, tid, part);
+  const int qn = tid >> 3, row_rel = rb * TILE + qn;
+  float Mq = sM[0][qn];
+#pragma unroll
+  for (int w = 1; w < NWAVES; ++w) Mq = fmaxf(Mq, sM[w][qn]);
+  float ltot = 0.f;
+#pragma unroll
+  for (int w = 0; w < NWAVES; ++w) {
+    const float mw = sM[w][qn];
+    ltot += sL[w][qn] * (mw == Mq ? 1.f : mw == -INFINITY ? 0.f : fast_exp2(mw - Mq));
+  }
+  if (row_rel >= Tq) return;
+  const float inv = 1.f / ltot;
+  const int64_t row = (int64_t)blockIdx.y * Tq + row_rel;
+  const int d0 = (tid & 7) * (D / 8);
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    const float4 x = make_float4(part[4 * c] * inv, part[4 * c + 1] * inv, part[4 * c + 2] * inv, part[4 * c + 3] * inv);
+    *reinterpret_cast<float4*>(out + row * D + d0 + 4 * c) = x;
+    if (y) *reinterpret_cast<float4*>(y + ys.at(b, hh) + (int64_t)row_rel * ys.row + d0 + 4 * c) = x;
+  }
+  if ((tid & 7) == 0) {
+    rmax[row] = Mq;
+    rden[row] = ltot;
+  }
+}
+
+// Key side (bwd_kv_kernel's tile work). grid (ceil(T/32), nseq * H); step t takes the four query tiles
+// NB - 1 - 4t - w, one per wavefront w. The selection suffix entering a wavefront's tile is the one entering
+// the step plus the sums of dz of the later wavefronts' tiles, exchanged through LDS with the step's barrier.
+template <int D>
+__global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
+    Strides qs, Strides ks, Strides vs, Strides dos, const float* __restrict__ lse, const float* __restrict__ ndbar,
+    const float* __restrict__ carry, float* __restrict__ ucheck, float* __restrict__ dk0h, float* __restrict__ dk0x,
+    GradView dkv, GradView dvv, int nseq, int H, int T, int64_t ldt, int exempt, float scale) {
+  constexpr int DB = D / 32;
+  __shared__ __attribute__((aligned(16))) float sSum[NWAVES][32 * (D + 4)];
+  __shared__ float sU[2][NWAVES][TILE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  const int n = lane & 31, h = lane >> 5;
+  const int b = blockIdx.y / H, hh = blockIdx.y % H;
+  const bool has_h0 = hh == 0;
+  const int NB = (T + TILE - 1) / TILE;
+  const int kt = blockIdx.x, key0 = kt * TILE, j = key0 + n;
+  auto head = [&](const float* p, const Strides& s, int x) { return rsrc(p + s.at(b, x), (int64_t)T * s.row * 4); };
+  const __amdgpu_buffer_rsrc_t rs_q = head(q, qs, hh), rs_q0 = head(q, qs, 0), rs_do = head(dout, dos, hh);
+  HalfRow<D> kf, k0f, vf;   // B operands: lane = key
+  kf.load(head(k, ks, hh), ks.row, j, h);
+  k0f.load(head(k, ks, 0), ks.row, j, h);
+  vf.load(head(v, vs, hh), vs.row, j, h);
+  f32x16 dkt[DB], dvt[DB], dk0t[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) {
+    dkt[db] = zero16();
+    dvt[db] = zero16();
+    dk0t[db] = zero16();
+  }
+  float* uplane = ucheck + ((int64_t)hh * nseq + b) * utri_floats(NB);
+  const float* carry_col = carry + (int64_t)b * NB * T + min(j, T - 1);
+  const float* lse_row = lse + (int64_t)blockIdx.y * ldt;
+  const float* ndb_row = ndbar + (int64_t)blockIdx.y * ldt;
+  const float sl2 = scale * LOG2E, neg_inv_scale = -1.f / scale;
+  const int ntiles = NB - kt;
+  float ucarry = 0.f;
+  for (int t = 0; 4 * t < ntiles; ++t) {
+    const int qb = NB - 1 - 4 * t - wave;
+    const bool mine = qb >= kt;
+    f32x16 dz = zero16();
+    uint32_t gate = 0;
+    const int qbase = qb * TILE;
+    if (mine) {
+      const bool edge = (qbase <= key0 + TILE - 1) || key0 < exempt;
+      const TileMasks mk(j, qbase, T, exempt, h);
+      HalfRow<D> rows;
+      rows.load(rs_q0, qs.row, qbase + n, h);
+      const float hist = j < T ? carry_col[(int64_t)qb * T] : 0.f;
+      const f32x16 l0 = mma_rows<D>(rows, k0f, zero16());
+      f32x16 lg;
+      selection_tile<false>(l0, hist * neg_inv_scale, h, edge, mk, gate, lg);
+      if (has_h0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) lg[i] = l0[i] + lg[i];
+      } else {
+        rows.load(rs_q, qs.row, qbase + n, h);
+        lg = mma_rows<D>(rows, kf, lg);
+      }
+      rows.load(rs_do, dos.row, qbase + n, h);
+      const f32x16 dp = mma_rows<D>(rows, vf, rows16(ndb_row + qbase, h));   // dO.v - dbar
+      f32x16 pr;
+      p_dz_tile_r(lg, dp, rows16(lse_row + qbase, h), sl2, edge, mk, pr, dz);
+      mma_cols<D>(dvt, rs_do, dos.row, qbase, n, h, pr);
+      if (!has_h0) mma_cols<D>(dkt, rs_q, qs.row, qbase, n, h, dz);
+    }
+    float tot = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) tot += dz[i];
+    tot += xor32(tot);
+    if (h == 0) sU[t & 1][wave][n] = tot;
+    __syncthreads();   // (the buffer is written again two steps on, past the next step's barrier)
+    float u_in = ucarry;
+#pragma unroll
+    for (int w = 0; w < NWAVES; ++w) {
+      const float x = sU[t & 1][w][n];
+      if (w < wave) u_in += x;
+      ucarry += x;
+    }
+    if (mine) {
+      if (h == 0 && j < T) uplane[utri_row(qb) + j] = u_in;
+      f32x16 gp;
+      gpath_tile(dz, u_in, gate, h, gp);
+      if (has_h0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dz[i] += gp[i];
+        mma_cols<D>(dkt, rs_q, qs.row, qbase, n, h, dz);
+      } else {
+        mma_cols<D>(dk0t, rs_q0, qs.row, qbase, n, h, gp);
+      }
+    }
+  }
+  const int jn = key0 + (tid >> 3), d0 = (tid & 7) * (D / 8);
+  float part[D / 8];
+  auto quad = [&](int c) { return make_float4(part[4 * c], part[4 * c + 1], part[4 * c + 2], part[4 * c + 3]); };
+  sum_tiles<D>(sSum, dvt, 1.f, n, h, wave, tid, part);
+#pragma unroll
+  for (int c = 0; c < DB; ++c)
+    if (jn < T) store_grad4(dvv, b, hh, jn, d0 + 4 * c, quad(c));
+  sum_tiles<D>(sSum, dkt, scale, n, h, wave, tid, part);
+#pragma unroll
+  for (int c = 0; c < DB; ++c) {
+    if (jn >= T) continue;
+    if (has_h0 && H > 1) *reinterpret_cast<float4*>(dk0h + ((int64_t)b * T + jn) * D + d0 + 4 * c) = quad(c);
+    else store_grad4(dkv, b, hh, jn, d0 + 4 * c, quad(c));
+  }
+  if (has_h0) return;
+  sum_tiles<D>(sSum, dk0t, scale, n, h, wave, tid, part);
+#pragma unroll
+  for (int c = 0; c < DB; ++c)
+    if (jn < T)
+      *reinterpret_cast<float4*>(dk0x + ((int64_t)(hh - 1) * nseq * T + (int64_t)b * T + jn) * D + d0 + 4 * c) = quad(c);
+}
+
+// Query side (bwd_dq_kernel's tile work). grid (ceil(T/32), nseq * H), the longest sweeps first.
+template <int D>
+__global__ __launch_bounds__(NTHREADS, 1) void bwd_dq_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
+    Strides qs, Strides ks, Strides vs, Strides dos, const float* __restrict__ lse, const float* __restrict__ ndbar,
+    const float* __restrict__ carry, const float* __restrict__ ucheck, float* __restrict__ dq0h, float* __restrict__ dq0x,
+    GradView dqv, int nseq, int H, int T, int64_t ldt, int exempt, float scale) {
+  constexpr int DB = D / 32, LDZ = TILE + 4;
+  __shared__ __attribute__((aligned(16))) float sZ[NWAVES][TILE * LDZ];
+  __shared__ __attribute__((aligned(16))) float sSum[NWAVES][32 * (D + 4)];
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  const int n = lane & 31, h = lane >> 5;
+  const int b = blockIdx.y / H, hh = blockIdx.y % H;
+  const bool has_h0 = hh == 0;
+  const int NB = (T + TILE - 1) / TILE;
+  const int qb = gridDim.x - 1 - blockIdx.x, qbase = qb * TILE;
+  auto head = [&](const float* p, const Strides& s, int x) { return rsrc(p + s.at(b, x), (int64_t)T * s.row * 4); };
+  const __amdgpu_buffer_rsrc_t rs_k = head(k, ks, hh), rs_k0 = head(k, ks, 0), rs_v = head(v, vs, hh);
+  HalfRow<D> qa, q0a, doa;   // A operands: lane = query row
+  qa.load(head(q, qs, hh), qs.row, qbase + n, h);
+  q0a.load(head(q, qs, 0), qs.row, qbase + n, h);
+  doa.load(head(dout, dos, hh), dos.row, qbase + n, h);
+  const f32x16 lse_r = rows16(lse + (int64_t)blockIdx.y * ldt + qbase, h);
+  const f32x16 ndb_r = rows16(ndbar + (int64_t)blockIdx.y * ldt + qbase, h);
+  const float* carry_row = carry + ((int64_t)b * NB + qb) * T;
+  const float* urow = ucheck + ((int64_t)hh * nseq + b) * utri_floats(NB) + utri_row(qb);
+  const float sl2 = scale * LOG2E, neg_inv_scale = -1.f / scale;
+  f32x16 dq[DB], dq0[DB];   // (D x queries)
+#pragma unroll
+  for (int db = 0; db < DB; ++db) {
+    dq[db] = zero16();
+    dq0[db] = zero16();
+  }
+  // acc (D x queries) += K^T X^T: X a (queries x keys) C-layout tile, transposed through the wavefront's LDS
+  // rows into the (keys x queries) layout that mma_cols takes
+  auto acc_xk = [&](f32x16 (&acc)[DB], const f32x16& x, __amdgpu_buffer_rsrc_t rs, int kbase) {
+    float* z = sZ[wave];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z[crow(i, h) * LDZ + n] = x[i];
+    lds_wave_sync();
+    const f32x16 xt = rows16(z + n * LDZ, h);
+    lds_wave_sync();
+    mma_cols<D>(acc, rs, ks.row, kbase, n, h, xt);
+  };
+  for (int kt = wave; kt <= qb; kt += NWAVES) {
+    const int kbase = kt * TILE, j = kbase + n;
+    const bool edge = (kbase + TILE - 1 >= qbase) || (kbase + TILE > T) || kbase < exempt;
+    const TileMasks mk(j, qbase, T, exempt, h);
+    HalfRow<D> rows;
+    rows.load(rs_k0, ks.row, j, h);
+    const float hist = j < T ? carry_row[j] : 0.f, uin = j < T ? urow[j] : 0.f;
+    const f32x16 l0 = mma_rows<D>(q0a, rows, zero16());
+    f32x16 lg;
+    uint32_t gate;
+    selection_tile<false>(l0, hist * neg_inv_scale, h, edge, mk, gate, lg);
+    if (has_h0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lg[i] = l0[i] + lg[i];
+    } else {
+      rows.load(rs_k, ks.row, j, h);
+      lg = mma_rows<D>(qa, rows, lg);
+    }
+    rows.load(rs_v, vs.row, j, h);
+    const f32x16 dp = mma_rows<D>(doa, rows, ndb_r);
+    f32x16 pr, dz, gp;
+    p_dz_tile_r(lg, dp, lse_r, sl2, edge, mk, pr, dz);
+    gpath_tile(dz, uin, gate, h, gp);
+    if (has_h0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dz[i] += gp[i];
+      acc_xk(dq, dz, rs_k, kbase);
+    } else {
+      acc_xk(dq, dz, rs_k, kbase);
+      acc_xk(dq0, gp, rs_k0, kbase);
+    }
+  }
+  const int rn = qbase + (tid >> 3), d0 = (tid & 7) * (D / 8);
+  float part[D / 8];
+  const bool sums = has_h0 && H > 1;   // head 0's unscaled sums, which the other heads' shares join
+  sum_tiles<D>(sSum, dq, sums ? 1.f : scale, n, h, wave, tid, part);
+#pragma unroll
+  for (int c = 0; c < DB; ++c) {
+    if (rn >= T) continue;
+    const float4 x = make_float4(part[4 * c], part[4 * c + 1], part[4 * c + 2], part[4 * c + 3]);
+    if (sums) *reinterpret_cast<float4*>(dq0h + ((int64_t)b * T + rn) * D + d0 + 4 * c) = x;
+    else store_grad4(dqv, b, hh, rn, d0 + 4 * c, x);
+  }
+  if (has_h0) return;
+  sum_tiles<D>(sSum, dq0, 1.f, n, h, wave, tid, part);
+#pragma unroll
+  for (int c = 0; c < DB; ++c)
+    if (rn < T)
+      *reinterpret_cast<float4*>(dq0x + ((int64_t)(hh - 1) * nseq * T + (int64_t)b * T + rn) * D + d0 + 4 * c) =
+          make_float4(part[4 * c], part[4 * c + 1], part[4 * c + 2], part[4 * c + 3]);
+}
+
 // The gradient epilogue. Workgroups [0, main_blocks): head 0's gradients, its own fp32 sums plus the other
 // groups' shares, summed slot after slot in group order (so every run adds the same values in the same
 // order), (b, t, D) contiguous, four elements per thread, to the caller's views; nslots slots of total4
@@ -4305,6 +4744,20 @@ int forward_impl(const FwdCall& c) {
   if constexpr (sizeof(elem) == 2 && D <= 64) {
     if (c.group <= 0 && G >= 2) G = fwd64_group(c.nseq, c.H, c.Tq, device_cus());
   }
+  if constexpr (sizeof(elem) == 4 && D <= 64) {
+    if (c.damp_mode == 0 && split_f32_grid(c.nseq, c.H, c.Tq, c.Tk, device_cus())) {
+      FwdCall sc = c;
+      sc.kn = sc.kt = nullptr;   // (every tile is visited)
+      const int rc = run_selection<OP, D>(sc, c.st);
+      if (rc) return rc;
+      TimedLaunch timed(SA_KERNEL_FORWARD, c.st);
+      hipLaunchKernelGGL((fwd_split_kernel<D>), dim3((unsigned)cdiv(c.Tq, TILE), (unsigned)(c.nseq * c.H)), dim3(NTHREADS),
+                         0, c.st, static_cast<const float*>(c.q), static_cast<const float*>(c.k),
+                         static_cast<const float*>(c.v), c.carry, c.out, c.rmax, c.rden, static_cast<float*>(c.y), c.ys, c.H,
+                         c.Tq, c.Tk, c.qs, c.ks, c.vs, c.q_off, c.exempt, c.scale);
+      return launch_status();
+    }
+  }
   // V^T for fwd_kernel (fwd64_kernel, bf16 at head dim 64 with G <= 2, reads the V rows transposed
   // from LDS)
   if (!(sizeof(elem) == 2 && D == 64 && G <= 2))
@@ -4446,7 +4899,9 @@ int backward_impl(const BwdCall& c) {
 
   // bf16 at head dim 64 the backward kernels read their Q, dO and K rows transposed from LDS
   // (bwd_kv64_kernel, bwd_dq64_kernel): no transposed copies
-  if constexpr (!(sizeof(elem) == 2 && D == 64)) {
+  bool split = false;
+  if constexpr (sizeof(elem) == 4 && D <= 64) split = split_f32_grid(nseq, H, T, T, device_cus());
+  if (!(sizeof(elem) == 2 && D == 64) && !split) {
     launch_transpose<elem, D>(q, qt, T, ldt, c.qs, H, R, st);
     launch_transpose<elem, D>(dout, dot, T, ldt, c.dos, H, R, st);
     launch_transpose<elem, D>(k, kt, T, ldt, c.ks, H, R, st);
@@ -4454,7 +4909,7 @@ int backward_impl(const BwdCall& c) {
   BwdReach reach{};
   reach.nseg = (int)cdiv(T, QSTAT_ROWS);
   reach.nkg = (int)cdiv(T, NWAVES * TILE);
-  if (c.reach) {
+  if (c.reach && !split) {
     const BwdReachLayout RL = bwd_reach_layout(nseq, H, T, D);
     reach.qstat = reinterpret_cast<float2*>(c.reach + RL.qstat);
     reach.hi = reinterpret_cast<int*>(c.reach + RL.hi);
@@ -4469,6 +4924,22 @@ int backward_impl(const BwdCall& c) {
 #define SA_LAUNCH_BWD(GG) launch_bwd<OP, D, GG>(c, qt, kt, dot, lse, dbar, ucheck, dq0h, dk0h, dq0x, dk0x, ldt, reach)
   if constexpr (sizeof(elem) == 2 && D <= 32) {
     rc = (G == 2) ? SA_LAUNCH_BWD(2) : SA_LAUNCH_BWD(1);
+  } else if (split) {
+    if constexpr (sizeof(elem) == 4 && D <= 64) {
+      const dim3 grid((unsigned)cdiv(T, TILE), (unsigned)R);
+      const int gf32 = c.grad_dtype == SA_DTYPE_F32;
+      const float* v = static_cast<const float*>(c.v);
+      {
+        TimedLaunch timed(SA_KERNEL_BACKWARD, st);
+        hipLaunchKernelGGL((bwd_kv_split_kernel<D>), grid, dim3(NTHREADS), 0, st, q, k, v, dout, c.qs, c.ks, c.vs, c.dos, lse,
+                           dbar, c.carry, ucheck, dk0h, dk0x, GradView{c.dk, c.dks, gf32}, GradView{c.dv, c.dvs, gf32}, nseq,
+                           H, T, ldt, c.exempt, c.scale);
+      }
+      TimedLaunch timed(SA_KERNEL_BACKWARD_DQ, st);
+      hipLaunchKernelGGL((bwd_dq_split_kernel<D>), grid, dim3(NTHREADS), 0, st, q, k, v, dout, c.qs, c.ks, c.vs, c.dos, lse,
+                         dbar, c.carry, ucheck, dq0h, dq0x, GradView{c.dq, c.dqs, gf32}, nseq, H, T, ldt, c.exempt, c.scale);
+      rc = launch_status();
+    }
   } else {
     rc = SA_LAUNCH_BWD(1);
   }

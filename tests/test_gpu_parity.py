@@ -427,3 +427,34 @@ def test_chunked_prefill_unaligned_offsets(cuda, chunk, exempt):
     want = sa_oracle.attention(q.double(), k.double(), v.double(), exempt)
     _close(torch.cat(outs, dim=2).cpu(), want, 2e-5, 2e-5, "chunked out")
     _close(state.cpu(), sa_oracle.selection_totals(q.double(), k.double(), exempt), 2e-4, 2e-5, "state")
+
+
+@pytest.mark.parametrize("heads,seq,head_dim,exempt,chunk", [
+    (1, 1, 64, 1, 0), (2, 31, 64, 1, 0), (3, 33, 32, 16, 0), (1, 97, 64, 40, 0), (4, 128, 32, 1, 0), (2, 129, 64, 3, 0),
+    (2, 513, 64, 1, 0), (1, 1500, 64, 1, 0), (2, 300, 64, 1, 45), (1, 2048, 32, 16, 33)])
+def test_fp32_split_tiles_match_oracle(cuda, heads, seq, head_dim, exempt, chunk):
+    """Small fp32 grids, whose kernels split each tile row between a workgroup's wavefronts: fewer tiles than
+    wavefronts, remainders of four tiles, odd lengths, one-head sequences, a chunk at an odd offset."""
+    print(f"case fp32 split {heads} {seq} {head_dim} {exempt} {chunk}", flush=True)
+    q, k, v = _qkv(1, heads, seq, head_dim, seed=seq)
+    w = torch.randn(1, heads, seq, head_dim, generator=torch.Generator().manual_seed(seq))
+    qd, kd, vd = (x.to(cuda).requires_grad_(True) for x in (q, k, v))
+    qr, kr, vr = (x.double().requires_grad_(True) for x in (q, k, v))
+    want = sa_oracle.attention(qr, kr, vr, exempt=exempt)
+    want.backward(w.double())
+    if chunk:
+        state = torch.zeros(1, seq, device=cuda)
+        with torch.no_grad():
+            got = [kernels.selective_attention_prefill(qd[:, :, a:b], kd[:, :, :b], vd[:, :, :b], state, a, exempt=exempt)
+                   for a, b in ((0, seq - chunk), (seq - chunk, seq))]
+        torch.testing.assert_close(torch.cat(got, 2).double().cpu(), want.detach(), rtol=0, atol=2e-5)
+        return
+    out = kernels.selective_attention(qd, kd, vd, exempt=exempt)
+    grads = torch.autograd.grad(out, (qd, kd, vd), w.to(cuda))
+    torch.testing.assert_close(out.detach().double().cpu(), want.detach(), rtol=0, atol=2e-5)
+    for a, b in zip(grads, (qr, kr, vr)):
+        torch.testing.assert_close(a.double().cpu(), b.grad, rtol=5e-4, atol=5e-5)
+    again = kernels.selective_attention(qd, kd, vd, exempt=exempt)
+    assert torch.equal(out, again)
+    for a, b in zip(grads, torch.autograd.grad(again, (qd, kd, vd), w.to(cuda))):
+        assert torch.equal(a, b)
