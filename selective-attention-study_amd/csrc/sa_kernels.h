@@ -1968,7 +1968,7 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
 // TB/s), 33 us with one of them, 39 with 16.
 
 template <class OP, int D>
-__global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 && D <= 64 ? 4 : 1)) void bwd_rowprep_kernel(
+__global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 64 ? 4 : 2) : 1)) void bwd_rowprep_kernel(
     const typename OP::elem* __restrict__ q, const typename OP::elem* __restrict__ k,
     const typename OP::elem* __restrict__ v, const typename OP::elem* __restrict__ dout, Strides qs, Strides ks,
     Strides vs, Strides dos, int H, int T, const float* __restrict__ out, const float* __restrict__ rmax,
@@ -2088,13 +2088,19 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 && D <= 6
   }
   f32x16 dkx[DB], dvx[DB];
   if (xk > 0) {
-    frag kx[NS], vx[NS];   // the first keys and values (B operands: lane = key)
-    const elem* kh = k + ks.at(b, hh);
-    const elem* vh = v + vs.at(b, hh);
+    // the first keys and values (B operands: lane = key), and the rows as A operands (lane = query row). The
+    // fp32 products run over the head dim with lane half h at elements [h D/2, (h+1) D/2), so that both load
+    // as 16-byte pieces.
+    const elem* kh = k + ks.at(b, hh) + (int64_t)min(n, T - 1) * ks.row;   // (columns from xk on are masked)
+    const elem* vh = v + vs.at(b, hh) + (int64_t)min(n, T - 1) * vs.row;
+    constexpr int PIECES = sizeof(elem) == 2 ? NS : D / 8;
+    constexpr int STEP = sizeof(elem) == 2 ? 16 : 4;   // elements between a lane's pieces
+    const int at = sizeof(elem) == 2 ? 8 * h : h * (D / 2);
+    uint4 kx[PIECES], vx[PIECES];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      kx[s] = ld_std_bounded<OP>(kh, ks.row, n, T, h, s);
-      vx[s] = ld_std_bounded<OP>(vh, vs.row, n, T, h, s);
+    for (int s = 0; s < PIECES; ++s) {
+      kx[s] = *reinterpret_cast<const uint4*>(kh + at + STEP * s);
+      vx[s] = *reinterpret_cast<const uint4*>(vh + at + STEP * s);
     }
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
@@ -2102,10 +2108,20 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 && D <= 6
       dvx[db] = zero16();
     }
     lds_wave_sync();
-    auto rfrag = [&](int x, int s) -> frag {   // A operand: lane = query row
+    auto piece = [&](int x, int s) -> uint4 {
       const elem* y = sh.rows[wave][x];
-      if constexpr (TR) return *reinterpret_cast<const frag*>(y + swzq(n, 2 * s + h));
-      else return OP::ld_std(y, LD, n, h, s);
+      if constexpr (TR) return *reinterpret_cast<const uint4*>(y + swzq(n, 2 * s + h));
+      else return *reinterpret_cast<const uint4*>(y + n * LD + at + STEP * s);
+    };
+    auto mma_piece = [&](const uint4& a, const uint4& b4, f32x16 c) -> f32x16 {
+      if constexpr (sizeof(elem) == 2) {
+        return OP::mma(*reinterpret_cast<const frag*>(&a), *reinterpret_cast<const frag*>(&b4), c);
+      } else {
+        c = OP::mma(__uint_as_float(a.x), __uint_as_float(b4.x), c);
+        c = OP::mma(__uint_as_float(a.y), __uint_as_float(b4.y), c);
+        c = OP::mma(__uint_as_float(a.z), __uint_as_float(b4.z), c);
+        return OP::mma(__uint_as_float(a.w), __uint_as_float(b4.w), c);
+      }
     };
     // acc[db] (D x keys) += Y^T X: Y the wavefront's rows, X a (queries x keys) tile
     auto acc_t = [&](f32x16 (&acc)[DB], int which, const f32x16& x) {
@@ -2132,9 +2148,9 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 && D <= 6
     };
     f32x16 p = zero16(), dz = rows16(sRow[wave][1], h);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      p = OP::mma(rfrag(1, s), kx[s], p);
-      dz = OP::mma(rfrag(0, s), vx[s], dz);
+    for (int s = 0; s < PIECES; ++s) {
+      p = mma_piece(piece(1, s), kx[s], p);
+      dz = mma_piece(piece(0, s), vx[s], dz);
     }
     const f32x16 ls = rows16(sRow[wave][0], h);
     const float sl2 = scale * LOG2E;
