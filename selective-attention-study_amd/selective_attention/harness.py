@@ -170,6 +170,7 @@ def perhead_rate(batch: int = 2, heads: int = 16, seq: int = 32768, head_dim: in
     return {"config": f"C5 per-head fwd+bwd, B={batch} H={heads} T={seq} D={head_dim} bf16, k x2 on 10% of keys",
             "ms_per_step": ms, "tflops": tf, "frac_of_peak": tf / PEAK_BF16_TFLOPS,
             "kernel_ms": kernel_ms, "peak_mem_gib": peak,
+            "flop_note": "dense causal products, whether a tile is computed or left out (its weights exact zeros)",
             "roofline": {"bound": "mfma", "kernel": f"{dominant} ({KERNEL_PRODUCTS[dominant]:.0f}*B*H*D*T^2 FLOP)",
                          "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                          "frac": achieved / PEAK_BF16_TFLOPS}}
