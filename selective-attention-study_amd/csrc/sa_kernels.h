@@ -2203,7 +2203,7 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
   }
 }
 
-// (Measured, N(0,1) inputs, B=1 H=16 T=16384 bf16: the key side 1560 -> 195 us, the query side 1510 -> 215 us.)
+// (Measured, N(0,1) inputs, B=1 H=16 T=16384 bf16: the key side 1560 -> 190 us, the query side 1510 -> 203 us.)
 // The last query block on which some key of a wavefront's 32 (from key0) keeps a weight that is not an
 // exact zero, of the blocks up to NB - 1 (the key tile's own block at least): a lane group of 8 probes one
 // block (4 keys per lane), eight blocks at a time; the history never falls, so the blocks past the last
@@ -3911,8 +3911,8 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
 // contraction runs over the head dim in the order that gives each lane contiguous elements (lane half h
 // takes elements [h D/2, (h+1) D/2)), so a lane's rows load as 16-byte pieces; the products that contract
 // over rows read the untransposed matrices a row per half-wavefront, whole 128-byte segments, so no
-// transposed copies are made. Measured at B=1 H=4 T=512 D=64: forward 72 -> 26 us, key side 122 -> 40, query side
-// 116 -> 35.
+// transposed copies are made. Measured at B=1 H=4 T=512 D=64: forward 72 -> 26 us, key side 122 -> 53, query side
+// 116 -> 45.
 //
 // Taken by split_f32_grid.
 
