@@ -84,8 +84,9 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
  * invalid sizes): given a workspace larger by this much, sa_forward and sa_backward leave out the tiles
  * whose softmax weights are exact fp32 zeros because their keys' history has outgrown every logit. The
  * results have the same bits with and without it, but for the gradients of at most 32 exempt keys, which
- * the backward then sums in another order. t: the number of keys. */
-int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim);
+ * the backward then sums in another order. t: the number of keys;
+ * backward: 0 for sa_forward's workspace, 1 for sa_backward's. */
+int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim, int backward);
 
 /*
  * Forward pass, and one chunk of a chunked prefill.

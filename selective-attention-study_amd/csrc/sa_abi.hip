@@ -76,9 +76,9 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
   return align_up(nseq * heads * head_dim * sa_transposed_ld(tk) * es, 256);
 }
 
-int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim) {
+int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim, int backward) {
   if (!valid_dims(nseq, heads, t) || (head_dim != 32 && head_dim != 64 && head_dim != 128)) return -1;
-  return std::max(fwd_reach_bytes(nseq, heads, t), bwd_reach_layout(nseq, heads, t, head_dim).total);
+  return backward ? bwd_reach_layout(nseq, heads, t, head_dim).total : fwd_reach_bytes(nseq, heads, t);
 }
 
 int sa_forward(const void* q, const void* k, const void* v, float* out, float* rmax, float* rden, float* carry,

@@ -204,13 +204,13 @@ def _stream(device: torch.device) -> int:
 def _forward_scratch(lib, batch: int, heads: int, tk: int, kdim: int, code: int, group: int) -> int:
     """Bytes of sa_forward's workspace, the part for skipping tiles without weight included."""
     return max(int(lib.sa_forward_workspace_bytes(batch, heads, tk, kdim, code, group))
-               + int(lib.sa_reach_bytes(batch, heads, tk, kdim)), 1)
+               + int(lib.sa_reach_bytes(batch, heads, tk, kdim, 0)), 1)
 
 
 def _backward_scratch(lib, batch: int, heads: int, seq: int, kdim: int, code: int, group: int) -> int:
     """Bytes of sa_backward's workspace, the part for skipping tiles without weight included."""
     return (int(lib.sa_backward_workspace_bytes(batch, heads, seq, kdim, code, group))
-            + int(lib.sa_reach_bytes(batch, heads, seq, kdim)))
+            + int(lib.sa_reach_bytes(batch, heads, seq, kdim, 1)))
 
 
 def _launch_forward(qs: Tensor, ks: Tensor, vs: Tensor, kstride: int, scale: float, exempt: int, group: int,

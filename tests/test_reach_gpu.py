@@ -50,7 +50,7 @@ def _forward(q, k, v, exempt, reach, chunk=0, group=0):
     state = (0.4 * (tk - tq - 1 - pos).clamp_min(0)).expand(b, tk) + torch.rand(b, tk, device=dev, generator=g)
     state[:, :exempt] = 0.0
     base = lib.sa_forward_workspace_bytes(b, h, tk, d, code, group)
-    size = base + (lib.sa_reach_bytes(b, h, tk, d) if reach else 0)
+    size = base + (lib.sa_reach_bytes(b, h, tk, d, 0) if reach else 0)
     ws = torch.empty(max(size, 1), dtype=torch.uint8, device=dev)
     _lib.check(lib.sa_forward(qs.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), rmax.data_ptr(),
                               rden.data_ptr(), carry.data_ptr(), state.data_ptr() if chunk else None, state.data_ptr(), tk,
@@ -90,7 +90,7 @@ def _backward(q, k, v, do, aux, exempt, reach, grad_bf16):
     code = kernels._code_of(q)
     out, rmax, rden, carry = aux
     grads = [torch.empty(q.shape, device=q.device, dtype=torch.bfloat16 if grad_bf16 else torch.float32) for _ in range(3)]
-    size = lib.sa_backward_workspace_bytes(b, h, t, d, code, 0) + (lib.sa_reach_bytes(b, h, t, d) if reach else 0)
+    size = lib.sa_backward_workspace_bytes(b, h, t, d, code, 0) + (lib.sa_reach_bytes(b, h, t, d, 1) if reach else 0)
     # (the rows of the checkpoint planes that no sweep writes are read as NaN if anything takes them)
     ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=q.device)
     _lib.check(lib.sa_backward(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), rmax.data_ptr(),
