@@ -2268,11 +2268,9 @@ __device__ __forceinline__ float2 head_qstat(const BwdReach& reach, int64_t r, i
   return make_float2(qm, lm);
 }
 
-// kv_last_block's threshold of one head for a wavefront's keys: kf, vf the lane's parts of its key and value.
-template <class OP, int NS>
-__device__ __forceinline__ float kv_threshold(const typename OP::frag (&kf)[NS], const typename OP::frag (&vf)[NS],
-                                              const float2& qstat, float scale) {
-  float kk = frag_sumsq<OP, NS>(kf), vv = frag_sumsq<OP, NS>(vf);
+// kv_last_block's threshold of one head for a wavefront's keys: kk, vv the sums of squares of the lane's parts of
+// its key and value.
+__device__ __forceinline__ float kv_threshold(float kk, float vv, const float2& qstat, float scale) {
   kk += xor32(kk);
   vv += xor32(vv);
   const float kn = sqrtf(half_max(kk < REACH_NORM2 && vv < REACH_NORM2 ? kk : INFINITY));
@@ -2699,7 +2697,7 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
         kg[s] = k_frag(g, s);
         vg[s] = v_frag(g, s);
       }
-      thr = fmaxf(thr, kv_threshold<OP, NS>(kg, vg, head_qstat(reach, seq_row + hd0 + g, lane), scale));
+      thr = fmaxf(thr, kv_threshold(frag_sumsq<OP, NS>(kg), frag_sumsq<OP, NS>(vg), head_qstat(reach, seq_row + hd0 + g, lane), scale));
     }
     const int last = key0 < T ? kv_last_block(carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane) : 0;
     if (lane == 0) sLast[wave] = last;
@@ -3033,7 +3031,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
     frag vg[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) vg[s] = rfrag(sV[wave], s);
-    const float thr = kv_threshold<OP, NS>(kf, vg, head_qstat(reach, seq_row + hh, lane), scale);
+    const float thr = kv_threshold(frag_sumsq<OP, NS>(kf), frag_sumsq<OP, NS>(vg), head_qstat(reach, seq_row + hh, lane), scale);
     const int last = key0 < T ? kv_last_block(carry_b, T, NB, key0, reach.xk, thr, lane) : 0;
     if (lane == 0) sLast[wave] = last;
     __syncthreads();
@@ -3928,6 +3926,12 @@ struct HalfRow {
       for (int e = 0; e < 4; ++e) f[4 * c + e] = __uint_as_float(x[e]);
     }
   }
+  __device__ __forceinline__ float sumsq() const {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < D / 2; ++i) s = fmaf(f[i], f[i], s);
+    return s;
+  }
 };
 // c += A B^T over the head dim, a and b the lanes' rows of A and B.
 template <int D>
@@ -4129,12 +4133,15 @@ __global__ __launch_bounds__(NTHREADS, 1) void fwd_split_kernel(
 // Key side (bwd_kv_kernel's tile work). grid (ceil(T/32), nseq * H); step t takes the four query tiles
 // NB - 1 - 4t - w, one per wavefront w. The selection suffix entering a wavefront's tile is the one entering
 // the step plus the sums of dz of the later wavefronts' tiles, exchanged through LDS with the step's barrier.
+// With reach.qstat the steps without weight for these keys are left out (kv_last_block, the same search in
+// every wavefront) and the query side finds the last block in hi, one per key tile; a tile stays with the
+// wavefront that had it, so the sums keep their order.
 template <int D>
 __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
     Strides qs, Strides ks, Strides vs, Strides dos, const float* __restrict__ lse, const float* __restrict__ ndbar,
     const float* __restrict__ carry, float* __restrict__ ucheck, float* __restrict__ dk0h, float* __restrict__ dk0x,
-    GradView dkv, GradView dvv, int nseq, int H, int T, int64_t ldt, int exempt, float scale) {
+    GradView dkv, GradView dvv, int nseq, int H, int T, int64_t ldt, int exempt, float scale, BwdReach reach) {
   constexpr int DB = D / 32;
   __shared__ __attribute__((aligned(16))) float sSum[NWAVES][32 * (D + 4)];
   __shared__ float sU[2][NWAVES][TILE];
@@ -4163,8 +4170,16 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
   const float* ndb_row = ndbar + (int64_t)blockIdx.y * ldt;
   const float sl2 = scale * LOG2E, neg_inv_scale = -1.f / scale;
   const int ntiles = NB - kt;
+  int t0 = 0;
+  if (reach.qstat) {
+    const float thr = kv_threshold(kf.sumsq(), vf.sumsq(), head_qstat(reach, blockIdx.y, lane), scale);
+    const int top = __builtin_amdgcn_readfirstlane(
+        kv_last_block(carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane));
+    if (tid == 0) reach.hi[((int64_t)hh * nseq + b) * reach.nkg + kt] = top;
+    t0 = (NB - 1 - top) / 4;
+  }
   float ucarry = 0.f;
-  for (int t = 0; 4 * t < ntiles; ++t) {
+  for (int t = t0; 4 * t < ntiles; ++t) {
     const int qb = NB - 1 - 4 * t - wave;
     const bool mine = qb >= kt;
     f32x16 dz = zero16();
@@ -4172,7 +4187,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
     const int qbase = qb * TILE;
     if (mine) {
       const bool edge = (qbase <= key0 + TILE - 1) || key0 < exempt;
-      const TileMasks mk(j, qbase, T, exempt, h);
+      const TileMasks mk(j, qbase, T, exempt, h, reach.xk);
       HalfRow<D> rows;
       rows.load(rs_q0, qs.row, qbase + n, h);
       const float hist = j < T ? carry_col[(int64_t)qb * T] : 0.f;
@@ -4220,16 +4235,17 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
     }
   }
   const int jn = key0 + (tid >> 3), d0 = (tid & 7) * (D / 8);
+  const bool mine = jn < T && jn >= reach.xk;   // (the first xk keys' gradients: bwd_finish_kernel)
   float part[D / 8];
   auto quad = [&](int c) { return make_float4(part[4 * c], part[4 * c + 1], part[4 * c + 2], part[4 * c + 3]); };
   sum_tiles<D>(sSum, dvt, 1.f, n, h, wave, tid, part);
 #pragma unroll
   for (int c = 0; c < DB; ++c)
-    if (jn < T) store_grad4(dvv, b, hh, jn, d0 + 4 * c, quad(c));
+    if (mine) store_grad4(dvv, b, hh, jn, d0 + 4 * c, quad(c));
   sum_tiles<D>(sSum, dkt, scale, n, h, wave, tid, part);
 #pragma unroll
   for (int c = 0; c < DB; ++c) {
-    if (jn >= T) continue;
+    if (!mine) continue;
     if (has_h0 && H > 1) *reinterpret_cast<float4*>(dk0h + ((int64_t)b * T + jn) * D + d0 + 4 * c) = quad(c);
     else store_grad4(dkv, b, hh, jn, d0 + 4 * c, quad(c));
   }
@@ -4237,17 +4253,20 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
   sum_tiles<D>(sSum, dk0t, scale, n, h, wave, tid, part);
 #pragma unroll
   for (int c = 0; c < DB; ++c)
-    if (jn < T)
+    if (mine)
       *reinterpret_cast<float4*>(dk0x + ((int64_t)(hh - 1) * nseq * T + (int64_t)b * T + jn) * D + d0 + 4 * c) = quad(c);
 }
 
-// Query side (bwd_dq_kernel's tile work). grid (ceil(T/32), nseq * H), the longest sweeps first.
+// Query side (bwd_dq_kernel's tile work). grid (ceil(T/32), nseq * H), the longest sweeps first. With
+// reach.qstat it visits the key tiles whose sweep reached its block, and those of exempt keys, which keep
+// weight but have no selection suffix: one bit per key tile.
+static_assert(SPLIT_MAX_T <= 64 * TILE, "a key tile per bit");
 template <int D>
 __global__ __launch_bounds__(NTHREADS, 1) void bwd_dq_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
     Strides qs, Strides ks, Strides vs, Strides dos, const float* __restrict__ lse, const float* __restrict__ ndbar,
     const float* __restrict__ carry, const float* __restrict__ ucheck, float* __restrict__ dq0h, float* __restrict__ dq0x,
-    GradView dqv, int nseq, int H, int T, int64_t ldt, int exempt, float scale) {
+    GradView dqv, int nseq, int H, int T, int64_t ldt, int exempt, float scale, BwdReach reach) {
   constexpr int DB = D / 32, LDZ = TILE + 4;
   __shared__ __attribute__((aligned(16))) float sZ[NWAVES][TILE * LDZ];
   __shared__ __attribute__((aligned(16))) float sSum[NWAVES][32 * (D + 4)];
@@ -4285,13 +4304,18 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_dq_split_kernel(
     lds_wave_sync();
     mma_cols<D>(acc, rs, ks.row, kbase, n, h, xt);
   };
+  uint64_t reached = ~0ull;
+  if (reach.qstat)
+    reached = __ballot(lane < NB && reach.hi[((int64_t)hh * nseq + b) * reach.nkg + min(lane, NB - 1)] >= qb);
   for (int kt = wave; kt <= qb; kt += NWAVES) {
     const int kbase = kt * TILE, j = kbase + n;
+    const bool suffix = (reached >> kt) & 1;
+    if (!suffix && kbase >= exempt) continue;
     const bool edge = (kbase + TILE - 1 >= qbase) || (kbase + TILE > T) || kbase < exempt;
     const TileMasks mk(j, qbase, T, exempt, h);
     HalfRow<D> rows;
     rows.load(rs_k0, ks.row, j, h);
-    const float hist = j < T ? carry_row[j] : 0.f, uin = j < T ? urow[j] : 0.f;
+    const float hist = j < T ? carry_row[j] : 0.f, uin = suffix && j < T ? urow[j] : 0.f;
     const f32x16 l0 = mma_rows<D>(q0a, rows, zero16());
     f32x16 lg;
     uint32_t gate;
@@ -4761,7 +4785,7 @@ int forward_impl(const FwdCall& c) {
     if (c.group <= 0 && G >= 2) G = fwd64_group(c.nseq, c.H, c.Tq, device_cus());
   }
   if constexpr (sizeof(elem) == 4 && D <= 64) {
-    if (c.damp_mode == 0 && split_f32_grid(c.nseq, c.H, c.Tq, c.Tk, device_cus())) {
+    if (c.damp_mode == 0 && split_f32_grid(c.nseq, c.H, c.Tq, c.Tk, device_cus(), false)) {
       FwdCall sc = c;
       sc.kn = sc.kt = nullptr;   // (every tile is visited)
       const int rc = run_selection<OP, D>(sc, c.st);
@@ -4916,7 +4940,7 @@ int backward_impl(const BwdCall& c) {
   // bf16 at head dim 64 the backward kernels read their Q, dO and K rows transposed from LDS
   // (bwd_kv64_kernel, bwd_dq64_kernel): no transposed copies
   bool split = false;
-  if constexpr (sizeof(elem) == 4 && D <= 64) split = split_f32_grid(nseq, H, T, T, device_cus());
+  if constexpr (sizeof(elem) == 4 && D <= 64) split = split_f32_grid(nseq, H, T, T, device_cus(), true);
   if (!(sizeof(elem) == 2 && D == 64) && !split) {
     launch_transpose<elem, D>(q, qt, T, ldt, c.qs, H, R, st);
     launch_transpose<elem, D>(dout, dot, T, ldt, c.dos, H, R, st);
@@ -4924,8 +4948,8 @@ int backward_impl(const BwdCall& c) {
   }
   BwdReach reach{};
   reach.nseg = (int)cdiv(T, QSTAT_ROWS);
-  reach.nkg = (int)cdiv(T, NWAVES * TILE);
-  if (c.reach && !split) {
+  reach.nkg = (int)cdiv(T, split ? TILE : NWAVES * TILE);
+  if (c.reach) {
     const BwdReachLayout RL = bwd_reach_layout(nseq, H, T, D);
     reach.qstat = reinterpret_cast<float2*>(c.reach + RL.qstat);
     reach.hi = reinterpret_cast<int*>(c.reach + RL.hi);
@@ -4949,11 +4973,12 @@ int backward_impl(const BwdCall& c) {
         TimedLaunch timed(SA_KERNEL_BACKWARD, st);
         hipLaunchKernelGGL((bwd_kv_split_kernel<D>), grid, dim3(NTHREADS), 0, st, q, k, v, dout, c.qs, c.ks, c.vs, c.dos, lse,
                            dbar, c.carry, ucheck, dk0h, dk0x, GradView{c.dk, c.dks, gf32}, GradView{c.dv, c.dvs, gf32}, nseq,
-                           H, T, ldt, c.exempt, c.scale);
+                           H, T, ldt, c.exempt, c.scale, reach);
       }
       TimedLaunch timed(SA_KERNEL_BACKWARD_DQ, st);
       hipLaunchKernelGGL((bwd_dq_split_kernel<D>), grid, dim3(NTHREADS), 0, st, q, k, v, dout, c.qs, c.ks, c.vs, c.dos, lse,
-                         dbar, c.carry, ucheck, dq0h, dq0x, GradView{c.dq, c.dqs, gf32}, nseq, H, T, ldt, c.exempt, c.scale);
+                         dbar, c.carry, ucheck, dq0h, dq0x, GradView{c.dq, c.dqs, gf32}, nseq, H, T, ldt, c.exempt, c.scale,
+                         reach);
       rc = launch_status();
     }
   } else {

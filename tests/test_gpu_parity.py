@@ -431,7 +431,8 @@ def test_chunked_prefill_unaligned_offsets(cuda, chunk, exempt):
 
 @pytest.mark.parametrize("heads,seq,head_dim,exempt,chunk", [
     (1, 1, 64, 1, 0), (2, 31, 64, 1, 0), (3, 33, 32, 16, 0), (1, 97, 64, 40, 0), (4, 128, 32, 1, 0), (2, 129, 64, 3, 0),
-    (2, 513, 64, 1, 0), (1, 1500, 64, 1, 0), (2, 300, 64, 1, 45), (1, 2048, 32, 16, 33)])
+    (2, 513, 64, 1, 0), (1, 1500, 64, 1, 0), (2, 300, 64, 1, 45), (1, 2048, 32, 16, 33),
+    (3, 1377, 64, 40, 0), (8, 2047, 64, 16, 0)])
 def test_fp32_split_tiles_match_oracle(cuda, heads, seq, head_dim, exempt, chunk):
     """Small fp32 grids, whose kernels split each tile row between a workgroup's wavefronts: fewer tiles than
     wavefronts, remainders of four tiles, odd lengths, one-head sequences, a chunk at an odd offset."""
