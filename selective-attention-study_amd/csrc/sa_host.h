@@ -109,17 +109,19 @@ inline int fwd64_group(int64_t nseq, int64_t heads, int64_t tq, int cus) {
 // Whether the fp32 kernels of head dim <= 64 split each tile row between the wavefronts of a workgroup
 // (fwd_split_kernel and its backward counterparts): where the unsplit grid leaves half the CUs without a
 // workgroup; in the forward, whose split kernel computes every tile, three quarters from REACH_MIN_KEYS keys
-// on, where the unsplit one leaves tiles out. Past SPLIT_MAX_T keys what that leaves out can outweigh any split.
+// on, where the unsplit one leaves tiles out: past SPLIT_MAX_T keys what that leaves out can outweigh any split.
 // Measured (fwd + bwd, us, split / unsplit, B x H x T, N(0,1) inputs): 1x4x512 159 / 361 (16 workgroups),
 // 2x12x129 126 / 241 (48), 4x8x512 300 / 368 (128), at head dim 32 1x8x1024 140 / 276 (64); beyond the rule
 // 8x8x512 561 / 384 (256), 2x8x1024 507 / 405 (128, both directions split and the backward computing every
 // tile): the split reads every operand four times. The backward alone, its split kernels leaving tiles out (key
 // + query side, us, split / unsplit): 1x1x2048 71 / 203 (16), 1x4x2048 117 / 357 (64), 1x8x2048 221 / 264 (128),
-// 1x12x1024 217 / 263 (96); every tile computed 1x8x2048 714 / 879, 1x12x1024 378 / 460.
+// 1x12x1024 217 / 263 (96), 1x2x8192 202 / 290 (128), 1x1x16384 165 / 203 (128), at head dim 32 1x1x5003 55 / 132
+// (40); every tile computed 1x8x2048 714 / 879, 1x12x1024 378 / 460, 1x4x4096 1049 / 1721, 1x1x16384 1678 / 4638.
 constexpr int64_t SPLIT_MAX_T = 2048;
 inline bool split_f32_grid(int64_t nseq, int64_t heads, int64_t tq, int64_t tk, int cus, bool backward) {
   const int64_t workgroups = nseq * heads * cdiv(cdiv(tq, TILE), NWAVES);
-  return tk <= SPLIT_MAX_T && workgroups <= (backward || tk < REACH_MIN_KEYS ? cus / 2 : cus / 4);
+  if (backward) return workgroups <= cus / 2;
+  return tk <= SPLIT_MAX_T && workgroups <= (tk < REACH_MIN_KEYS ? cus / 2 : cus / 4);
 }
 
 // The dispatch order of the query-side backward kernel at head dim 64 (work_order_block): the number

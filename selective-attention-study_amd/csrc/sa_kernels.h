@@ -3910,7 +3910,7 @@ __global__ __launch_bounds__(DQ64_WAVES * 64, 1) void bwd_dq64_kernel(
 // takes elements [h D/2, (h+1) D/2)), so a lane's rows load as 16-byte pieces; the products that contract
 // over rows read the untransposed matrices a row per half-wavefront, whole 128-byte segments, so no
 // transposed copies are made. Measured at B=1 H=4 T=512 D=64: forward 72 -> 26 us, key side 122 -> 53, query side
-// 116 -> 45.
+// 116 -> 45; at B=1 H=8 T=2048 every tile computed: key side 456 -> 382, query side 422 -> 331.
 //
 // Taken by split_f32_grid.
 
@@ -4259,8 +4259,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
 
 // Query side (bwd_dq_kernel's tile work). grid (ceil(T/32), nseq * H), the longest sweeps first. With
 // reach.qstat it visits the key tiles whose sweep reached its block, and those of exempt keys, which keep
-// weight but have no selection suffix: one bit per key tile.
-static_assert(SPLIT_MAX_T <= 64 * TILE, "a key tile per bit");
+// weight but have no selection suffix: one bit per key tile, 64 tiles at a time.
 template <int D>
 __global__ __launch_bounds__(NTHREADS, 1) void bwd_dq_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
@@ -4305,11 +4304,13 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_dq_split_kernel(
     mma_cols<D>(acc, rs, ks.row, kbase, n, h, xt);
   };
   uint64_t reached = ~0ull;
-  if (reach.qstat)
-    reached = __ballot(lane < NB && reach.hi[((int64_t)hh * nseq + b) * reach.nkg + min(lane, NB - 1)] >= qb);
   for (int kt = wave; kt <= qb; kt += NWAVES) {
+    if (reach.qstat && kt % 64 == wave) {
+      const int x = kt - wave + lane;
+      reached = __ballot(x < NB && reach.hi[((int64_t)hh * nseq + b) * reach.nkg + min(x, NB - 1)] >= qb);
+    }
     const int kbase = kt * TILE, j = kbase + n;
-    const bool suffix = (reached >> kt) & 1;
+    const bool suffix = (reached >> (kt % 64)) & 1;
     if (!suffix && kbase >= exempt) continue;
     const bool edge = (kbase + TILE - 1 >= qbase) || (kbase + TILE > T) || kbase < exempt;
     const TileMasks mk(j, qbase, T, exempt, h);

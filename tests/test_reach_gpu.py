@@ -65,7 +65,8 @@ SHAPES = [(1, 2, 1024, 64, "bf16"), (2, 3, 2081, 64, "bf16"), (1, 16, 8200, 64, 
           (1, 4, 1500, 32, "bf16"), (1, 2, 2049, 128, "bf16"), (1, 2, 1377, 64, "f32"), (1, 1, 1111, 32, "f32"),
           (1, 2, 1056, 128, "f32"),
           # fp32 backward on the split kernels: one tile past 1024, the longest and widest grid; unsplit beside them
-          (1, 3, 1025, 32, "f32"), (1, 8, 2048, 64, "f32"), (1, 12, 1411, 64, "f32")]
+          (1, 3, 1025, 32, "f32"), (1, 8, 2048, 64, "f32"), (1, 12, 1411, 64, "f32"),
+          (1, 2, 4129, 64, "f32")]
 
 
 @pytest.mark.parametrize("kind", ["normal", "holes", "sparse", "special"])
