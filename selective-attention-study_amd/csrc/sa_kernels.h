@@ -792,12 +792,17 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 struct TileRun {
   int hi, lo;
 };
-constexpr int REACH_RUNS = 64;   // at most; what would need more ends in one run down to tile 0
+constexpr int REACH_RUNS = 64;   // entries of the list
 
-// The set bits of the words (bit i of word w: tile first + 64 w + i), then every tile below first, as runs
-// ending in {-1, INT_MIN}, below which a sweep finds no tile. One wavefront.
+// The set bits of the words (bit i of word w: tile first + 64 w + i), then the tiles below first, as runs
+// ending in {-1, INT_MIN}, below which a sweep finds no tile. What the list does not hold -- the tiles below
+// first, and whatever is left once it is full -- becomes one run down to tile 0 with REST (for a reader to
+// whom a tile too many costs time only: the forward), else an entry {-2, INT_MIN}, at which the reader
+// has to look for itself. One wavefront.
+template <bool REST>
 __device__ __forceinline__ void write_reach_runs(TileRun* runs, const uint64_t* words, int nwords, int first, int lane) {
   int n = 0;
+  bool full = false;
   TileRun open{-1, -1};
   auto add = [&](int hi, int lo) {
     if (open.hi >= 0 && hi == open.lo - 1) {
@@ -826,18 +831,18 @@ __device__ __forceinline__ void write_reach_runs(TileRun* runs, const uint64_t* 
       const int len = min(gaps != 0 ? __builtin_clzll(gaps) : 64, bit + 1);
       add(first + 64 * w + bit, first + 64 * w + bit - len + 1);
       word &= (bit - len >= 0) ? (2ull << (bit - len)) - 1 : 0;
-      if (n == REACH_RUNS - 2) {
-        open.lo = 0;
+      if (n == REACH_RUNS - 2) {   // full, with the open run and the ending
+        if (REST) open.lo = 0;
+        full = true;
         word = 0;
         w = 0;
-        first = 0;
       }
     }
   }
-  if (first > 0) add(first - 1, 0);
+  if (REST && !full && first > 0) add(first - 1, 0);
   if (lane == 0) {
     if (open.hi >= 0) runs[n++] = open;
-    runs[n] = {-1, INT_MIN};
+    runs[n] = {!REST && (full || first > 0) ? -2 : -1, INT_MIN};
   }
 }
 
@@ -929,7 +934,7 @@ __device__ __forceinline__ void find_reach(const typename OP::frag (&qf)[G][NS],
     if (lane == 0) words[w] = bits;
   }
   __syncthreads();
-  if (wave == 0) write_reach_runs(runs, words, nwords, first, lane);
+  if (wave == 0) write_reach_runs<true>(runs, words, nwords, first, lane);
   __syncthreads();
 }
 
@@ -3221,12 +3226,21 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
 // The key tiles that a query-side workgroup has to visit, ascending, from the key side's sweep starts
 // (hi, one per four key tiles): those whose sweep reached the workgroup's first query block qb0 -- past
 // it their weights and selection suffixes are zeros -- and the tiles of exempt keys, [0, i_lo). As runs of
-// groups of four tiles counted from the workgroup's last group (write_reach_runs counts down).
+// groups of four tiles counted from the workgroup's last group (write_reach_runs counts down). No other
+// group may be visited: past its sweep's start the key side has written no checkpoint of the suffixes. Where
+// the list ends short of the last group (selected and unselected keys in turn over more than 16K keys), the
+// walk takes the next groups from hi itself, 64 at a time.
 struct QueryWalk {
   const TileRun* runs;
+  const int* starts;   // hi
+  int first_qb;        // qb0
   int groups, run_to, i;
   bool far;   // the first group is visited for its exempt keys alone
   __device__ __forceinline__ void none() {   // every tile
+    runs = nullptr;
+    starts = nullptr;
+    first_qb = 0;
+    groups = 0;
     run_to = INT_MAX;
     far = false;
     i = 0;
@@ -3234,6 +3248,8 @@ struct QueryWalk {
   template <int NW>
   __device__ __forceinline__ void find(const int* hi, int qb0, int wg_end, int i_lo, uint64_t* words, TileRun* r,
                                        int lane, int wave) {
+    starts = hi;
+    first_qb = qb0;
     groups = (wg_end + 3) / 4;
     far = __builtin_amdgcn_readfirstlane(hi[0]) < qb0;
     const int all = (groups + 63) / 64, nwords = min(all, REACH_MASK_WORDS), first = 64 * (all - nwords);
@@ -3243,7 +3259,7 @@ struct QueryWalk {
       if (lane == 0) words[w] = bits;
     }
     __syncthreads();
-    if (wave == 0) write_reach_runs(r, words, nwords, first, lane);
+    if (wave == 0) write_reach_runs<false>(r, words, nwords, first, lane);
     __syncthreads();
     runs = r;
     i = 0;
@@ -3255,10 +3271,32 @@ struct QueryWalk {
     }
   }
   __device__ __forceinline__ void next_run(int& from) {
-    const TileRun r = runs[i++];
+    const TileRun r = runs[i];
     const int hi = __builtin_amdgcn_readfirstlane(r.hi), lo = __builtin_amdgcn_readfirstlane(r.lo);
+    if (__builtin_expect(hi == -2, 0)) {   // (and again at the next call: i stays)
+      search(from);
+      return;
+    }
+    ++i;
     from = 4 * (groups - 1 - hi);   // (past the workgroup's last tile at the end)
     run_to = hi < 0 ? INT_MAX : 4 * (groups - 1 - lo) + 3;
+  }
+  // The next run past tile run_to from hi: within 64 groups.
+  __device__ __forceinline__ void search(int& from) {
+    const int lane = threadIdx.x & 63;
+    for (int g = (run_to + 1) / 4; g < groups; g += 64) {
+      const uint64_t bits = __ballot(g + lane < groups && starts[min(g + lane, groups - 1)] >= first_qb);
+      if (bits != 0) {
+        const int at = __builtin_ctzll(bits);
+        const uint64_t gaps = ~(bits >> at);   // (a shifted-in zero ends the run at the 64 groups' end)
+        const int len = gaps != 0 ? __builtin_ctzll(gaps) : 64;
+        from = 4 * (g + at);
+        run_to = from + 4 * len - 1;
+        return;
+      }
+    }
+    from = 4 * groups;
+    run_to = INT_MAX;
   }
   __device__ __forceinline__ int after(int kt) {
     int n = kt + 1;

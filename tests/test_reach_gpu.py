@@ -27,6 +27,11 @@ def _inputs(cuda, b, h, t, d, dtype, kind, seed=11):
         k[:, 0] -= math.sqrt(3.0 * math.sqrt(d) / d)
     elif kind == "holes":     # a few keys that nobody selects among selected ones: short and long runs
         k[:, 0, torch.arange(5, t, 97, device=cuda)] = 0.0
+    elif kind == "groups":    # nobody selects the keys of every second workgroup of the key side
+        k[:, 0, (torch.arange(t, device=cuda) // 128) % 2 == 1] = 0.0
+    elif kind == "random":    # ... or of a random half of them
+        some = torch.rand((t + 127) // 128, device=cuda, generator=g) < 0.5
+        k[:, 0, some.repeat_interleave(128)[:t]] = 0.0
     elif kind == "special":   # values a zero weight does not silence, keys and queries beyond the bound
         v[:, -1, 3] = float("inf")
         v[:, 0, 200] = float("nan")
@@ -69,7 +74,7 @@ SHAPES = [(1, 2, 1024, 64, "bf16"), (2, 3, 2081, 64, "bf16"), (1, 16, 8200, 64, 
           (1, 2, 4129, 64, "f32")]
 
 
-@pytest.mark.parametrize("kind", ["normal", "holes", "sparse", "special"])
+@pytest.mark.parametrize("kind", ["normal", "holes", "groups", "sparse", "special"])
 @pytest.mark.parametrize("b,h,t,d,dtype", SHAPES)
 def test_forward_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
     print(f"case forward {b} {h} {t} {d} {dtype} {kind}", flush=True)
@@ -103,7 +108,28 @@ def _backward(q, k, v, do, aux, exempt, reach, grad_bf16):
     return grads
 
 
-@pytest.mark.parametrize("kind", ["normal", "holes", "sparse", "special"])
+def _compare_backward(q, k, v, do, exempt, half):
+    bf16 = q.dtype == torch.bfloat16
+    aux = _forward(q, k, v, exempt, True)[:4]
+    got = _backward(q, k, v, do, aux, exempt, True, half)
+    want = _backward(q, k, v, do, aux, exempt, False, half)
+    first = 128 if exempt <= 32 else 0
+    for x, y in zip(got[1:], want[1:]):
+        assert torch.equal(_bits(x[:, :, first:]), _bits(y[:, :, first:])), exempt
+    if first == 0:
+        assert torch.equal(_bits(got[0]), _bits(want[0])), exempt
+        return
+    for x, y in zip(got, want):
+        x, y = x.double(), y.double()
+        assert torch.equal(x.isnan(), y.isnan())
+        fine = y.isfinite()
+        # dQ: 1e-7 of fp32 rounding; dK, dV of the exempt keys: split bf16 operands (2^-16 each) or fp32
+        # products summed in another order; a bf16 gradient's own rounding beside that
+        tol = 2.0 ** -8 if half else 2.0 ** -14 if bf16 else 2.0 ** -18
+        assert (x - y)[fine].norm() <= tol * y[fine].norm() + 1e-30, exempt
+
+
+@pytest.mark.parametrize("kind", ["normal", "holes", "groups", "sparse", "special"])
 @pytest.mark.parametrize("b,h,t,d,dtype", SHAPES)
 def test_backward_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
     """With more than 32 exempt keys the same instances of the kernels run: every bit. Up to 32 of them the
@@ -114,21 +140,16 @@ def test_backward_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
     bf16 = dtype == "bf16"
     q, k, v, do = _inputs(cuda, b, h, t, d, torch.bfloat16 if bf16 else torch.float32, kind)
     for exempt in (1, 16, 32, 40):
-        aux = _forward(q, k, v, exempt, True)[:4]
-        half = bf16 and exempt == 1
-        got = _backward(q, k, v, do, aux, exempt, True, half)
-        want = _backward(q, k, v, do, aux, exempt, False, half)
-        first = 128 if exempt <= 32 else 0
-        for x, y in zip(got[1:], want[1:]):
-            assert torch.equal(_bits(x[:, :, first:]), _bits(y[:, :, first:])), exempt
-        if first == 0:
-            assert torch.equal(_bits(got[0]), _bits(want[0])), exempt
-            continue
-        for x, y in zip(got, want):
-            x, y = x.double(), y.double()
-            assert torch.equal(x.isnan(), y.isnan())
-            fine = y.isfinite()
-            # dQ: 1e-7 of fp32 rounding; dK, dV of the exempt keys: split bf16 operands (2^-16 each) or fp32
-            # products summed in another order; a bf16 gradient's own rounding beside that
-            tol = 2.0 ** -8 if half else 2.0 ** -14 if bf16 else 2.0 ** -18
-            assert (x - y)[fine].norm() <= tol * y[fine].norm() + 1e-30, exempt
+        _compare_backward(q, k, v, do, exempt, bf16 and exempt == 1)
+
+
+# More runs of kept 128-key groups than the query side's list holds (64): bwd_dq64_kernel with several heads and
+# one, bwd_dq_kernel at one and two heads per wavefront, head dim 128, fp32
+@pytest.mark.parametrize("kind", ["groups", "random"])
+@pytest.mark.parametrize("b,h,t,d,dtype", [(1, 2, 20001, 64, "bf16"), (1, 1, 40000, 64, "bf16"), (1, 2, 40001, 32, "bf16"),
+                                           (1, 1, 20001, 32, "bf16"), (1, 1, 33000, 128, "bf16"), (1, 1, 24001, 64, "f32")])
+def test_backward_past_the_run_list_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
+    print(f"case backward runs {b} {h} {t} {d} {dtype} {kind}", flush=True)
+    q, k, v, do = _inputs(cuda, b, h, t, d, torch.bfloat16 if dtype == "bf16" else torch.float32, kind)
+    for exempt in (1, 40):
+        _compare_backward(q, k, v, do, exempt, False)
