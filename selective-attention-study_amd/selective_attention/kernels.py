@@ -38,6 +38,7 @@ listing, exported as in the reference.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -244,14 +245,33 @@ def _launch_forward(qs: Tensor, ks: Tensor, vs: Tensor, kstride: int, scale: flo
 
 # -- the C-ABI calls as custom ops ------------------------------------------------------------------
 
+def _custom_op(name: str, impl):
+    """The custom op of an implementation. A zero tensor reaches it as one element expanded to the shape: the
+    implementations read contiguous storage."""
+
+    @functools.wraps(impl)
+    def run(*args, **kwargs):
+        dense = lambda x: x.contiguous() if isinstance(x, Tensor) else x
+        return impl(*map(dense, args), **{n: dense(x) for n, x in kwargs.items()})
+
+    return torch.library.custom_op(f"selective_attention::{name}", mutates_args=(), device_types="cuda")(run)
+
+
 def _plain(*tensors: Tensor) -> bool:
-    """Whether a custom op call on these tensors could only end in its own CUDA implementation: plain tensors,
-    nothing that traces, transforms or records ops, and no gradient to ask of the op itself (which has no
-    formula: a second derivative raises). The implementation is then called as it is: the op's Python
-    layers take 13 us of host time per call, a tenth of a short training step."""
-    return (all(type(t) in (Tensor, torch.nn.Parameter) for t in tensors)
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            and not torch.compiler.is_compiling()
+    """Whether a custom op call on these tensors could only end in its own CUDA implementation: plain tensors
+    (nothing that the dispatcher would resolve, or refuse, first: a pending negation, names, no storage of
+    their own as a zero tensor or a functional wrapper), nothing that traces, transforms or records ops, and
+    no gradient to ask of the op itself (which has no formula: a second derivative raises). The
+    implementation is then called as it is: the op's Python layers take 13 us of host time per call, a tenth
+    of a short training step."""
+    if torch.compiler.is_compiling():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if ((type(t) is not Tensor and type(t) is not torch.nn.Parameter) or (grad and t.requires_grad)
+                or t.is_neg() or t.has_names() or t.data_ptr() == 0):
+            return False
+    return (torch._C._len_torch_function_stack() == 0
             and torch._C._len_torch_dispatch_stack() == 0
             and torch._ops._len_torch_dispatch_stack_pre_dispatch() == 0
             and torch._C._functorch.peek_interpreter_stack() is None
@@ -266,7 +286,7 @@ def _forward_impl(q: Tensor, k: Tensor, v: Tensor, scale: float, exempt: int, gr
     return _launch_forward(q, k, v, k.shape[-2] * k.shape[-1], scale, exempt, group, damp_mode, train_len)
 
 
-_forward_op = torch.library.custom_op("selective_attention::forward", mutates_args=(), device_types="cuda")(_forward_impl)
+_forward_op = _custom_op("forward", _forward_impl)
 
 
 @_forward_op.register_fake
@@ -300,7 +320,7 @@ def _backward_impl(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, r
     return dq, dk, dv
 
 
-_backward_op = torch.library.custom_op("selective_attention::backward", mutates_args=(), device_types="cuda")(_backward_impl)
+_backward_op = _custom_op("backward", _backward_impl)
 
 
 @_backward_op.register_fake
@@ -344,7 +364,7 @@ def _qkv_forward_impl(qkv: Tensor, heads: int, exempt: int) -> tuple[Tensor, Ten
     return y, out, rmax, rden, carry
 
 
-_qkv_forward_op = torch.library.custom_op("selective_attention::qkv_forward", mutates_args=(), device_types="cuda")(_qkv_forward_impl)
+_qkv_forward_op = _custom_op("qkv_forward", _qkv_forward_impl)
 
 
 @_qkv_forward_op.register_fake
@@ -380,7 +400,7 @@ def _qkv_backward_impl(qkv: Tensor, dy: Tensor, out: Tensor, rmax: Tensor, rden:
     return dqkv
 
 
-_qkv_backward_op = torch.library.custom_op("selective_attention::qkv_backward", mutates_args=(), device_types="cuda")(_qkv_backward_impl)
+_qkv_backward_op = _custom_op("qkv_backward", _qkv_backward_impl)
 
 
 @_qkv_backward_op.register_fake

@@ -264,3 +264,30 @@ def test_ops_are_passed_by_only_for_plain_eager_tensors():
     torch.func.vmap(lambda t: seen.append(kernels._plain(x)) or t)(torch.zeros(3, 2))
     assert seen == [False]
     assert not kernels._plain(torch.zeros(2).as_subclass(type("Sub", (torch.Tensor,), {})))
+
+
+def test_ops_are_not_passed_by_where_the_dispatcher_has_work():
+    """A real tensor whose negation is pending, a zero tensor without storage, a functional wrapper and a named
+    tensor are of type Tensor too: the dispatcher resolves or refuses them, so the op has to be called. Nor is an
+    op hidden from a torch function mode; autocast and inference mode change nothing for it."""
+    from torch.overrides import TorchFunctionMode
+
+    class Seen(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.ones(2)
+    neg = torch._neg_view(x).to(x.dtype).contiguous()   # as the operator's storage step leaves it
+    assert neg.is_neg() and type(neg) is torch.Tensor
+    for odd in (neg, torch._efficientzerotensor((2,)), torch._to_functional_tensor(x)):
+        assert not kernels._plain(odd)
+        assert not kernels._plain(x, odd)
+    with pytest.warns(UserWarning, match="[Nn]amed tensors"):
+        assert not kernels._plain(torch.ones(2, names=("a",)))
+    with Seen():
+        assert not kernels._plain(x)
+    assert kernels._plain(x)
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        assert kernels._plain(x)
+    with torch.inference_mode():
+        assert kernels._plain(x, torch.ones(2))

@@ -51,3 +51,27 @@ def test_custom_ops_pass_opcheck(cuda):
                           (q, k, v, out, q, rmax, rden, carry, 0.125, 1, 0, True),
                           test_utils=("test_schema", "test_faketensor"))
     assert kernels.HAS_HIP
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_pending_negations_and_zero_tensors_are_resolved(cuda, dtype):
+    """Inputs and gradients whose negation is pending (a negative view: type Tensor, the storage not negated yet),
+    and tensors of zeros without storage, give what their values give."""
+    g = torch.Generator(device=cuda).manual_seed(1)
+    q, k, v, do = (torch.randn(1, 2, 70, 64, device=cuda, generator=g).to(dtype) for _ in range(4))
+    do = do.float()
+
+    def step(q, k, v, do):
+        leaves = [x.detach().requires_grad_(True) for x in (q, k, v)]
+        out = kernels.selective_attention(*leaves)
+        return (out.detach(), kernels.selective_attention_forward(q, k, v)) + torch.autograd.grad(out, leaves, do)
+
+    zeros = torch._efficientzerotensor(q.shape, dtype=dtype, device=cuda)
+    for got, want in ((step(torch._neg_view(q), k, torch._neg_view(v), torch._neg_view(do)), step(-q, k, -v, -do)),
+                      (step(q, k, zeros, do), step(q, k, torch.zeros_like(q), do))):
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    qkv = torch.randn(1, 70, 3 * 128, device=cuda, generator=g).to(dtype)
+    precision = None if dtype == torch.bfloat16 else "tf32"
+    assert torch.equal(kernels.selective_attention_qkv(torch._neg_view(qkv), 2, precision),
+                       kernels.selective_attention_qkv(-qkv, 2, precision))
