@@ -943,7 +943,7 @@ __device__ __forceinline__ void find_reach(const typename OP::frag (&qf)[G][NS],
 // of S[r, j]. One wavefront per key block (its K rows in registers); a workgroup walks RB query
 // blocks, each staged once in LDS for its four wavefronts while the next one loads. The grid's z past the
 // sequences takes the key norms (key_norms_block) of all heads along: work of the same launch that the
-// forward needs next to the carry, in place of a launch of its own (2-3 us).
+// forward needs next to the carry, in place of a launch of its own (2-3 us), where the grid has room for them.
 constexpr int SEL_RB = 8;   // query blocks per workgroup
 
 template <class OP, int D>
@@ -4757,6 +4757,10 @@ int run_selection(const FwdCall& c, hipStream_t st) {
   const int NBq = (int)cdiv(c.Tq, TILE), NKT = (int)cdiv(c.Tk, TILE);
   const int64_t nkb = cdiv(c.Tk, NORM_KEYS);
   TimedLaunch timed(SA_KERNEL_SELECTION, st);
+  auto norms_apart = [&]() {
+    hipLaunchKernelGGL((key_norms_kernel<elem, D>), dim3((unsigned)nkb, (unsigned)(c.nseq * c.H)), dim3(NTHREADS), 0, st,
+                       static_cast<const elem*>(c.k), static_cast<const elem*>(c.v), c.ks, c.vs, c.H, c.Tk, c.kn);
+  };
   if constexpr (sizeof(elem) == 2 && D == 64) {
     const int64_t wgs = cdiv(NKT, NWAVES * SEL_CARRY_KPW);
     // (its carry stores address one sequence's plane through a 32-bit buffer range)
@@ -4764,16 +4768,17 @@ int run_selection(const FwdCall& c, hipStream_t st) {
       hipLaunchKernelGGL(sel_carry64_kernel, dim3((unsigned)wgs, (unsigned)c.nseq), dim3(NTHREADS), 0,
                          st, static_cast<const uint16_t*>(c.q), static_cast<const uint16_t*>(c.k), c.carry,
                          c.state_in, c.state_out, c.state_ld, c.Tq, c.Tk, c.qs, c.ks, c.q_off, c.exempt, c.scale, c.kt);
-      if (c.kn)
-        hipLaunchKernelGGL((key_norms_kernel<elem, D>), dim3((unsigned)nkb, (unsigned)(c.nseq * c.H)), dim3(NTHREADS), 0,
-                           st, static_cast<const elem*>(c.k), static_cast<const elem*>(c.v), c.ks, c.vs, c.H, c.Tk,
-                           c.kn);
+      if (c.kn) norms_apart();
       return launch_status();
     }
   }
   const int RB = SEL_RB;
   dim3 g1((unsigned)cdiv(NKT, NWAVES), (unsigned)cdiv(NBq, RB), (unsigned)c.nseq);
-  if (c.kn) g1.z += (unsigned)cdiv((int64_t)c.nseq * c.H * nkb, (int64_t)g1.x * g1.y);   // the key norms' workgroups
+  // the key norms' workgroups, unless they would take z past a grid's limit (tens of thousands of sequences)
+  const int64_t znorms = c.kn ? cdiv((int64_t)c.nseq * c.H * nkb, (int64_t)g1.x * g1.y) : 0;
+  const bool norms_along = c.nseq + znorms <= 65535;
+  if (norms_along) g1.z += (unsigned)znorms;
+  else norms_apart();
   hipLaunchKernelGGL((sel_colsum_kernel<OP, D>), g1, dim3(NTHREADS), 0, st, static_cast<const elem*>(c.q),
                      static_cast<const elem*>(c.k), c.carry, c.H, c.Tq, c.Tk, c.qs, c.ks, c.q_off, c.exempt, c.scale,
                      RB, static_cast<const elem*>(c.v), c.vs, c.nseq, c.kn);

@@ -153,3 +153,26 @@ def test_backward_past_the_run_list_keeps_its_bits(cuda, b, h, t, d, dtype, kind
     q, k, v, do = _inputs(cuda, b, h, t, d, torch.bfloat16 if dtype == "bf16" else torch.float32, kind)
     for exempt in (1, 40):
         _compare_backward(q, k, v, do, exempt, False)
+
+
+def test_key_norms_of_more_sequences_than_a_grid_extent_holds_beside_them(cuda):
+    """60000 sequences of 1024 keys, head dim 32, the last 32 queries: the key norms' workgroups no longer fit beside
+    the column sums' (65535 in z). One sequence's rows, read by all of them."""
+    lib = _lib.load()
+    n, tq, tk, d = 60000, 32, 1024, 32
+    q, k, v, _ = _inputs(cuda, 1, 1, tk, d, torch.bfloat16, "normal")
+    q = q[:, :, tk - tq:].contiguous()
+    before = (0.4 * (tk - tq - 1 - torch.arange(tk, device=cuda)).clamp_min(0)).float()[None]
+    state = before.repeat(n, 1)
+    out, rmax, rden = (torch.empty(n, 1, tq, *s, device=cuda) for s in ((d,), (), ()))
+    carry = torch.empty(n, tq // 32, tk, device=cuda)
+    size = lib.sa_forward_workspace_bytes(n, 1, tk, d, _lib.DTYPE_BF16, 0) + lib.sa_reach_bytes(n, 1, tk, d, 0)
+    ws = torch.empty(size, dtype=torch.uint8, device=cuda)
+    one = _lib.ViewStrides(0, 0, d)
+    _lib.check(lib.sa_forward_strided(q.data_ptr(), one, k.data_ptr(), one, v.data_ptr(), one, out.data_ptr(), None, None,
+                                      rmax.data_ptr(), rden.data_ptr(), carry.data_ptr(), state.data_ptr(), state.data_ptr(),
+                                      tk, ws.data_ptr(), size, n, 1, tq, tk, tk - tq, d, 1 / math.sqrt(d), _lib.DTYPE_BF16, 1,
+                                      0, 0, 0, torch.cuda.current_stream().cuda_stream))
+    want = kernels.selective_attention_prefill(q, k, v, before, tk - tq)   # (before: the state after it)
+    assert torch.equal(out, want.expand_as(out))
+    assert torch.equal(state, before.expand_as(state))
