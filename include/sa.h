@@ -84,9 +84,12 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
  * invalid sizes): given a workspace larger by this much, sa_forward and sa_backward leave out the tiles
  * whose softmax weights are exact fp32 zeros because their keys' history has outgrown every logit. The
  * results have the same bits with and without it, but for the gradients of at most 32 exempt keys, which
- * the backward then sums in another order. t: the number of keys;
- * backward: 0 for sa_forward's workspace, 1 for sa_backward's. */
+ * the backward then sums in another order. t: the number of keys (0 bytes below 1024, where nothing is
+ * looked for); backward: 0 for sa_forward's workspace, 1 for sa_backward's with any number of exempt keys.
+ * sa_backward_reach_bytes: what sa_backward's workspace takes with `exempt` of them; less, the fewer of them up
+ * to 32 (at one about a thirtieth of sa_reach_bytes' figure). */
 int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim, int backward);
+int64_t sa_backward_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim, int64_t exempt);
 
 /*
  * Forward pass, and one chunk of a chunked prefill.

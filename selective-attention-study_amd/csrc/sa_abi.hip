@@ -21,7 +21,7 @@ using namespace sa_host;
 
 extern "C" {
 
-int sa_abi_version(void) { return 6; }
+int sa_abi_version(void) { return 7; }
 
 int sa_timing_enable(int on) {
   TimingRegistry& r = timing();
@@ -78,7 +78,13 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
 
 int64_t sa_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim, int backward) {
   if (!valid_dims(nseq, heads, t) || (head_dim != 32 && head_dim != 64 && head_dim != 128)) return -1;
-  return backward ? bwd_reach_layout(nseq, heads, t, head_dim).total : fwd_reach_bytes(nseq, heads, t);
+  if (t < REACH_MIN_KEYS) return 0;   // (nothing is looked for)
+  return backward ? bwd_reach_layout(nseq, heads, t, head_dim, EXEMPT_APART).total : fwd_reach_bytes(nseq, heads, t);
+}
+
+int64_t sa_backward_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t head_dim, int64_t exempt) {
+  if (!valid_dims(nseq, heads, t) || (head_dim != 32 && head_dim != 64 && head_dim != 128) || exempt < 1) return -1;
+  return t < REACH_MIN_KEYS ? 0 : bwd_reach_layout(nseq, heads, t, head_dim, exempt_apart(exempt)).total;
 }
 
 int sa_forward(const void* q, const void* k, const void* v, float* out, float* rmax, float* rden, float* carry,
@@ -230,7 +236,7 @@ int sa_backward_strided(const void* q, const sa_view_strides* q_strides, const v
   c.dv = dv;
   c.ws = workspace;
   const int64_t base = sa_backward_workspace_bytes(nseq, heads, t, head_dim, dtype, group);
-  if (t >= REACH_MIN_KEYS && workspace_bytes >= base + bwd_reach_layout(nseq, heads, t, head_dim).total &&
+  if (t >= REACH_MIN_KEYS && workspace_bytes >= base + sa_backward_reach_bytes(nseq, heads, t, head_dim, exempt) &&
       (uintptr_t)workspace % 16 == 0)
     c.reach = static_cast<char*>(workspace) + base;
   c.dqs = st(dq_strides);

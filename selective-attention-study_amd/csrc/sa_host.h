@@ -202,7 +202,7 @@ constexpr int REACH_MASK_WORDS = 128;   // a workgroup's tile mask: its newest 6
 
 // Backward: per head and QSTAT_ROWS rows the largest query norm and the least lse; per head group and 128
 // keys the last query block their weights reach; and the exempt keys' gradients, summed per QSTAT_ROWS
-// rows, where there are at most EXEMPT_APART of them (bwd_rowprep_kernel).
+// rows, where there are at most EXEMPT_APART of them (bwd_rowprep_kernel): exempt_apart(exempt) of them.
 constexpr int QSTAT_ROWS = 128;
 constexpr int EXEMPT_APART = 32;
 struct BwdReach {
@@ -215,13 +215,14 @@ struct BwdReach {
 struct BwdReachLayout {
   int64_t qstat, hi, xpart, total;
 };
-inline BwdReachLayout bwd_reach_layout(int64_t nseq, int64_t heads, int64_t t, int64_t D) {
+inline int exempt_apart(int64_t exempt) { return exempt <= EXEMPT_APART ? (int)exempt : 0; }
+inline BwdReachLayout bwd_reach_layout(int64_t nseq, int64_t heads, int64_t t, int64_t D, int xk) {
   const int64_t R = nseq * heads, nseg = cdiv(t, QSTAT_ROWS);
   BwdReachLayout L;
   L.qstat = 0;
   L.hi = align_up(R * nseg * 8, 256);
   L.xpart = L.hi + align_up(R * cdiv(t, TILE) * 4, 256);
-  L.total = L.xpart + align_up(R * nseg * EXEMPT_APART * 2 * D * 4, 256);
+  L.total = L.xpart + align_up(R * nseg * xk * 2 * D * 4, 256);
   return L;
 }
 

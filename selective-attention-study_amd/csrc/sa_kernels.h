@@ -4994,11 +4994,11 @@ int backward_impl(const BwdCall& c) {
   reach.nseg = (int)cdiv(T, QSTAT_ROWS);
   reach.nkg = (int)cdiv(T, split ? TILE : NWAVES * TILE);
   if (c.reach) {
-    const BwdReachLayout RL = bwd_reach_layout(nseq, H, T, D);
+    reach.xk = exempt_apart(c.exempt);
+    const BwdReachLayout RL = bwd_reach_layout(nseq, H, T, D, reach.xk);
     reach.qstat = reinterpret_cast<float2*>(c.reach + RL.qstat);
     reach.hi = reinterpret_cast<int*>(c.reach + RL.hi);
     reach.xpart = reinterpret_cast<float*>(c.reach + RL.xpart);
-    reach.xk = c.exempt <= EXEMPT_APART ? c.exempt : 0;
   }
   const PrepLaunch prep{lse, dbar, ldt, reach};
   if constexpr (sizeof(elem) == 2) launch_rowprep_bf16(c, prep);

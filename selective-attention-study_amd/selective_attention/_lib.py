@@ -46,6 +46,7 @@ SIGNATURES = {
     "sa_timing_read": (_I, [_I, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_I64)]),
     "sa_forward_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I, _I]),
     "sa_reach_bytes": (_I64, [_I64, _I64, _I64, _I64, _I]),
+    "sa_backward_reach_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
     "sa_forward": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _I64,
                         _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _I, _I, _I, _I, _I64, _P]),
     "sa_forward_strided": (_I, [_P, _VS, _P, _VS, _P, _VS, _P, _P, _VS, _P, _P, _P, _P, _P, _I64, _P, _I64,

@@ -210,10 +210,10 @@ def _forward_scratch(lib, batch: int, heads: int, tk: int, kdim: int, code: int,
                + int(lib.sa_reach_bytes(batch, heads, tk, kdim, 0)), 1)
 
 
-def _backward_scratch(lib, batch: int, heads: int, seq: int, kdim: int, code: int, group: int) -> int:
+def _backward_scratch(lib, batch: int, heads: int, seq: int, kdim: int, code: int, group: int, exempt: int) -> int:
     """Bytes of sa_backward's workspace, the part for skipping tiles without weight included."""
     return (int(lib.sa_backward_workspace_bytes(batch, heads, seq, kdim, code, group))
-            + int(lib.sa_reach_bytes(batch, heads, seq, kdim, 1)))
+            + int(lib.sa_backward_reach_bytes(batch, heads, seq, kdim, exempt)))
 
 
 def _launch_forward(qs: Tensor, ks: Tensor, vs: Tensor, kstride: int, scale: float, exempt: int, group: int,
@@ -312,7 +312,7 @@ def _backward_impl(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, r
     code = _code_of(q)
     gdt = torch.bfloat16 if grad_bf16 else torch.float32
     dq, dk, dv = (torch.empty(q.shape, device=dev, dtype=gdt) for _ in range(3))
-    ws = torch.empty(_backward_scratch(lib, batch, heads, seq, kdim, code, group), device=dev, dtype=torch.uint8)
+    ws = torch.empty(_backward_scratch(lib, batch, heads, seq, kdim, code, group, exempt), device=dev, dtype=torch.uint8)
     with torch.cuda.device(dev):
         _lib.check(lib.sa_backward(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dout.data_ptr(), rmax.data_ptr(),
@@ -390,7 +390,7 @@ def _qkv_backward_impl(qkv: Tensor, dy: Tensor, out: Tensor, rmax: Tensor, rden:
     dev = qkv.device
     code, es = _code_of(qkv), qkv.element_size()
     dqkv = torch.empty_like(qkv)
-    ws = torch.empty(_backward_scratch(lib, batch, heads, seq, head_dim, code, 0), device=dev, dtype=torch.uint8)
+    ws = torch.empty(_backward_scratch(lib, batch, heads, seq, head_dim, code, 0, exempt), device=dev, dtype=torch.uint8)
     qkv_s, dy_s = _packed_strides(batch, seq, heads, head_dim)
     base, gbase = qkv.data_ptr(), dqkv.data_ptr()
     with torch.cuda.device(dev):

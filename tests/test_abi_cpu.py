@@ -291,3 +291,21 @@ def test_ops_are_not_passed_by_where_the_dispatcher_has_work():
         assert kernels._plain(x)
     with torch.inference_mode():
         assert kernels._plain(x, torch.ones(2))
+
+
+def test_scratch_for_left_out_tiles_follows_the_exempt_keys():
+    """Nothing where nothing is looked for (below 1024 keys); the exempt keys' partial gradients for as many as there
+    are, none where there are too many to be taken apart; sa_reach_bytes holds any number of them."""
+    lib = _lib.load()
+    for t in (1, 1023):
+        assert lib.sa_reach_bytes(2, 12, t, 64, 0) == lib.sa_reach_bytes(2, 12, t, 64, 1) == 0
+        assert lib.sa_backward_reach_bytes(2, 12, t, 64, 1) == 0
+    for t, d in ((1024, 32), (5003, 64), (16384, 128)):
+        most = lib.sa_reach_bytes(2, 12, t, d, 1)
+        sizes = [lib.sa_backward_reach_bytes(2, 12, t, d, x) for x in (33, 1, 2, 16, 32)]
+        assert sizes == sorted(sizes) and 0 < sizes[0] < sizes[1] and sizes[-1] == most
+        rows = 2 * 12 * ((t + 127) // 128)
+        assert sizes[1] - sizes[0] <= rows * 2 * d * 4 + 256   # one key's dK and dV per head and 128 rows
+        assert sizes[1] < most / 16
+        assert kernels._backward_scratch(lib, 2, 12, t, d, 0, 0, 1) == lib.sa_backward_workspace_bytes(2, 12, t, d, 0, 0) + sizes[1]
+    assert lib.sa_backward_reach_bytes(2, 12, 2048, 64, 0) == -1 and lib.sa_backward_reach_bytes(2, 12, 2048, 16, 1) == -1

@@ -98,7 +98,7 @@ def _backward(q, k, v, do, aux, exempt, reach, grad_bf16):
     code = kernels._code_of(q)
     out, rmax, rden, carry = aux
     grads = [torch.empty(q.shape, device=q.device, dtype=torch.bfloat16 if grad_bf16 else torch.float32) for _ in range(3)]
-    size = lib.sa_backward_workspace_bytes(b, h, t, d, code, 0) + (lib.sa_reach_bytes(b, h, t, d, 1) if reach else 0)
+    size = lib.sa_backward_workspace_bytes(b, h, t, d, code, 0) + (lib.sa_backward_reach_bytes(b, h, t, d, exempt) if reach else 0)
     # (the rows of the checkpoint planes that no sweep writes are read as NaN if anything takes them)
     ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=q.device)
     _lib.check(lib.sa_backward(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), rmax.data_ptr(),
