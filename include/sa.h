@@ -83,8 +83,10 @@ int64_t sa_forward_workspace_bytes(int64_t nseq, int64_t heads, int64_t tk, int6
 /* Optional bytes of scratch beyond sa_forward_workspace_bytes and sa_backward_workspace_bytes (-1 for
  * invalid sizes): given a workspace larger by this much, sa_forward and sa_backward leave out the tiles
  * whose softmax weights are exact fp32 zeros because their keys' history has outgrown every logit. The
- * results have the same bits with and without it, but for the gradients of at most 32 exempt keys, which
- * the backward then sums in another order. t: the number of keys (0 bytes below 1024, where nothing is
+ * forward's results have the same bits with and without it, and so have the backward's with more than 32 exempt
+ * keys. Up to 32 of them (the usual 1 included) the backward takes their dK and dV apart, in another order of
+ * summation, and the dK and dV of the first 128 keys and, at bf16 head dim 64, head 0's dQ agree to rounding;
+ * the rest has the same bits. t: the number of keys (0 bytes below 1024, where nothing is
  * looked for); backward: 0 for sa_forward's workspace, 1 for sa_backward's with any number of exempt keys.
  * sa_backward_reach_bytes: what sa_backward's workspace takes with `exempt` of them; less, the fewer of them up
  * to 32 (at one about a thirtieth of sa_reach_bytes' figure). */
@@ -107,8 +109,8 @@ int64_t sa_backward_reach_bytes(int64_t nseq, int64_t heads, int64_t t, int64_t 
  * layout); a prefill over a preallocated (nseq, heads, capacity, head_dim) cache passes
  * capacity * head_dim, so no prefix is copied. A multiple of 8.
  * scale: the logit scale s (the reference uses 1/sqrt(D); a caller that zero-pads D passes the
- * unpadded value). group: heads per wavefront (0 = automatic: at bf16 head dim 64 two, or one when
- * the two-head grid would fill the CUs only once; both give the same bits there); damp_mode 0 none, 1 linear, 2 sqrt scales F of
+ * unpadded value). group: heads per wavefront (0 = automatic: at bf16 head dims 32 and 64 two, or one when
+ * the two-head grid would fill the CUs only once; one and two give the same bits there, and four at 32); damp_mode 0 none, 1 linear, 2 sqrt scales F of
  * query i by min(1, train_len/(i+1)) (or its square root), reference kernels.py:179-182.
  * Limits (all entry points): one head's rows below 2 GiB ((t + 64) * row stride * element size
  * < 2^31; the row stride is head_dim here).

@@ -1,5 +1,6 @@
-"""Leaving out the tiles without weight keeps every bit: the C ABI called with the scratch that finds them
-(sa_reach_bytes) and without it, on inputs whose histories outgrow their logits, on inputs whose histories
+"""Leaving out the tiles without weight keeps the results: the C ABI called with the scratch that finds them
+(sa_reach_bytes) and without it -- every bit of the forward, and of the backward but for what the exempt
+keys' separate sums touch (_compare_backward) -- on inputs whose histories outgrow their logits, on inputs whose histories
 do not, and on inputs that are not finite or too large for the bound. The kernels' results against the
 oracle are the other tests' matter."""
 
@@ -116,15 +117,26 @@ def _compare_backward(q, k, v, do, exempt, half):
     first = 128 if exempt <= 32 else 0
     for x, y in zip(got[1:], want[1:]):
         assert torch.equal(_bits(x[:, :, first:]), _bits(y[:, :, first:])), exempt
+    # dQ: every bit, but for head 0 at bf16 head dim 64 beside keys taken apart. There a suffix sum of the first
+    # workgroup may round elsewhere, which can turn the bf16 rounding of an element of dz + g: 2e-7 of all of dQ
+    # and 1.3e-5 of a row seen
+    d64 = bf16 and q.shape[-1] == 64 and first
+    same = slice(1, None) if d64 else slice(None)
+    assert torch.equal(_bits(got[0][:, same]), _bits(want[0][:, same])), exempt
+    if d64:
+        x, y = got[0][:, 0].double(), want[0][:, 0].double()
+        rows = y.isfinite().all(-1)
+        off, size = (x - y)[rows].norm(dim=-1), y[rows].norm(dim=-1)
+        assert (off <= (2.0 ** -7 if half else 2.0 ** -13) * size).all(), exempt
+        assert off.norm() <= (2.0 ** -9 if half else 2.0 ** -20) * size.norm(), exempt
     if first == 0:
-        assert torch.equal(_bits(got[0]), _bits(want[0])), exempt
         return
     for x, y in zip(got, want):
         x, y = x.double(), y.double()
         assert torch.equal(x.isnan(), y.isnan())
         fine = y.isfinite()
-        # dQ: 1e-7 of fp32 rounding; dK, dV of the exempt keys: split bf16 operands (2^-16 each) or fp32
-        # products summed in another order; a bf16 gradient's own rounding beside that
+        # dK, dV of the exempt keys: split bf16 operands (2^-16 each) or fp32 products summed in another order;
+        # a bf16 gradient's own rounding beside that
         tol = 2.0 ** -8 if half else 2.0 ** -14 if bf16 else 2.0 ** -18
         assert (x - y)[fine].norm() <= tol * y[fine].norm() + 1e-30, exempt
 
@@ -135,7 +147,7 @@ def test_backward_keeps_its_bits(cuda, b, h, t, d, dtype, kind):
     """With more than 32 exempt keys the same instances of the kernels run: every bit. Up to 32 of them the
     exempt keys' dK, dV are summed by row segments, and the first 128 keys' tiles run an instance of their own,
     whose suffix sums the compiler may round elsewhere (one fp32 ulp seen, in head 0's dQ too): every bit of
-    the later keys' dK, dV, the rest to rounding."""
+    the later keys' dK, dV and of dQ but head 0's at bf16 head dim 64, the rest to rounding."""
     print(f"case backward {b} {h} {t} {d} {dtype} {kind}", flush=True)
     bf16 = dtype == "bf16"
     q, k, v, do = _inputs(cuda, b, h, t, d, torch.bfloat16 if bf16 else torch.float32, kind)
