@@ -47,7 +47,7 @@ STEP_FLOP = 7.0 * UNIT             # fwd 2 products + bwd 5 (FlashAttention conv
 # Products each timed kernel computes (recomputation included): the forward QK^T and PV; the
 # key-side backward QK^T, dO V^T, P^T dO, dz^T Q; the query-side backward QK^T, dO V^T, dz K.
 KERNEL_FLOP = {"forward": 2.0 * UNIT, "backward_kv": 4.0 * UNIT, "backward_dq": 3.0 * UNIT}
-# HBM bytes per launch of each kernel at this workload, measured with rocprofv3's FETCH_SIZE and
+# HBM bytes per launch of each kernel where every tile is computed, measured with rocprofv3's FETCH_SIZE and
 # WRITE_SIZE counters (one pass each) and scaled by a 1 GiB copy's readings (FETCH x 2.0, WRITE x
 # 1.0): profiles/c2_attention_kernels_traffic.md. The counters need the profiler, so bench.py
 # reports the committed measurement, labelled with the hash of the kernel sources it was taken on
@@ -55,10 +55,6 @@ KERNEL_FLOP = {"forward": 2.0 * UNIT, "backward_kv": 4.0 * UNIT, "backward_dq": 
 MEASURED_TRAFFIC_BYTES = {"forward": (2.0 * 460_700 + 67_588) * 1024,
                           "backward_kv": (2.0 * 330_872 + 391_687) * 1024,
                           "backward_dq": (2.0 * 352_457 + 96_256) * 1024}
-# C4 (131072-token prefill, 8 chunks): the forward kernel's HBM bytes per launch (mean over the
-# chunks, FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0) and MFMA busy fraction, measured with rocprofv3:
-# profiles/c4_prefill_kernels.md. The run's own per-launch time turns the bytes into a rate.
-MEASURED_C4 = {"hbm_bytes_per_launch": (2.0 * 3_288_204 + 67_584) * 1024, "mfma_busy": 0.35}
 # sha256 (first 16 hex digits) of csrc/sa_kernels.h when the figures above were profiled
 PROFILED_SOURCES = "686b814c501d5591"
 KERNEL_SOURCE = os.path.join(ROOT, "selective-attention-study_amd", "csrc", "sa_kernels.h")
@@ -251,8 +247,8 @@ def main() -> int:
                                       "whether a tile is computed or left out because its weights are exact zeros"},
         "every_tile": {"data": "the same, the selector's logits centred on -3: no tile is left out",
                        "ms_per_step": round(ms_every, 4), "tflops": round(STEP_FLOP / (ms_every * 1e-3) / 1e12, 2),
+                       "frac_of_peak": round(STEP_FLOP / (ms_every * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4),
                        "kernel_ms": {k_: round(v_, 4) for k_, v_ in every.items()}},
-        "frac_of_peak": round(tflops / PEAK_BF16_TFLOPS, 4),
         "kernel_ms": {k_: round(v_, 4) for k_, v_ in per_kernel.items()},
         "peak_mem_gib": round(peak_gib, 4),
         "roofline": {"bound": "mfma", "data": "every_tile",
@@ -279,12 +275,6 @@ def main() -> int:
         record["train_tok_s"] = round(record["train"]["d768"]["tokens_per_s"], 1)
     if not args.no_configs:
         c4 = harness.prefill_rate(reps=2, warmup=1)
-        c4["counters"] = {"source": dict(_profiled_label(), file="profiles/c4_prefill_kernels.md (rocprofv3 --pmc)"),
-                          "mfma_busy": MEASURED_C4["mfma_busy"],
-                          "hbm_bytes_per_launch": MEASURED_C4["hbm_bytes_per_launch"],
-                          "hbm_tb_s": MEASURED_C4["hbm_bytes_per_launch"] / (c4["per_layer_chunk_forward_ms"] * 1e9),
-                          "hbm_frac_of_peak": MEASURED_C4["hbm_bytes_per_launch"]
-                          / (c4["per_layer_chunk_forward_ms"] * 1e-3) / 8e12}
         record["c4"] = _rounded(c4)
         torch.cuda.empty_cache()
         _progress(f"C4 {record['c4']['tokens_per_s']:.0f} tok/s")
