@@ -1969,10 +1969,13 @@ __global__ __launch_bounds__(NTHREADS, G == 1 ? 3 : 2) void fwd64_kernel(
 // masked), dV += P^T dO and dK += dz^T Q with P and dz as split operands (hi + lo, as these sums run over
 // every query), the rows taken transposed from LDS. The wavefronts' sums add up in LDS, the workgroups' in
 // bwd_finish_kernel, both in a fixed order.
-// Bound by HBM (dO, O and Q once). Measured at B=1 H=16 T=16384 bf16: 25 us without exempt keys apart (5.4
-// TB/s), 33 us with one of them, 39 with 16.
+// ONE (xk = 1, the usual number): a matrix product of 32 columns for one key, and the rows' way through LDS for it,
+// cost as much again as what they overlapped with. Its logit and dO.v are two more row sums beside -dbar's, and
+// each lane adds P dO and dz q of its eight elements in registers.
+// Bound by HBM (dO, O and Q once). Measured at B=1 H=16 T=16384 bf16: 25 us with no or one exempt key apart (5.4
+// TB/s; one through the matrix products 33), 39 with 16; B=2 H=12 T=2048 9 us (12), fp32 B=1 H=8 T=2048 6 (11.5).
 
-template <class OP, int D>
+template <class OP, int D, bool ONE>
 __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 64 ? 4 : 2) : 1)) void bwd_rowprep_kernel(
     const typename OP::elem* __restrict__ q, const typename OP::elem* __restrict__ k,
     const typename OP::elem* __restrict__ v, const typename OP::elem* __restrict__ dout, Strides qs, Strides ks,
@@ -1987,10 +1990,15 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
   constexpr int LD = TR ? D : D + OP::KPAD;
   static_assert(QSTAT_ROWS == NWAVES * TILE, "a wavefront per row tile");
   constexpr int SUMLD = 2 * D + 4;   // floats of one key's dK and dV (padded: keys on shifted banks)
-  union Shared {
+  union Many {
     elem rows[NWAVES][2][TILE * LD];   // a wavefront's dO rows and Q rows
     float sum[NWAVES][8 * SUMLD];      // then its dK and dV sums of eight keys
   };
+  struct Single {
+    float sum[NWAVES * RPW][2 * D];           // dK and dV of the key over the rows of one lane group
+    float4 part[NTHREADS];                    // then over four of those
+  };
+  using Shared = typename std::conditional<ONE, Single, Many>::type;
   __shared__ __attribute__((aligned(16))) Shared sh;
   __shared__ __attribute__((aligned(16))) float sRow[NWAVES][2][TILE];   // a wavefront's rows' lse and -dbar
   __shared__ float sStat[NWAVES][2];
@@ -1999,7 +2007,7 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
   const int n = lane & 31, h = lane >> 5;
   const int r = blockIdx.y, seg = blockIdx.x;
   const int b = r / H, hh = r % H;
-  const int xk = reach.xk;
+  const int xk = ONE ? 1 : reach.xk;
   const int qbase = (seg * NWAVES + wave) * TILE;
   const int part = lane % LPR;
   const bool stats = reach.qstat != nullptr;
@@ -2021,12 +2029,23 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
 #pragma unroll
     for (int c = 0; c < (int)(sizeof(elem) / 2); ++c) {
       dr[p].u[c] = ds[c];
-      if (stats) qr[p].u[c] = qv[c];
+      if (ONE || stats) qr[p].u[c] = qv[c];
     }
     o4[p][0] = os[0];
     o4[p][1] = os[1];
     mv[p] = rmax[(int64_t)r * T + rr];
     nv[p] = rden[(int64_t)r * T + rr];
+  }
+  Row k0, v0;   // ONE: this lane's part of the key and its value
+  float dk0[8], dv0[8];
+  if constexpr (ONE) {
+#pragma unroll
+    for (int c = 0; c < (int)(sizeof(elem) / 2); ++c) {
+      k0.u[c] = reinterpret_cast<const uint4*>(k + ks.at(b, hh) + 8 * part)[c];
+      v0.u[c] = reinterpret_cast<const uint4*>(v + vs.at(b, hh) + 8 * part)[c];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dk0[e] = dv0[e] = 0.f;
   }
   float qmax = 0.f, lmin = INFINITY;
 #pragma unroll
@@ -2039,21 +2058,29 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
       for (int c = 0; c < (int)(sizeof(elem) / 2); ++c) dr[p].u[c] = qr[p].u[c] = make_uint4(0u, 0u, 0u, 0u);
     }
     const float ov[8] = {o4[p][0].x, o4[p][0].y, o4[p][0].z, o4[p][0].w, o4[p][1].x, o4[p][1].y, o4[p][1].z, o4[p][1].w};
-    float acc = 0.f, dd = 0.f, qq = 0.f;
+    float acc = 0.f, dd = 0.f, qq = 0.f, qk = 0.f, dov = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float d = OP::to_float(dr[p].e[e]);
       acc += d * ov[e];
-      if (stats) {
+      if (ONE || stats) {
         const float x = OP::to_float(qr[p].e[e]);
         dd = fmaf(d, d, dd);
         qq = fmaf(x, x, qq);
+        if constexpr (ONE) {
+          qk = fmaf(x, OP::to_float(k0.e[e]), qk);
+          dov = fmaf(d, OP::to_float(v0.e[e]), dov);
+        }
       }
     }
 #pragma unroll
     for (int o = LPR / 2; o > 0; o >>= 1) {
       acc += __shfl_xor(acc, o);
-      if (stats) {
+      if constexpr (ONE) {
+        qk += __shfl_xor(qk, o);
+        dov += __shfl_xor(dov, o);
+      }
+      if (ONE || stats) {
         dd += __shfl_xor(dd, o);
         qq += __shfl_xor(qq, o);
       }
@@ -2063,11 +2090,26 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
       lse[(int64_t)r * ldt + row] = lv;
       ndbar[(int64_t)r * ldt + row] = nd;
     }
-    if (stats && ok) {
+    if ((ONE || stats) && ok) {
       qmax = fmaxf(qmax, qq < REACH_NORM2 && dd < REACH_NORM2 && fabsf(nd) < REACH_NORM2 ? qq : INFINITY);
       lmin = fminf(lmin, fabsf(lv) < 3.0e38f ? lv : -INFINITY);
     }
-    if (xk > 0) {
+    if constexpr (ONE) {   // key 0 precedes every query
+      const float pr = fast_exp2(fmaf(qk, scale * LOG2E, -lv)), dz = pr * (dov + nd);
+      auto add = [&](float (&sum)[8], float x, const Row& y) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] = fmaf(x, OP::to_float(y.e[e]), sum[e]);
+      };
+      if constexpr (OP::SPLIT) {   // hi + lo as in the matrix products (the same results on infinite rows)
+        add(dv0, OP::to_float(OP::to_elem(pr)), dr[p]);
+        add(dv0, OP::to_float(OP::to_elem_lo(pr)), dr[p]);
+        add(dk0, OP::to_float(OP::to_elem(dz)), qr[p]);
+        add(dk0, OP::to_float(OP::to_elem_lo(dz)), qr[p]);
+      } else {
+        add(dv0, pr, dr[p]);
+        add(dk0, dz, qr[p]);
+      }
+    } else if (xk > 0) {
       if (part == 0) {
         sRow[wave][0][rl] = lv;
         sRow[wave][1][rl] = nd;
@@ -2080,7 +2122,7 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
       }
     }
   }
-  if (!stats) return;
+  if (!ONE && !stats) return;
 
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -2091,6 +2133,40 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
     sStat[wave][0] = qmax;
     sStat[wave][1] = lmin;
   }
+  auto store_stat = [&]() {   // (after a barrier)
+    if (tid != 0) return;
+    for (int w = 1; w < NWAVES; ++w) {
+      qmax = fmaxf(qmax, sStat[w][0]);
+      lmin = fminf(lmin, sStat[w][1]);
+    }
+    reach.qstat[(int64_t)r * reach.nseg + seg] = make_float2(sqrtf(qmax), lmin);
+  };
+  float4* dst = reinterpret_cast<float4*>(reach.xpart + ((int64_t)r * reach.nseg + seg) * xk * 2 * D);
+  if constexpr (ONE) {
+    // the key's sums: a lane's rows, then four lane groups at a time, then those
+    constexpr int QUADS = 2 * D / 4, SLICES = NTHREADS / QUADS;
+    static_assert(NWAVES * RPW == 4 * SLICES, "four lane groups per thread");
+    float4* mine = reinterpret_cast<float4*>(sh.sum[wave * RPW + lane / LPR]) + 2 * part;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      mine[c] = make_float4(dk0[4 * c], dk0[4 * c + 1], dk0[4 * c + 2], dk0[4 * c + 3]);
+      mine[D / 4 + c] = make_float4(dv0[4 * c], dv0[4 * c + 1], dv0[4 * c + 2], dv0[4 * c + 3]);
+    }
+    __syncthreads();
+    store_stat();
+    const int quad = tid % QUADS, slice = tid / QUADS;
+    auto add = [](const float4& x, const float4& y) { return make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w); };
+    float4 x = reinterpret_cast<const float4*>(sh.sum[4 * slice])[quad];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) x = add(x, reinterpret_cast<const float4*>(sh.sum[4 * slice + i])[quad]);
+    sh.part[tid] = x;
+    __syncthreads();
+    if (slice != 0) return;
+#pragma unroll
+    for (int i = 1; i < SLICES; ++i) x = add(x, sh.part[i * QUADS + quad]);
+    dst[quad] = x;
+    return;
+  } else {
   f32x16 dkx[DB], dvx[DB];
   if (xk > 0) {
     // the first keys and values (B operands: lane = key), and the rows as A operands (lane = query row). The
@@ -2169,15 +2245,8 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
     acc_t(dkx, 1, dz);
   }
   __syncthreads();
-  if (tid == 0) {
-    for (int w = 1; w < NWAVES; ++w) {
-      qmax = fmaxf(qmax, sStat[w][0]);
-      lmin = fminf(lmin, sStat[w][1]);
-    }
-    reach.qstat[(int64_t)r * reach.nseg + seg] = make_float2(sqrtf(qmax), lmin);
-  }
+  store_stat();
   if (xk == 0) return;
-  float4* dst = reinterpret_cast<float4*>(reach.xpart + ((int64_t)r * reach.nseg + seg) * xk * 2 * D);
   for (int j0 = 0; j0 < xk; j0 += 8) {   // (every wavefront is past its reads of the rows)
     if (n >= j0 && n < min(j0 + 8, xk)) {
       float* mine = &sh.sum[wave][(n - j0) * SUMLD];
@@ -2205,6 +2274,7 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
       dst[j0 * (2 * D / 4) + i] = x;
     }
     __syncthreads();
+  }
   }
 }
 
@@ -4861,10 +4931,14 @@ int forward_impl(const FwdCall& c) {
 template <class OP, int D>
 void launch_rowprep(const BwdCall& c, const PrepLaunch& p) {
   using elem = typename OP::elem;
-  hipLaunchKernelGGL((bwd_rowprep_kernel<OP, D>), dim3((unsigned)cdiv(p.ldt, QSTAT_ROWS), (unsigned)(c.nseq * c.H)),
-                     dim3(NTHREADS), 0, c.st, static_cast<const elem*>(c.q), static_cast<const elem*>(c.k),
-                     static_cast<const elem*>(c.v), static_cast<const elem*>(c.dout), c.qs, c.ks, c.vs, c.dos, c.H, c.T,
-                     c.out, c.rmax, c.rden, p.lse, p.ndbar, p.ldt, c.scale, p.reach);
+#define SA_LAUNCH_PREP(ONE)                                                                                        \
+  hipLaunchKernelGGL((bwd_rowprep_kernel<OP, D, ONE>), dim3((unsigned)cdiv(p.ldt, QSTAT_ROWS), (unsigned)(c.nseq * c.H)), \
+                     dim3(NTHREADS), 0, c.st, static_cast<const elem*>(c.q), static_cast<const elem*>(c.k),              \
+                     static_cast<const elem*>(c.v), static_cast<const elem*>(c.dout), c.qs, c.ks, c.vs, c.dos, c.H, c.T, \
+                     c.out, c.rmax, c.rden, p.lse, p.ndbar, p.ldt, c.scale, p.reach)
+  if (p.reach.xk == 1) SA_LAUNCH_PREP(true);
+  else SA_LAUNCH_PREP(false);
+#undef SA_LAUNCH_PREP
 }
 
 // Launch of the key-side kernel from its arguments (the grid as launch_bwd's).
