@@ -802,8 +802,8 @@ constexpr int REACH_RUNS = 64;   // entries of the list
 template <bool REST>
 __device__ __forceinline__ void write_reach_runs(TileRun* runs, const uint64_t* words, int nwords, int first, int lane) {
   int n = 0;
-  bool full = false;
   TileRun open{-1, -1};
+  bool more = first > 0;   // (not REST)
   auto add = [&](int hi, int lo) {
     if (open.hi >= 0 && hi == open.lo - 1) {
       open.lo = lo;
@@ -832,17 +832,20 @@ __device__ __forceinline__ void write_reach_runs(TileRun* runs, const uint64_t* 
       add(first + 64 * w + bit, first + 64 * w + bit - len + 1);
       word &= (bit - len >= 0) ? (2ull << (bit - len)) - 1 : 0;
       if (n == REACH_RUNS - 2) {   // full, with the open run and the ending
-        if (REST) open.lo = 0;
-        full = true;
+        if constexpr (REST) open.lo = 0;
+        else more = true;
         word = 0;
         w = 0;
+        first = 0;
       }
     }
   }
-  if (REST && !full && first > 0) add(first - 1, 0);
+  if constexpr (REST) {
+    if (first > 0) add(first - 1, 0);
+  }
   if (lane == 0) {
     if (open.hi >= 0) runs[n++] = open;
-    runs[n] = {!REST && (full || first > 0) ? -2 : -1, INT_MIN};
+    runs[n] = {!REST && more ? -2 : -1, INT_MIN};
   }
 }
 
