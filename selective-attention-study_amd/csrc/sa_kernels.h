@@ -1512,6 +1512,25 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
         run_lo = __builtin_amdgcn_readfirstlane(r.lo);
       }
     };
+    // tiles from cur down to `stop`; those inside a run in a loop of their own, in which the compiler sees that
+    // they follow each other (head dim 128, B=1 H=16, 256 queries over 16384 keys, no tile left out: 687 us, 732
+    // with every tile's addresses anew)
+    auto run = [&](int stop, auto interior_tag) {
+      while (cur >= stop) {
+        if (nxt == cur - 1) {
+          const int lim = max(max(stop, 1), run_lo + 2);
+          for (; cur >= lim; --cur, ++t) {
+            nxt = cur - 1;
+            tile_step(interior_tag, damp_tag);
+          }
+          nxt = cur - 1;
+        }
+        if (cur >= stop) {
+          tile_step(interior_tag, damp_tag);
+          shift();
+        }
+      }
+    };
     for (; cur >= i_hi; shift()) tile_step(std::false_type{}, damp_tag);
     nxt = cut - 1;   // the tiles below cut: all of them, or the runs found
     if (reach_worth(oldest)) {
@@ -1521,7 +1540,7 @@ __global__ __launch_bounds__(NTHREADS, (fwd_min_blocks<OP, D, G>())) void fwd_ke
       nxt = __builtin_amdgcn_readfirstlane(r.hi);
       run_lo = __builtin_amdgcn_readfirstlane(r.lo);
     }
-    for (; cur >= i_lo; shift()) tile_step(std::true_type{}, damp_tag);
+    run(i_lo, std::true_type{});
     for (; cur >= 0; shift()) tile_step(std::false_type{}, damp_tag);
   };
   if (damp_mode != 0) sweep(std::true_type{});
