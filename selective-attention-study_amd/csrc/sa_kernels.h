@@ -701,6 +701,7 @@ __device__ __forceinline__ float block_selection_sum(const f32x16& acc, bool int
 // one pair in a hundred is selected and nothing can be left out: B=2 H=12 T=5003 249 -> 250 us, B=1 H=12
 // T=16384 740 -> 751 us, and the key norms add 2 and 6 us to the column sums' launch.
 constexpr float REACH_ZERO = 132.f;
+constexpr float REACH_WORTH = REACH_ZERO - 16.f;   // a total (log2 units) from which looking for tiles can pay
 constexpr float REACH_NORM2 = 1e37f;      // sums of squares at or past this count as not finite
 constexpr float REACH_Q = 1.01f * LOG2E;
 constexpr float REACH_F = 0.999f * LOG2E;
@@ -730,21 +731,29 @@ __device__ __forceinline__ float sumsq8(const E* p) {
 }
 
 // kn[r][kt] = max |k_j| over the keys of tile kt of head r = b * H + head, infinity when a key or a
-// value of the tile is not finite (or too large, REACH_NORM2). Workgroup `blk` takes NORM_KEYS keys of
+// value of the tile is not finite (or too large, REACH_NORM2), and, unread, for the tiles that no query is likely
+// to leave out: wanted(kt), for the lane half's tile, false (only the time depends on it). Workgroup `blk` takes NORM_KEYS keys of
 // head r: a wavefront two tiles, D/8 lanes per row, a tile's loads all issued before their use. Bound
 // by HBM (each key and value read once).
-template <typename E, int D>
+template <typename E, int D, class Wanted>
 __device__ __forceinline__ void key_norms_block(const E* k, const E* v, const Strides& ks, const Strides& vs, int H,
-                                                int Tk, float* kn, int r, int blk) {
+                                                int Tk, float* kn, int r, int blk, Wanted wanted) {
   constexpr int LPR = D / 8, RPW = 64 / LPR, PASSES = TILE / RPW;
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int NKT = (Tk + TILE - 1) / TILE;
   const E* kh = k + ks.at(r / H, r % H) + (lane % LPR) * 8;
   const E* vh = v + vs.at(r / H, r % H) + (lane % LPR) * 8;
+  const int kt0 = blk * (NORM_KEYS / TILE) + wave * 2;
+  if (kt0 >= NKT) return;
+  const uint64_t want = __ballot(wanted(min(kt0 + (lane >> 5), NKT - 1)));
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const int kt = blk * (NORM_KEYS / TILE) + wave * 2 + u;
+    const int kt = kt0 + u;
     if (kt >= NKT) break;
+    if (((want >> (32 * u)) & 1) == 0) {
+      if (lane == 0) kn[(int64_t)r * NKT + kt] = INFINITY;
+      continue;
+    }
     float sk[PASSES], sv[PASSES];
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
@@ -768,10 +777,14 @@ __device__ __forceinline__ void key_norms_block(const E* k, const E* v, const St
   }
 }
 
+// The norms in a launch of their own, after the selection: of the tiles whose least total (kt_min) is enough.
 template <typename E, int D>
 __global__ __launch_bounds__(NTHREADS) void key_norms_kernel(const E* __restrict__ k, const E* __restrict__ v, Strides ks,
-                                                             Strides vs, int H, int Tk, float* __restrict__ kn) {
-  key_norms_block<E, D>(k, v, ks, vs, H, Tk, kn, blockIdx.y, blockIdx.x);
+                                                             Strides vs, int H, int Tk, float* __restrict__ kn,
+                                                             const float* __restrict__ kt_min) {
+  const float* totals = kt_min + (int64_t)(blockIdx.y / H) * ((Tk + TILE - 1) / TILE);
+  key_norms_block<E, D>(k, v, ks, vs, H, Tk, kn, blockIdx.y, blockIdx.x,
+                        [&](int kt) { return totals[kt] * LOG2E > REACH_WORTH; });
 }
 
 // The maximum over the 32 lanes of each half-wavefront (those of them that are active).
@@ -855,7 +868,7 @@ __device__ __forceinline__ void write_reach_runs(TileRun* runs, const uint64_t* 
 __device__ __forceinline__ float reach_total(const float* kt_min, int ntiles, int lane) {
   return kt_min != nullptr && lane < ntiles ? kt_min[lane] : 0.f;
 }
-__device__ __forceinline__ bool reach_worth(float total) { return __any(total * LOG2E > REACH_ZERO - 16.f); }
+__device__ __forceinline__ bool reach_worth(float total) { return __any(total * LOG2E > REACH_WORTH); }
 
 // Sum of squares of a lane's part of its query row.
 template <class OP, int NS>
@@ -953,12 +966,24 @@ template <class OP, int D>
 __global__ __launch_bounds__(NTHREADS) void sel_colsum_kernel(
     const typename OP::elem* __restrict__ q, const typename OP::elem* __restrict__ k,
     float* __restrict__ colsum, int H, int Tq, int Tk, Strides qs, Strides ks, int q_off, int exempt, float scale,
-    int RB, const typename OP::elem* __restrict__ v, Strides vs, int nseq, float* __restrict__ kn) {
+    int RB, const typename OP::elem* __restrict__ v, Strides vs, int nseq, float* __restrict__ kn,
+    const float* __restrict__ state_in, int64_t state_ld) {
   using elem = typename OP::elem;
   if ((int)blockIdx.z >= nseq) {
     const int nkb = (Tk + NORM_KEYS - 1) / NORM_KEYS;
     const int64_t e = ((int64_t)(blockIdx.z - nseq) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    if (e < (int64_t)nseq * H * nkb) key_norms_block<elem, D>(k, v, ks, vs, H, Tk, kn, (int)(e / nkb), (int)(e % nkb));
+    if (e >= (int64_t)nseq * H * nkb) return;
+    const int r = (int)(e / nkb);
+    // The totals are not known yet. Of a tile before the chunk, what its keys have received is, and with it about
+    // what the chunk's queries will add: half as much again per query as so far, to be on the safe side. At head
+    // dim 128, where it pays: B=1 H=16, 256 queries over 16384 keys, nothing left out 693 -> 676 us, most left out
+    // 74.9 -> 75.2; at 64 (half the bytes) 461 -> 457 and 36.8 -> 38.0.
+    key_norms_block<elem, D>(k, v, ks, vs, H, Tk, kn, r, (int)(e % nkb), [&](int kt) {
+      const int age = q_off - kt * TILE;   // the queries the tile's first key has seen, and itself
+      if (D < 128 || state_in == nullptr || age < NORM_KEYS) return true;
+      const float least = -half_max(-state_in[(int64_t)(r / H) * state_ld + kt * TILE + (threadIdx.x & 31)]);
+      return least * (1.f + 1.5f * (float)Tq / (float)age) * LOG2E > REACH_WORTH;
+    });
     return;
   }
   using frag = typename OP::frag;
@@ -4851,7 +4876,7 @@ int run_selection(const FwdCall& c, hipStream_t st) {
   TimedLaunch timed(SA_KERNEL_SELECTION, st);
   auto norms_apart = [&]() {
     hipLaunchKernelGGL((key_norms_kernel<elem, D>), dim3((unsigned)nkb, (unsigned)(c.nseq * c.H)), dim3(NTHREADS), 0, st,
-                       static_cast<const elem*>(c.k), static_cast<const elem*>(c.v), c.ks, c.vs, c.H, c.Tk, c.kn);
+                       static_cast<const elem*>(c.k), static_cast<const elem*>(c.v), c.ks, c.vs, c.H, c.Tk, c.kn, c.kt);
   };
   if constexpr (sizeof(elem) == 2 && D == 64) {
     const int64_t wgs = cdiv(NKT, NWAVES * SEL_CARRY_KPW);
@@ -4870,13 +4895,13 @@ int run_selection(const FwdCall& c, hipStream_t st) {
   const int64_t znorms = c.kn ? cdiv((int64_t)c.nseq * c.H * nkb, (int64_t)g1.x * g1.y) : 0;
   const bool norms_along = c.nseq + znorms <= 65535;
   if (norms_along) g1.z += (unsigned)znorms;
-  else norms_apart();
   hipLaunchKernelGGL((sel_colsum_kernel<OP, D>), g1, dim3(NTHREADS), 0, st, static_cast<const elem*>(c.q),
                      static_cast<const elem*>(c.k), c.carry, c.H, c.Tq, c.Tk, c.qs, c.ks, c.q_off, c.exempt, c.scale,
-                     RB, static_cast<const elem*>(c.v), c.vs, c.nseq, c.kn);
+                     RB, static_cast<const elem*>(c.v), c.vs, c.nseq, c.kn, c.q_off > 0 ? c.state_in : nullptr, c.state_ld);
   dim3 g2((unsigned)cdiv(c.Tk, NTHREADS), (unsigned)c.nseq);
   hipLaunchKernelGGL(sel_scan_kernel, g2, dim3(NTHREADS), 0, st, c.carry, c.state_in, c.state_out, c.state_ld, NBq,
                      c.Tk, c.q_off, c.kt);
+  if (!norms_along) norms_apart();
   return launch_status();
 }
 
