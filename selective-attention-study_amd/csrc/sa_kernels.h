@@ -731,10 +731,10 @@ __device__ __forceinline__ float sumsq8(const E* p) {
 }
 
 // kn[r][kt] = max |k_j| over the keys of tile kt of head r = b * H + head, infinity when a key or a
-// value of the tile is not finite (or too large, REACH_NORM2), and, unread, for the tiles that no query is likely
-// to leave out: wanted(kt), for the lane half's tile, false (only the time depends on it). Workgroup `blk` takes NORM_KEYS keys of
-// head r: a wavefront two tiles, D/8 lanes per row, a tile's loads all issued before their use. Bound
-// by HBM (each key and value read once).
+// value of the tile is not finite (or too large, REACH_NORM2), and, unread, for the tiles that no query is
+// likely to leave out: wanted(kt), asked of the lane half's tile, false (only the time depends on it).
+// Workgroup `blk` takes NORM_KEYS keys of head r: a wavefront two tiles, D/8 lanes per row, a tile's loads
+// all issued before their use. Bound by HBM (each key and value read once).
 template <typename E, int D, class Wanted>
 __device__ __forceinline__ void key_norms_block(const E* k, const E* v, const Strides& ks, const Strides& vs, int H,
                                                 int Tk, float* kn, int r, int blk, Wanted wanted) {
@@ -2214,114 +2214,114 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
     dst[quad] = x;
     return;
   } else {
-  f32x16 dkx[DB], dvx[DB];
-  if (xk > 0) {
-    // the first keys and values (B operands: lane = key), and the rows as A operands (lane = query row). The
-    // fp32 products run over the head dim with lane half h at elements [h D/2, (h+1) D/2), so that both load
-    // as 16-byte pieces.
-    const elem* kh = k + ks.at(b, hh) + (int64_t)min(n, T - 1) * ks.row;   // (columns from xk on are masked)
-    const elem* vh = v + vs.at(b, hh) + (int64_t)min(n, T - 1) * vs.row;
-    constexpr int PIECES = sizeof(elem) == 2 ? NS : D / 8;
-    constexpr int STEP = sizeof(elem) == 2 ? 16 : 4;   // elements between a lane's pieces
-    const int at = sizeof(elem) == 2 ? 8 * h : h * (D / 2);
-    uint4 kx[PIECES], vx[PIECES];
+    f32x16 dkx[DB], dvx[DB];
+    if (xk > 0) {
+      // the first keys and values (B operands: lane = key), and the rows as A operands (lane = query row). The
+      // fp32 products run over the head dim with lane half h at elements [h D/2, (h+1) D/2), so that both load
+      // as 16-byte pieces.
+      const elem* kh = k + ks.at(b, hh) + (int64_t)min(n, T - 1) * ks.row;   // (columns from xk on are masked)
+      const elem* vh = v + vs.at(b, hh) + (int64_t)min(n, T - 1) * vs.row;
+      constexpr int PIECES = sizeof(elem) == 2 ? NS : D / 8;
+      constexpr int STEP = sizeof(elem) == 2 ? 16 : 4;   // elements between a lane's pieces
+      const int at = sizeof(elem) == 2 ? 8 * h : h * (D / 2);
+      uint4 kx[PIECES], vx[PIECES];
 #pragma unroll
-    for (int s = 0; s < PIECES; ++s) {
-      kx[s] = *reinterpret_cast<const uint4*>(kh + at + STEP * s);
-      vx[s] = *reinterpret_cast<const uint4*>(vh + at + STEP * s);
-    }
-#pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      dkx[db] = zero16();
-      dvx[db] = zero16();
-    }
-    lds_wave_sync();
-    auto piece = [&](int x, int s) -> uint4 {
-      const elem* y = sh.rows[wave][x];
-      if constexpr (TR) return *reinterpret_cast<const uint4*>(y + swzq(n, 2 * s + h));
-      else return *reinterpret_cast<const uint4*>(y + n * LD + at + STEP * s);
-    };
-    auto mma_piece = [&](const uint4& a, const uint4& b4, f32x16 c) -> f32x16 {
-      if constexpr (sizeof(elem) == 2) {
-        return OP::mma(*reinterpret_cast<const frag*>(&a), *reinterpret_cast<const frag*>(&b4), c);
-      } else {
-        c = OP::mma(__uint_as_float(a.x), __uint_as_float(b4.x), c);
-        c = OP::mma(__uint_as_float(a.y), __uint_as_float(b4.y), c);
-        c = OP::mma(__uint_as_float(a.z), __uint_as_float(b4.z), c);
-        return OP::mma(__uint_as_float(a.w), __uint_as_float(b4.w), c);
+      for (int s = 0; s < PIECES; ++s) {
+        kx[s] = *reinterpret_cast<const uint4*>(kh + at + STEP * s);
+        vx[s] = *reinterpret_cast<const uint4*>(vh + at + STEP * s);
       }
-    };
-    // acc[db] (D x keys) += Y^T X: Y the wavefront's rows, X a (queries x keys) tile
-    auto acc_t = [&](f32x16 (&acc)[DB], int which, const f32x16& x) {
-      const elem* y = sh.rows[wave][which];
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+      for (int db = 0; db < DB; ++db) {
+        dkx[db] = zero16();
+        dvx[db] = zero16();
+      }
+      lds_wave_sync();
+      auto piece = [&](int x, int s) -> uint4 {
+        const elem* y = sh.rows[wave][x];
+        if constexpr (TR) return *reinterpret_cast<const uint4*>(y + swzq(n, 2 * s + h));
+        else return *reinterpret_cast<const uint4*>(y + n * LD + at + STEP * s);
+      };
+      auto mma_piece = [&](const uint4& a, const uint4& b4, f32x16 c) -> f32x16 {
+        if constexpr (sizeof(elem) == 2) {
+          return OP::mma(*reinterpret_cast<const frag*>(&a), *reinterpret_cast<const frag*>(&b4), c);
+        } else {
+          c = OP::mma(__uint_as_float(a.x), __uint_as_float(b4.x), c);
+          c = OP::mma(__uint_as_float(a.y), __uint_as_float(b4.y), c);
+          c = OP::mma(__uint_as_float(a.z), __uint_as_float(b4.z), c);
+          return OP::mma(__uint_as_float(a.w), __uint_as_float(b4.w), c);
+        }
+      };
+      // acc[db] (D x keys) += Y^T X: Y the wavefront's rows, X a (queries x keys) tile
+      auto acc_t = [&](f32x16 (&acc)[DB], int which, const f32x16& x) {
+        const elem* y = sh.rows[wave][which];
 #pragma unroll
-        for (int s = 0; s < AS; ++s) {
-          frag yt;
-          if constexpr (TR) {
-            yt = get_trq<true>(y, lane, db, s);
-          } else if constexpr (sizeof(elem) == 2) {
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const elem raw = y[(16 * s + 8 * (e >> 2) + 4 * h + (e & 3)) * LD + db * 32 + n];
-              yt[e] = *reinterpret_cast<const bf16_t*>(&raw);
+          for (int s = 0; s < AS; ++s) {
+            frag yt;
+            if constexpr (TR) {
+              yt = get_trq<true>(y, lane, db, s);
+            } else if constexpr (sizeof(elem) == 2) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                const elem raw = y[(16 * s + 8 * (e >> 2) + 4 * h + (e & 3)) * LD + db * 32 + n];
+                yt[e] = *reinterpret_cast<const bf16_t*>(&raw);
+              }
+            } else {
+              yt = y[crow(s, h) * LD + db * 32 + n];
             }
-          } else {
-            yt = y[crow(s, h) * LD + db * 32 + n];
+            acc[db] = OP::mma(yt, OP::from_acc(x, s), acc[db]);
+            if constexpr (OP::SPLIT) acc[db] = OP::mma(yt, OP::from_acc_lo(x, s), acc[db]);
           }
-          acc[db] = OP::mma(yt, OP::from_acc(x, s), acc[db]);
-          if constexpr (OP::SPLIT) acc[db] = OP::mma(yt, OP::from_acc_lo(x, s), acc[db]);
-        }
-    };
-    f32x16 p = zero16(), dz = rows16(sRow[wave][1], h);
+      };
+      f32x16 p = zero16(), dz = rows16(sRow[wave][1], h);
 #pragma unroll
-    for (int s = 0; s < PIECES; ++s) {
-      p = mma_piece(piece(1, s), kx[s], p);
-      dz = mma_piece(piece(0, s), vx[s], dz);
-    }
-    const f32x16 ls = rows16(sRow[wave][0], h);
-    const float sl2 = scale * LOG2E;
-    const int thr = n < xk ? n - qbase - 4 * h : 32;   // key n <= query qbase + crow(i, h)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      p[i] = crow(i, 0) >= thr ? fast_exp2(fmaf(p[i], sl2, -ls[i])) : 0.f;
-      dz[i] = p[i] * dz[i];
-    }
-    acc_t(dvx, 0, p);
-    acc_t(dkx, 1, dz);
-  }
-  __syncthreads();
-  store_stat();
-  if (xk == 0) return;
-  for (int j0 = 0; j0 < xk; j0 += 8) {   // (every wavefront is past its reads of the rows)
-    if (n >= j0 && n < min(j0 + 8, xk)) {
-      float* mine = &sh.sum[wave][(n - j0) * SUMLD];
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int d = db * 32 + 8 * a + 4 * h;
-          *reinterpret_cast<float4*>(mine + d) =
-              make_float4(dkx[db][4 * a], dkx[db][4 * a + 1], dkx[db][4 * a + 2], dkx[db][4 * a + 3]);
-          *reinterpret_cast<float4*>(mine + D + d) =
-              make_float4(dvx[db][4 * a], dvx[db][4 * a + 1], dvx[db][4 * a + 2], dvx[db][4 * a + 3]);
-        }
-    }
-    __syncthreads();
-    const int quads = min(8, xk - j0) * (2 * D / 4);
-    for (int i = tid; i < quads; i += NTHREADS) {
-      const int at = (i / (2 * D / 4)) * SUMLD + 4 * (i % (2 * D / 4));
-      float4 x = *reinterpret_cast<const float4*>(&sh.sum[0][at]);
-#pragma unroll
-      for (int w = 1; w < NWAVES; ++w) {
-        const float4 y = *reinterpret_cast<const float4*>(&sh.sum[w][at]);
-        x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+      for (int s = 0; s < PIECES; ++s) {
+        p = mma_piece(piece(1, s), kx[s], p);
+        dz = mma_piece(piece(0, s), vx[s], dz);
       }
-      dst[j0 * (2 * D / 4) + i] = x;
+      const f32x16 ls = rows16(sRow[wave][0], h);
+      const float sl2 = scale * LOG2E;
+      const int thr = n < xk ? n - qbase - 4 * h : 32;   // key n <= query qbase + crow(i, h)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        p[i] = crow(i, 0) >= thr ? fast_exp2(fmaf(p[i], sl2, -ls[i])) : 0.f;
+        dz[i] = p[i] * dz[i];
+      }
+      acc_t(dvx, 0, p);
+      acc_t(dkx, 1, dz);
     }
     __syncthreads();
-  }
+    store_stat();
+    if (xk == 0) return;
+    for (int j0 = 0; j0 < xk; j0 += 8) {   // (every wavefront is past its reads of the rows)
+      if (n >= j0 && n < min(j0 + 8, xk)) {
+        float* mine = &sh.sum[wave][(n - j0) * SUMLD];
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int a = 0; a < 4; ++a) {
+            const int d = db * 32 + 8 * a + 4 * h;
+            *reinterpret_cast<float4*>(mine + d) =
+                make_float4(dkx[db][4 * a], dkx[db][4 * a + 1], dkx[db][4 * a + 2], dkx[db][4 * a + 3]);
+            *reinterpret_cast<float4*>(mine + D + d) =
+                make_float4(dvx[db][4 * a], dvx[db][4 * a + 1], dvx[db][4 * a + 2], dvx[db][4 * a + 3]);
+          }
+      }
+      __syncthreads();
+      const int quads = min(8, xk - j0) * (2 * D / 4);
+      for (int i = tid; i < quads; i += NTHREADS) {
+        const int at = (i / (2 * D / 4)) * SUMLD + 4 * (i % (2 * D / 4));
+        float4 x = *reinterpret_cast<const float4*>(&sh.sum[0][at]);
+#pragma unroll
+        for (int w = 1; w < NWAVES; ++w) {
+          const float4 y = *reinterpret_cast<const float4*>(&sh.sum[w][at]);
+          x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+        }
+        dst[j0 * (2 * D / 4) + i] = x;
+      }
+      __syncthreads();
+    }
   }
 }
 
