@@ -2325,59 +2325,94 @@ __global__ __launch_bounds__(NTHREADS, (sizeof(typename OP::elem) == 2 ? (D <= 6
   }
 }
 
-// (Measured, N(0,1) inputs, B=1 H=16 T=16384 bf16: the key side 1560 -> 190 us, the query side 1510 -> 203 us.)
+// What a key-side wavefront's search reads first, loaded before its key rows so that the search adds no wait of
+// its own to them: the carry of its first round of probes (kv_last_block), and two of the head's row segments
+// per lane. (Key side, us, the search's loads behind the key rows / before them: B=1 H=16 T=16384 bf16, most tiles
+// left out 185 / 176; B=1 H=12 T=16384, none left out 1371 / 1367; fp32 B=1 H=8 T=2048, none 377 / 371.)
+struct KvProbe {
+  float f[4];
+  float2 q[2];
+};
+// The query block of a lane group's first probe: the last one, where nothing can be left out all there is to know,
+// and, for the usual reach of a few tiles, the blocks 2, 4, ... 128 on.
+__device__ __forceinline__ int kv_first_probe(int key0, int i, int NB) {
+  return i == 7 ? NB - 1 : min(key0 / TILE + (2 << i), NB - 1);
+}
+__device__ __forceinline__ KvProbe kv_probe(const BwdReach& reach, int64_t r, const float* carry_b, int T, int NB,
+                                            int key0, int lane) {
+  KvProbe x{};
+  if (reach.qstat) {
+    const float* p = carry_b + (int64_t)kv_first_probe(key0, lane >> 3, NB) * T;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.f[e] = p[min(key0 + 4 * (lane & 7) + e, T - 1)];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x.q[i] = reach.qstat[r * reach.nseg + min(lane + 64 * i, reach.nseg - 1)];
+  }
+  return x;
+}
+
+// Whether the search can find anything: every key of the wavefront (but those that do not count) has received
+// enough before the last query block. Only the time depends on the answer (see reach_worth).
+__device__ __forceinline__ bool kv_worth(const KvProbe& x, int key0, int T, int xk, int lane) {
+  bool ok = true;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int j = key0 + 4 * (lane & 7) + e;
+    ok = ok && (j >= T || j < xk || x.f[e] * LOG2E > REACH_WORTH);
+  }
+  return __all(lane < 56 || ok);
+}
+
+// (Measured, N(0,1) inputs, B=1 H=16 T=16384 bf16: the key side 1560 -> 176 us, the query side 1510 -> 203 us.)
 // The last query block on which some key of a wavefront's 32 (from key0) keeps a weight that is not an
 // exact zero, of the blocks up to NB - 1 (the key tile's own block at least): a lane group of 8 probes one
 // block (4 keys per lane), eight blocks at a time; the history never falls, so the blocks past the last
 // one are all without weight. thr: see find_reach, with the head's least lse for the row maxima. Keys
 // below xk (their gradients are taken elsewhere) and past the end do not count.
-__device__ __forceinline__ int kv_last_block(const float* carry_b, int T, int NB, int key0, int xk, float thr,
-                                             int lane) {
+__device__ __forceinline__ int kv_last_block(const KvProbe& first, const float* carry_b, int T, int NB, int key0, int xk,
+                                             float thr, int lane) {
   const int part = lane >> 3, j0 = key0 + 4 * (lane & 7);
-  auto gone = [&](int qb) {   // (qb < NB; lanes of a probe past the interval read a block inside it)
-    const float* p = carry_b + (int64_t)qb * T;
+  auto gone = [&](const float (&f)[4]) {
     bool ok = thr < INFINITY;   // every comparison that meets a NaN keeps the block
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int j = j0 + e;
-      const float f = p[min(j, T - 1)];
-      ok = ok && (j >= T || j < xk || f * REACH_F > thr);
-    }
+    for (int e = 0; e < 4; ++e) ok = ok && (j0 + e >= T || j0 + e < xk || f[e] * REACH_F > thr);
     return ok;
   };
   int lo = key0 / TILE, hi = NB;   // lo: kept; hi: without weight (or past the end)
-  auto narrow = [&](auto probe) {   // probe(i), i = 0..7, ascending
-    const uint64_t m = __ballot(gone(min(probe(part), NB - 1)));
+  auto narrow = [&](const float (&f)[4], auto probe) {   // f: the lane's carry at probe(part); probe(i), i = 0..7, ascending
+    const uint64_t m = __ballot(gone(f));
     int nlo = lo, nhi = hi;
 #pragma unroll
     for (int i = 7; i >= 0; --i) {
-      const int p = min(probe(i), NB - 1);
+      const int p = probe(i);
       if (((m >> (8 * i)) & 0xFF) == 0xFF) nhi = min(nhi, p);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int p = min(probe(i), NB - 1);
+      const int p = probe(i);
       if (((m >> (8 * i)) & 0xFF) != 0xFF && p < nhi) nlo = max(nlo, p);
     }
     lo = nlo;
     hi = nhi;
   };
-  // first the last block -- where nothing can be left out that is all -- and, for the usual reach of a few
-  // tiles, the blocks 2, 4, ... 128 on
-  const int at = lo;
-  narrow([&](int i) { return i == 7 ? NB - 1 : at + (2 << i); });
+  narrow(first.f, [&](int i) { return kv_first_probe(key0, i, NB); });
   if (hi == NB) return NB - 1;
   while (hi - lo > 1) {
-    const int from = lo, stride = max(1, (hi - lo) / 9);
-    narrow([&](int i) { return min(from + (i + 1) * stride, hi - 1); });
+    const int from = lo, stride = max(1, (hi - lo) / 9), end = hi - 1;
+    auto probe = [&](int i) { return min(from + (i + 1) * stride, end); };
+    const float* p = carry_b + (int64_t)probe(part) * T;
+    float f[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = p[min(j0 + e, T - 1)];
+    narrow(f, probe);
   }
   return lo;
 }
 
-// The head's bounds from its row segments: the largest |q| and the least lse.
-__device__ __forceinline__ float2 head_qstat(const BwdReach& reach, int64_t r, int lane) {
-  float qm = 0.f, lm = INFINITY;
-  for (int i = lane; i < reach.nseg; i += 64) {
+// The head's bounds from its row segments: the largest |q| and the least lse. first: two of them per lane.
+__device__ __forceinline__ float2 head_qstat(const BwdReach& reach, int64_t r, int lane, const float2 (&first)[2]) {
+  float qm = fmaxf(first[0].x, first[1].x), lm = fminf(first[0].y, first[1].y);
+  for (int i = lane + 128; i < reach.nseg; i += 64) {
     const float2 x = reach.qstat[r * reach.nseg + i];
     qm = fmaxf(qm, x.x);
     lm = fminf(lm, x.y);
@@ -2727,6 +2762,10 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
   float* uplane = ucheck + ((int64_t)gi * nseq + b) * utri_floats(NB);
   const float* carry_col = carry + (int64_t)b * NB * T + (j < T ? j : 0);
 
+  KvProbe probe[G];   // (the carry is the same for every head)
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+    probe[g] = kv_probe(reach, seq_row + hd0 + g, carry + (int64_t)b * NB * T, T, NB, key0, lane);
   // Key-side operands (B operands: lane = key column): this wavefront's K and V rows of the group
   // and head 0's K rows, in its LDS rows or in registers.
   frag kf[KVLDS ? 1 : G][NS], vf[KVLDS ? 1 : G][NS], k0f[NS];
@@ -2809,19 +2848,23 @@ __global__ __launch_bounds__(NTHREADS, (kv_min_blocks<OP, D, G>())) void bwd_kv_
   const int qb_lo = bxy.x * NWAVES;
   int qb_hi = NB - 1;   // the first tile of the sweep: later ones hold no weight for the workgroup's keys
   if (reach.qstat) {
-    if constexpr (KVLDS) lds_wave_sync();   // (the wavefront's own rows)
-    float thr = -INFINITY;
+    int last = key0 < T ? NB - 1 : 0;
+    if (key0 < T && kv_worth(probe[0], key0, T, reach.xk, lane)) {
+      if constexpr (KVLDS) lds_wave_sync();   // (the wavefront's own rows)
+      float thr = -INFINITY;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      frag kg[NS], vg[NS];
+      for (int g = 0; g < G; ++g) {
+        frag kg[NS], vg[NS];
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        kg[s] = k_frag(g, s);
-        vg[s] = v_frag(g, s);
+        for (int s = 0; s < NS; ++s) {
+          kg[s] = k_frag(g, s);
+          vg[s] = v_frag(g, s);
+        }
+        const float2 qstat = head_qstat(reach, seq_row + hd0 + g, lane, probe[g].q);
+        thr = fmaxf(thr, kv_threshold(frag_sumsq<OP, NS>(kg), frag_sumsq<OP, NS>(vg), qstat, scale));
       }
-      thr = fmaxf(thr, kv_threshold(frag_sumsq<OP, NS>(kg), frag_sumsq<OP, NS>(vg), head_qstat(reach, seq_row + hd0 + g, lane), scale));
+      last = kv_last_block(probe[0], carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane);
     }
-    const int last = key0 < T ? kv_last_block(carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane) : 0;
     if (lane == 0) sLast[wave] = last;
     __syncthreads();
     qb_hi = kv_sweep_start(sLast, NB, qb_lo, wave, lane, key0, T, uplane,
@@ -3097,6 +3140,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   float* uplane = ucheck + ((int64_t)hh * nseq + b) * utri_floats(NB);
   const float* carry_b = carry + (int64_t)b * NB * T;
 
+  const KvProbe probe = kv_probe(reach, seq_row + hh, carry_b, T, NB, key0, lane);
   // B operands (lane = key): the wavefront's K rows and head 0's in registers, its V rows in LDS
   frag kf[NS], k0f[NS];
   {
@@ -3149,12 +3193,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_kv64_kernel(
   const int qb_lo = bxy.x * NWAVES;
   int qb_hi = NB - 1;
   if (reach.qstat) {
-    lds_wave_sync();   // the wavefront's V rows
-    frag vg[NS];
+    int last = key0 < T ? NB - 1 : 0;
+    if (key0 < T && kv_worth(probe, key0, T, reach.xk, lane)) {
+      lds_wave_sync();   // the wavefront's V rows
+      frag vg[NS];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) vg[s] = rfrag(sV[wave], s);
-    const float thr = kv_threshold(frag_sumsq<OP, NS>(kf), frag_sumsq<OP, NS>(vg), head_qstat(reach, seq_row + hh, lane), scale);
-    const int last = key0 < T ? kv_last_block(carry_b, T, NB, key0, reach.xk, thr, lane) : 0;
+      for (int s = 0; s < NS; ++s) vg[s] = rfrag(sV[wave], s);
+      const float2 qstat = head_qstat(reach, seq_row + hh, lane, probe.q);
+      const float thr = kv_threshold(frag_sumsq<OP, NS>(kf), frag_sumsq<OP, NS>(vg), qstat, scale);
+      last = kv_last_block(probe, carry_b, T, NB, key0, reach.xk, thr, lane);
+    }
     if (lane == 0) sLast[wave] = last;
     __syncthreads();
     qb_hi = kv_sweep_start(sLast, NB, qb_lo, wave, lane, key0, T, uplane,
@@ -4309,6 +4357,8 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
   auto head = [&](const float* p, const Strides& s, int x) { return rsrc(p + s.at(b, x), (int64_t)T * s.row * 4); };
   const __amdgpu_buffer_rsrc_t rs_q = head(q, qs, hh), rs_q0 = head(q, qs, 0), rs_do = head(dout, dos, hh);
   HalfRow<D> kf, k0f, vf;   // B operands: lane = key
+  const float* carry_col = carry + (int64_t)b * NB * T + min(j, T - 1);
+  const KvProbe probe = kv_probe(reach, blockIdx.y, carry + (int64_t)b * NB * T, T, NB, key0, lane);
   kf.load(head(k, ks, hh), ks.row, j, h);
   k0f.load(head(k, ks, 0), ks.row, j, h);
   vf.load(head(v, vs, hh), vs.row, j, h);
@@ -4320,16 +4370,18 @@ __global__ __launch_bounds__(NTHREADS, 1) void bwd_kv_split_kernel(
     dk0t[db] = zero16();
   }
   float* uplane = ucheck + ((int64_t)hh * nseq + b) * utri_floats(NB);
-  const float* carry_col = carry + (int64_t)b * NB * T + min(j, T - 1);
   const float* lse_row = lse + (int64_t)blockIdx.y * ldt;
   const float* ndb_row = ndbar + (int64_t)blockIdx.y * ldt;
   const float sl2 = scale * LOG2E, neg_inv_scale = -1.f / scale;
   const int ntiles = NB - kt;
   int t0 = 0;
   if (reach.qstat) {
-    const float thr = kv_threshold(kf.sumsq(), vf.sumsq(), head_qstat(reach, blockIdx.y, lane), scale);
-    const int top = __builtin_amdgcn_readfirstlane(
-        kv_last_block(carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane));
+    int top = NB - 1;
+    if (kv_worth(probe, key0, T, reach.xk, lane)) {
+      const float thr = kv_threshold(kf.sumsq(), vf.sumsq(), head_qstat(reach, blockIdx.y, lane, probe.q), scale);
+      top = __builtin_amdgcn_readfirstlane(
+          kv_last_block(probe, carry + (int64_t)b * NB * T, T, NB, key0, reach.xk, thr, lane));
+    }
     if (tid == 0) reach.hi[((int64_t)hh * nseq + b) * reach.nkg + kt] = top;
     t0 = (NB - 1 - top) / 4;
   }
